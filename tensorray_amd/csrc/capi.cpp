@@ -11,6 +11,7 @@
 #include <string>
 
 #include "trc_internal.h"
+#include "common/tr_bsdf.h"
 
 using namespace trc;
 
@@ -194,6 +195,25 @@ void upload_scene(trc_scene* s, hipStream_t st) {
   d.shade = upload(s, h.shade, st);
   d.tris = upload(s, h.tris, st);
   d.nodes = upload(s, h.nodes, st);
+  float ext = 0.0f;
+  {
+    const Bvh4Node& root = h.nodes[0];
+    const float* lo[3] = {root.lox, root.loy, root.loz};
+    const float* hi[3] = {root.hix, root.hiy, root.hiz};
+    for (int k = 0; k < 3; ++k) {
+      float a = lo[k][0], b = hi[k][0];
+      for (int i = 1; i < 4; ++i)
+        if (root.child[i] != kEmpty) {
+          a = std::min(a, lo[k][i]);
+          b = std::max(b, hi[k][i]);
+        }
+      ext = std::max(ext, b - a);
+    }
+  }
+  d.qinv_scale = 1.0f / quant_scale(ext);
+  std::vector<QNode> qnodes(h.nodes.size());
+  for (size_t i = 0; i < qnodes.size(); ++i) qnodes[i] = quantize_node(h.nodes[i], d.qinv_scale);
+  d.qnodes = upload(s, qnodes, st);
   d.mats = upload(s, h.materials, st);
   std::vector<TexDesc> texs;
   for (size_t i = 0; i < h.textures.size(); ++i) {
@@ -208,6 +228,10 @@ void upload_scene(trc_scene* s, hipStream_t st) {
   d.light_tri = upload(s, h.light_tri, st);
   d.light_cdf = upload(s, h.light_cdf, st);
   d.light_f = upload(s, h.light_f, st);
+  std::vector<float> light_pdf(h.light_tri.size());
+  for (size_t i = 0; i < light_pdf.size(); ++i)
+    light_pdf[i] = light_area_pdf(h.light_f[i], h.light_integral, (int32_t)light_pdf.size(), h.shade[h.light_tri[i]].area);
+  d.light_pdf = upload(s, light_pdf, st);
   d.emit_rad = upload(s, h.emit_rad, st);
   // secondary-edge arrays sized for every edge: a device update may select
   // any number of them

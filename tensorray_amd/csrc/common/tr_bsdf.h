@@ -20,8 +20,7 @@ struct Its {
 // CoordinateSystem (LibTensorRay/Renderer/Utils.cpp:118-140).
 TR_HD void coordinate_system(F3 n, F3* t, F3* b) {
   bool cond = fabsf(n.x) > fabsf(n.y);
-  float il = cond ? 1.0f / sqrtf(maxf(n.x * n.x + n.z * n.z, 1e-3f))
-                  : 1.0f / sqrtf(maxf(n.y * n.y + n.z * n.z, 1e-3f));
+  const float il = rsqrt_rn(maxf((cond ? n.x * n.x : n.y * n.y) + n.z * n.z, 1e-3f));
   *t = cond ? F3{-n.z * il, 0.0f, n.x * il} : F3{0.0f, n.z * il, -n.y * il};
   *b = cross(n, *t);
 }
@@ -92,7 +91,7 @@ TR_HD F3 cosine_sample_hemisphere(float s0, float s1) {
   float sp, cp;
   tr_sincos(phi, &sp, &cp);
   float x = r_ * cp, y = r_ * sp;
-  float z = sqrtf(maxf(1e-4f, 1.0f - x * x - y * y));
+  float z = sqrt_rn(maxf(1e-4f, 1.0f - x * x - y * y));
   return F3{x, y, z};
 }
 
@@ -135,7 +134,7 @@ TR_HD float tan_theta2(F3 v) {
   float c2 = v.z * v.z;
   return maxf(1.0f - c2, 0.0f) / c2;
 }
-TR_HD float sin_theta(F3 v) { return sqrtf(maxf(1.0f - v.z * v.z, 0.0f)); }
+TR_HD float sin_theta(F3 v) { return sqrt_rn(maxf(1.0f - v.z * v.z, 0.0f)); }
 TR_HD float cos_phi(F3 v) {
   float st = sin_theta(v);
   return st == 0.0f ? 1.0f : clampf(v.x / st, -1.0f, 1.0f);
@@ -162,7 +161,7 @@ TR_HD float smith_g(F3 v, F3 wh, float alpha) {
   float t2 = tan_theta2(wh);
   bool ok = t2 < 3.402823466e38f;
   float root = (alpha * alpha) * t2;
-  float G = 2.0f / (1.0f + sqrtf(1.0f + root * root));
+  float G = 2.0f / (1.0f + sqrt_rn(1.0f + root * root));
   G = ok ? G : 0.0f;
   float voh = dot(v, wh);
   G = (t2 == 0.0f) ? 1.0f : G;
@@ -373,6 +372,7 @@ struct LightSample {
   F3 p, n;
   float pdf;       // pmf / area (area measure)
   int32_t tri;     // global triangle id
+  int32_t index;   // emitter triangle (of the light arrays)
   int32_t emitter;
   float bu, bv;    // barycentrics of the sampled point
 };
@@ -380,9 +380,8 @@ struct LightSample {
 TR_HD LightSample light_sample(const SceneDev& S, float u0, float u1) {
   LightSample ls;
   int32_t i = cdf_search(S.light_cdf, S.n_light, u0);
-  float pmf = S.light_f[i] / (S.light_integral * (float)S.n_light);
   float reuse = cdf_reuse(S.light_cdf, i, u0);
-  float t = sqrtf(reuse);
+  float t = sqrt_rn(reuse);
   float bu = 1.0f - t;
   float bv = t * u1;
   float bw = 1.0f - bu - bv;
@@ -391,19 +390,24 @@ TR_HD LightSample light_sample(const SceneDev& S, float u0, float u1) {
   ls.p = bw * q0 + bu * q1 + bv * q2;
   const TriShade& sh = S.shade[tri];
   ls.n = F3{sh.n[0], sh.n[1], sh.n[2]};
-  ls.pdf = pmf / sh.area;
+  ls.pdf = S.light_pdf[i];
   ls.tri = tri;
+  ls.index = i;
   ls.emitter = sh.emitter;
   ls.bu = bu;
   ls.bv = bv;
   return ls;
 }
 
+// Area density of the samples on one emitter triangle: its probability over
+// its area (SceneDev::light_pdf).
+TR_HD float light_area_pdf(float f, float integral, int32_t n, float area) {
+  return f / (integral * (float)n) / area;
+}
+
 // AreaLight::Pdf (Light.cpp:177-184) for a BSDF-sampled emitter hit.
 TR_HD float light_pdf_tri(const SceneDev& S, int32_t tri) {
-  const TriShade& sh = S.shade[tri];
-  float pmf = S.light_f[sh.emit_tri] / (S.light_integral * (float)S.n_light);
-  return pmf / sh.area;
+  return S.light_pdf[S.shade[tri].emit_tri];
 }
 
 // AreaLight::Eval (Light.cpp:134-144): one-sided emission.
@@ -453,7 +457,8 @@ TR_HD SensorSample sensor_sample(const CameraDev& c, F3 p) {
   s.pixel = py * c.width + px;
   F3 d = p - F3{c.eye[0], c.eye[1], c.eye[2]};
   float d2 = len2(d);
-  F3 dn = d / sqrtf(d2);
+  float dl;
+  F3 dn = over_sqrt(d, d2, &dl);
   float ct = dot(F3{c.dir[0], c.dir[1], c.dir[2]}, dn);
   float ic = 1.0f / ct;
   s.value = 1.0f / d2 * ic * ic * ic * c.inv_area;

@@ -8,7 +8,8 @@
 //   vnrm     float[V][3]      vertex normals (smooth-shaded meshes only)
 //   shade    TriShade[T]      per-triangle face normal, area, material, emitter
 //   tris     TriRecord[T]     triangle vertices in BVH leaf order (48 B)
-//   nodes    Bvh4Node[N]      4-wide BVH, 128 B per node (one cache line)
+//   nodes    Bvh4Node[N]      4-wide BVH with float child boxes (refit, SAH cost)
+//   qnodes   QNode[N]         the same tree as the traversal reads it, 64 B per node
 //   mats     Material[M]
 //   light_*  emitter triangles, their CDF and sampling weights
 //
@@ -24,9 +25,12 @@ namespace trc {
 // Longest path the integrators record for replay (bounces after the primary hit).
 constexpr int kMaxBounces = 8;
 
-// 4-wide BVH node.  Child boxes are stored SoA so one node is read with
-// eight 16-byte loads; `child` encodes inner nodes (index), leaves
-// (kLeafBit | (count-1) << 27 | first) and empty slots (kEmpty).
+// 4-wide BVH node.  Child boxes are stored SoA; `child` encodes inner nodes
+// (index), leaves (kLeafBit | (count-1) << 27 | first) and empty slots
+// (kEmpty).  The builder fills the slots with the inner children first, then
+// the leaves, numbers the inner children of a node consecutively, and puts
+// one triangle into each leaf, consecutive ones into the leaves of a node:
+// QNode names all children by two base indices.
 struct alignas(128) Bvh4Node {
   float lox[4], loy[4], loz[4];
   float hix[4], hiy[4], hiz[4];
@@ -45,6 +49,94 @@ TR_HD uint32_t leaf_first(uint32_t c) { return c & kLeafFirstMask; }
 TR_HD uint32_t leaf_count(uint32_t c) { return ((c >> 27) & 0xFu) + 1u; }
 TR_HD uint32_t make_leaf(uint32_t first, uint32_t count) {
   return kLeafBit | ((count - 1u) << 27) | first;
+}
+
+// A 4-wide node as the traversal reads it: 64 bytes, four 16-byte loads.
+// Child box planes are half-precision offsets from the node's origin in units
+// of the tree's scale (SceneDev::qinv_scale is its reciprocal, a power of
+// two), rounded outwards; v_fma_mix_f32 reads them without a conversion.
+//   w[0..1]  origin / scale, 21 bits per axis: sign, exponent and 12 mantissa
+//            bits of a float rounded down (x in w0[31:11], y in w0[10:0] and
+//            w1[31:22], z in w1[21:1])
+//   w[2]     index of the first inner child | inner children << kQCountShift
+//   w[3]     first leaf's triangle record  | leaves << kQCountShift
+//   w[4k+4 .. 4k+7]  axis k: lower planes of slots 0 1, 2 3, upper planes of
+//            slots 0 1, 2 3
+// The forward is bound by VALU issue (92 % of the SIMDs' cycles with the 112
+// bytes and 232 instructions of a Bvh4Node visit).  8-bit planes in 48 bytes
+// need a conversion per plane and round the large boxes near the root so far
+// out that a query tests 21 % more triangles and visits 6 % more nodes of the
+// 20k-triangle sphere scene; 11 bits of mantissa do not.
+struct alignas(16) QNode {
+  uint32_t w[16];
+};
+static_assert(sizeof(QNode) == 64, "four 16-byte loads");
+constexpr int kQCountShift = 27;
+constexpr uint32_t kQIndexMask = (1u << kQCountShift) - 1u;
+// Relative widening of the plane offsets: covers the rounding of the
+// traversal's t = h i + b in its h i part (3 x 2^-24 of it).
+constexpr double kQWiden = 1.0 / 1048576.0;
+
+// Bits of the half-precision number at or below (up = false) or at or above
+// (up = true) x >= 0; beyond the largest one 65504 or infinity, 0 or infinity
+// for NaN.
+TR_HD uint32_t half_bits(double x, bool up) {
+  if (!(x < 65504.0)) return up ? 0x7C00u : (x >= 65504.0 ? 0x7BFFu : 0u);
+  if (!(x > 0.0)) return 0u;
+  int e = 0;
+  frexp(x, &e);  // x = m 2^e, m in [0.5, 1)
+  if (e < -13) e = -13;
+  const double m = ldexp(x, 11 - e);  // [1024, 2048), below for denormals
+  const uint32_t k = (uint32_t)(up ? ceil(m) : floor(m));
+  return ((uint32_t)(e + 13) << 10) + k;  // a normal number's leading 1024 carries into the exponent
+}
+
+// The scale of a tree of extent `ext`: offsets up to 2^14 steps, which leaves
+// room for a refit to grow the boxes fourfold (beyond that the upper planes
+// become infinite: the boxes only stop culling).
+TR_HD float quant_scale(float ext) {
+  int e = 0;
+  if (ext > 0.0f && ext < 1e30f) frexp((double)ext, &e);
+  e = e < -80 ? -80 : e;
+  return (float)ldexp(1.0, e - 14);
+}
+
+// The QNode of `n`, whose slots are laid out as described at Bvh4Node.  The
+// differences to the origin are taken in double (exact, or within 2^-53 of
+// coordinates whose boxes were padded by 2^-20), so the planes never lie
+// inside the padded boxes.
+TR_HD QNode quantize_node(const Bvh4Node& n, float inv_scale) {
+  QNode q;
+  uint32_t ni = 0u, nl = 0u;
+  const float* lo[3] = {n.lox, n.loy, n.loz};
+  const float* hi[3] = {n.hix, n.hiy, n.hiz};
+  for (int s = 0; s < 4; ++s) {
+    if (n.child[s] == kEmpty) continue;
+    if (n.child[s] & kLeafBit) ++nl;
+    else ++ni;
+  }
+  uint32_t org[3];
+  for (int k = 0; k < 3; ++k) {
+    float o = lo[k][0];
+    for (uint32_t s = 1; s < ni + nl; ++s) o = lo[k][s] < o ? lo[k][s] : o;
+    union { float f; uint32_t u; } c;
+    c.f = o * inv_scale;
+    if (c.u & 0x80000000u) c.u += 0x7FFu;  // towards minus infinity
+    c.u &= ~0x7FFu;
+    org[k] = c.u >> 11;
+    for (uint32_t j = 0; j < 4; ++j) q.w[4 + 4 * k + j] = 0u;
+    for (uint32_t s = 0; s < ni + nl; ++s) {
+      const double a = (double)lo[k][s] * (double)inv_scale - (double)c.f;
+      const double b = (double)hi[k][s] * (double)inv_scale - (double)c.f;
+      q.w[4 + 4 * k + (s >> 1)] |= half_bits(a * (1.0 - kQWiden), false) << (16u * (s & 1u));
+      q.w[6 + 4 * k + (s >> 1)] |= half_bits(b * (1.0 + kQWiden), true) << (16u * (s & 1u));
+    }
+  }
+  q.w[0] = org[0] << 11 | org[1] >> 10;
+  q.w[1] = org[1] << 22 | org[2] << 1;
+  q.w[2] = (ni ? n.child[0] : 0u) | ni << kQCountShift;
+  q.w[3] = (nl ? leaf_first(n.child[ni]) : 0u) | nl << kQCountShift;
+  return q;
 }
 
 // SAH costs of a 4-wide node visit and of a triangle test, used by the
@@ -162,11 +254,13 @@ struct SceneDev {
   const TriShade* shade;
   const TriRecord* tris;
   const Bvh4Node* nodes;
+  const QNode* qnodes;
   const Material* mats;
   const TexDesc* texs;
   const int32_t* light_tri;   // emitter triangle -> global triangle id
   const float* light_cdf;     // normalized CDF over emitter triangles
   const float* light_f;       // luminance * area per emitter triangle
+  const float* light_pdf;     // area density of its samples (light_area_pdf)
   const float* emit_rad;      // [n_emitters][3]
   EdgeSet sec;                // secondary edges (ConstructSecEdgeList, Edge.cpp:42-88)
   int32_t n_light;
@@ -174,6 +268,7 @@ struct SceneDev {
   int32_t n_tris;
   int32_t n_mats;
   int32_t stack_need;         // worst-case traversal stack depth of this BVH
+  float qinv_scale;           // 1 / scale of the quantized nodes' offsets, a power of two
   int32_t n_verts;
   // smooth-shaded faces incident to each vertex, in triangle order (CSR:
   // faces of vertex v are vf_list[vf_off[v] .. vf_off[v+1])), for the

@@ -44,7 +44,10 @@ struct BinNode {
 constexpr int kBins = 32;
 constexpr double kCostTraverse = kSahTraverse;
 constexpr double kCostIntersect = kSahIntersect;
-constexpr int kMaxLeaf = 4;
+// One triangle per leaf: the quantized node names its leaves' triangles by
+// one base index.  (At a node visit costing kSahTraverse triangle tests,
+// almost no larger leaf was ever chosen.)
+constexpr int kMaxLeaf = 1;
 
 struct Builder {
   const std::vector<float>& pos;
@@ -257,29 +260,29 @@ struct Collapser {
       kids.push_back(bn[k].left);
       kids.push_back(bn[k].right);
     }
+    // inner children in the first slots, numbered consecutively; leaves after
+    // them, their triangles consecutive (QNode)
+    std::stable_partition(kids.begin(), kids.end(), [&](int32_t k) { return !bn[k].leaf(); });
     Bvh4Node node;
     for (int s = 0; s < 4; ++s) set_empty(node, s);
     int need = 0;
     int nk = (int)kids.size();
-    std::vector<std::pair<int, uint32_t>> inner;  // (slot, binary id)
+    int ni = 0;
+    const uint32_t first_child = (uint32_t)out.size();
     for (int s = 0; s < nk; ++s) {
       const BinNode& c = bn[kids[s]];
       set_child_box(node, s, c.box);
       if (c.leaf()) {
         node.child[s] = emit_leaf(c);
       } else {
-        inner.push_back({s, (uint32_t)kids[s]});
+        node.child[s] = first_child + (uint32_t)s;
+        ++ni;
       }
     }
     out[out_index] = node;
-    for (auto& pr : inner) {
-      uint32_t ci = (uint32_t)out.size();
-      out.push_back(Bvh4Node{});
-      out[out_index].child[pr.first] = ci;
-      // at most nk-1 siblings are pending on the stack while a child is visited
-      int sub = collapse((int32_t)pr.second, ci, depth + 1);
-      need = std::max(need, (nk - 1) + sub);
-    }
+    out.resize(out.size() + (size_t)ni);
+    // at most nk-1 siblings are pending on the stack while a child is visited
+    for (int s = 0; s < ni; ++s) need = std::max(need, (nk - 1) + collapse(kids[s], first_child + (uint32_t)s, depth + 1));
     return need;
   }
 };

@@ -47,8 +47,7 @@ TR_HD FaceGeom face_geom(F3 p0, F3 p1, F3 p2) {
   g.p0 = p0; g.p1 = p1; g.p2 = p2;
   g.e0 = p1 - p0; g.e1 = p2 - p0;
   g.c = cross(g.e0, g.e1);
-  g.len = length(g.c);
-  g.n = g.c / g.len;
+  g.n = over_sqrt(g.c, len2(g.c), &g.len);
   g.area = g.len * 0.5f;
   return g;
 }
@@ -70,7 +69,7 @@ TR_HD F3 coordsys_vjp(F3 n, F3 adj_t, F3 adj_b) {
   bool cond = fabsf(n.x) > fabsf(n.y);
   if (cond) {
     float q = n.x * n.x + n.z * n.z;
-    float il = 1.0f / sqrtf(maxf(q, 1e-3f));
+    float il = rsqrt_rn(maxf(q, 1e-3f));
     adj_n.z += -adj_t.x * il;
     adj_n.x += adj_t.z * il;
     float adj_il = -adj_t.x * n.z + adj_t.z * n.x;
@@ -81,7 +80,7 @@ TR_HD F3 coordsys_vjp(F3 n, F3 adj_t, F3 adj_b) {
     }
   } else {
     float q = n.y * n.y + n.z * n.z;
-    float il = 1.0f / sqrtf(maxf(q, 1e-3f));
+    float il = rsqrt_rn(maxf(q, 1e-3f));
     adj_n.z += adj_t.y * il;
     adj_n.y += -adj_t.z * il;
     float adj_il = adj_t.y * n.z - adj_t.z * n.y;
@@ -104,8 +103,8 @@ TR_HD F3 microfacet_inner_vjp(F3 wo, F3 wi, float r, F3 kd, F3 F0, F3 adj_f, F3*
   const float c1 = -5.55473f, c2 = 6.8316f;
   float nv = wo.z, nl = wi.z;
   F3 hr = wo + wi;
-  float hl = length(hr);
-  F3 wh = hr / hl;
+  float hl;
+  F3 wh = over_sqrt(hr, len2(hr), &hl);
   float nh = wh.z, vh = dot(wo, wh);
   float alpha = r * r;
   float k = (r + 1.0f) * (r + 1.0f) * 0.125f;
@@ -178,7 +177,7 @@ TR_HD void smith_g_vjp(F3 v, F3 wh, float a, float gG, float* g_z, float* g_a) {
   float t2 = tan_theta2(wh);
   if (!(t2 < 3.402823466e38f) || t2 == 0.0f || (dot(v, wh) * v.z) <= 0.0f) return;
   float root = (a * a) * t2;
-  float sq = sqrtf(1.0f + root * root);
+  float sq = sqrt_rn(1.0f + root * root);
   float g_root = gG * (-2.0f / ((1.0f + sq) * (1.0f + sq))) * root / sq;
   *g_a += g_root * 2.0f * a * t2;
   *g_z += g_root * (a * a) * tan2_dz(wh.z);
@@ -240,8 +239,8 @@ TR_HD void roughconductor_inner_vjp(F3 wo, F3 wi, float r, F3 eta, F3 kk, F3 adj
   *adj_r = 0.0f;
   if (!(wo.z > 0.0f && wi.z > 0.0f)) return;
   F3 hr = wo + wi;
-  float hl = length(hr);
-  F3 wh = hr / hl;
+  float hl;
+  F3 wh = over_sqrt(hr, len2(hr), &hl);
   float D = ggx_d(wh, r);
   if (D == 0.0f) return;
   float Go = smith_g(wo, wh, r), Gi = smith_g(wi, wh, r), G = Go * Gi;
@@ -437,8 +436,8 @@ __device__ void path_backward(const SceneDev& S, const CameraDev& C, const PathP
       xprev = (1.0f - uu - vv) * q0 + uu * q1 + vv * q2;
     }
     F3 dinr = xi - xprev;
-    float dinl = length(dinr);
-    F3 din = dinr / dinl;
+    float dinl;
+    F3 din = over_sqrt(dinr, len2(dinr), &dinl);
     F3 wo = -din;
     const F3 beta = R.beta[i];
     F3 adj_x = zero, adj_wo = zero, adj_ng = zero, adj_xprev = zero;
@@ -456,8 +455,8 @@ __device__ void path_backward(const SceneDev& S, const CameraDev& C, const PathP
         float lbu = R.lbu[i], lbv = R.lbv[i], lbw = 1.0f - lbu - lbv;
         F3 pL = lbw * q0 + lbu * q1 + lbv * q2;
         F3 wr = pL - xi;
-        float d2 = len2(wr), dist = sqrtf(d2);
-        F3 wl = wr / dist;
+        float d2 = len2(wr), dist;
+        F3 wl = over_sqrt(wr, d2, &dist);
         float dsh = dot(its.ns, wl);
         float absSh = fabsf(dsh);
         float q = dot(lg.n, -wl);
@@ -496,8 +495,8 @@ __device__ void path_backward(const SceneDev& S, const CameraDev& C, const PathP
       float nu = R.bu[i + 1], nvv = R.bv[i + 1], nw = 1.0f - nu - nvv;
       F3 xn = nw * r0 + nu * r1 + nvv * r2;
       F3 dr = xn - xi;
-      float dd2 = len2(dr), dl = sqrtf(dd2);
-      F3 d = dr / dl;
+      float dd2 = len2(dr), dl;
+      F3 d = over_sqrt(dr, dd2, &dl);
       float qn = dot(ng.n, -d);
       float G = fabsf(qn) / dd2;
       float dc = dot(its.ns, d);
@@ -529,8 +528,8 @@ __device__ void path_backward(const SceneDev& S, const CameraDev& C, const PathP
       // beta_0 = G_cam / detach(G_cam) * area / detach(area)
       float ab = Qi.x + Qi.y + Qi.z;
       F3 cdr = xi - eye;
-      float dist = length(cdr);
-      F3 cd = cdr / dist;
+      float dist;
+      F3 cd = over_sqrt(cdr, len2(cdr), &dist);
       const F3 cdir{C.dir[0], C.dir[1], C.dir[2]};
       float cosy = dot(cd, cdir);
       float cosx = dot(-cd, its.ng);

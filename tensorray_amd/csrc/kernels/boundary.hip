@@ -24,8 +24,6 @@ constexpr uint32_t kSensorBlock0 = 64u;
 __device__ inline TraceCtx make_trace_ctx_b(uint32_t* lds, const LaunchCfg& L) {
   TraceCtx t;
   t.lds = lds + threadIdx.x;
-  t.lds_stride = kBlock;
-  t.lds_depth = kStackLds;
   t.leafq = lds + kStackLds * kBlock + threadIdx.x;
   t.spill = L.spill;
   t.spill_stride = L.grid * kBlock;
@@ -217,8 +215,8 @@ struct XdnAdj {
 __device__ inline XdnAdj x_dot_n_vjp(F3 P0, F3 P1, F3 P2, F3 org, F3 through, F3 n, float w) {
   XdnAdj a;
   F3 dr = through - org;
-  float dl = length(dr);
-  F3 dir = dr / dl;
+  float dl;
+  F3 dir = over_sqrt(dr, len2(dr), &dl);
   F3 e1 = P1 - P0, e2 = P2 - P0;
   F3 h = cross(dir, e2);
   float aa = dot(e1, h);
@@ -678,8 +676,8 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
       F3 edge2 = normalize(g.p2 - g.p0);
       LightSample ls = light_sample(S, rnd.b, rnd.c);
       F3 ev = ls.p - p;
-      float d2 = len2(ev), dist = sqrtf(d2);
-      F3 en = ev / dist;
+      float d2 = len2(ev), dist;
+      F3 en = over_sqrt(ev, d2, &dist);
       float cosT = dot(ls.n, -en);
       float c0 = dot(en, g.n0), c1 = dot(en, g.n1);
       bool valid0 = fabsf(c0) > kEdgeEpsilon;
@@ -802,7 +800,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
         F3 ft, fb;
         coordinate_system(nrm, &ft, &fb);
         float z = minf(1.0f - 2.0f * rnd.b, 1.0f - kEdgeEpsilon);
-        float rr = sqrtf(maxf(0.0f, 1.0f - z * z));
+        float rr = sqrt_rn(maxf(0.0f, 1.0f - z * z));
         float sp, cp;
         tr_sincos(2.0f * kPi * rnd.c, &sp, &cp);
         dir = ((rr * cp) * ft + (rr * sp) * fb) + z * nrm;
@@ -820,7 +818,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
         F3 x1 = x * cp + z * sp;
         bool m0 = rnd.c > 0.5f;
         float bb = 4.0f * rnd.c - (m0 ? 3.0f : 1.0f);
-        float aa = sqrtf(1.0f - bb * bb) * (m0 ? -1.0f : 1.0f);
+        float aa = sqrt_rn(1.0f - bb * bb) * (m0 ? -1.0f : 1.0f);
         dir = x1 * aa + y * bb;
       }
       float pdf = pdf_e * pdf_d;

@@ -132,8 +132,8 @@ __device__ void path_bounces(const SceneDev& S, Src& tc, Its its, F3 beta, F3 ra
     {
       F3 wi = ls.p - its.p;
       float d2 = len2(wi);
-      float dist = sqrtf(d2);
-      wi = wi / dist;
+      float dist;
+      wi = over_sqrt(wi, d2, &dist);
       float dsh = dot(its.ns, wi), dgeo = dot(its.ng, wi);
       bool stable = dist > kShadowEpsilon && fabsf(dsh) > kEdgeEpsilon;
       bool noleak = (dsh * dgeo) > 0.0f;
@@ -144,7 +144,7 @@ __device__ void path_bounces(const SceneDev& S, Src& tc, Its its, F3 beta, F3 ra
       float pbs;
       F3 f = bsdf_eval_pdf(S, its, wo, wi, &pbs) * fabsf(dsh);
       F3 Le = emitted(S, ls.emitter, ls.n, -wi);
-      float JL = S.shade[ls.tri].area / S.shade[ls.tri].area;
+      float JL = ratio_self(S.shade[ls.tri].area);
       F3 val = valid * beta * f * JL * Gl * Le / ls.pdf;
       float pb = pbs * Gl;
       float mis = (ls.pdf * ls.pdf) / (ls.pdf * ls.pdf + pb * pb);
@@ -174,11 +174,12 @@ __device__ void path_bounces(const SceneDev& S, Src& tc, Its its, F3 beta, F3 ra
     Its its2 = post_intersect(S, h2.tri, h2.u, h2.v);
     F3 dd = its2.p - its.p;
     float dd2 = len2(dd);
-    F3 nd = dd / sqrtf(dd2);
+    float dl;
+    F3 nd = over_sqrt(dd, dd2, &dl);
     float G2 = fabsf(dot(its2.ng, -nd)) / dd2;
     F3 f2 = bsdf_eval(S, its, wo, nd) * fabsf(dot(its.ns, nd));
     float ppdf = pdfb * G2;
-    float J2 = S.shade[its2.tri].area / S.shade[its2.tri].area;
+    float J2 = ratio_self(S.shade[its2.tri].area);
     F3 beta2 = beta * f2 * G2 * J2 / ppdf;
     bool gpos = G2 > 0.0f;
     if (!gpos) beta2 = zero;
@@ -230,18 +231,18 @@ __device__ F3 path_forward(const SceneDev& S, const CameraDev& C, const PathPara
   Its its = post_intersect(S, h.tri, h.u, h.v);
   // EvalFilter: G / detach(G) with G = |cos_x| / (cos_y^3 d^2); times J
   float beta0;
+  F3 raydir;
   {
     F3 cd = its.p - eye;
-    float dist = length(cd);
-    cd = cd / dist;
+    float dist;
+    cd = over_sqrt(cd, len2(cd), &dist);
+    raydir = cd;
     float cosy = dot(cd, cdir);
     float cosx = dot(-cd, its.ng);
     float G = fabsf(cosx) / (cosy * cosy * cosy * (dist * dist));
-    float area = S.shade[its.tri].area;
-    beta0 = (G / G) * (area / area);
+    beta0 = ratio_self(G) * ratio_self(S.shade[its.tri].area);
   }
   F3 beta{beta0, beta0, beta0};
-  F3 raydir = normalize(its.p - eye);
   F3 contrib = zero;
   F3 e0c = zero;
   if (its.emitter >= 0) {
@@ -284,15 +285,19 @@ constexpr int kTraceKeep64 = 16;
 struct PathLane {
   uint64_t path;
   // stage (bits 0-1), the bounce's BSDF direction has a nonzero pdf (bit 2),
-  // bounce index b (bits 3-31): one register
+  // its shadow ray is traced (bit 3), bounce index b (bits 4-31): one register
   uint32_t sb;
   __device__ uint32_t stage() const { return sb & 3u; }
-  __device__ uint32_t b() const { return sb >> 3; }
+  __device__ uint32_t b() const { return sb >> 4; }
   __device__ void set_stage(uint32_t s) { sb = (sb & ~3u) | s; }
   int32_t tri;           // current vertex x_b
   float u, v;
   F3 beta, raydir, contrib;
-  float la, lb;          // light-sample uniforms of bounce b
+  // light sample of bounce b: emitter triangle and squared distance (its
+  // direction is d); shading needs nothing else of it, so the sample is not
+  // drawn and its geometry not evaluated a second time
+  int32_t li;
+  float ld2;
   float pdfb;            // pdf of the BSDF direction d2 of bounce b
   // query of this iteration from o (tmin = kShadowEpsilon): the camera ray
   // along d, or the bounce's shadow ray along d (any hit) chained with its
@@ -313,8 +318,7 @@ __device__ inline NeeGeo nee_geo(const SceneDev& S, const Its& its, float la, fl
   g.ls = light_sample(S, la, lb);
   F3 wi = g.ls.p - its.p;
   g.d2 = len2(wi);
-  g.dist = sqrtf(g.d2);
-  g.wi = wi / g.dist;
+  g.wi = over_sqrt(wi, g.d2, &g.dist);
   g.dsh = dot(its.ns, g.wi);
   float dgeo = dot(its.ng, g.wi);
   bool stable = g.dist > kShadowEpsilon && fabsf(g.dsh) > kEdgeEpsilon;
@@ -400,11 +404,12 @@ __device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const Ck
   Its its2 = post_intersect(S, h.tri, h.u, h.v);
   F3 dd = its2.p - its.p;
   float dd2 = len2(dd);
-  F3 nd = dd / sqrtf(dd2);
+  float dl;
+  F3 nd = over_sqrt(dd, dd2, &dl);
   float G2 = fabsf(dot(its2.ng, -nd)) / dd2;
   F3 f2 = bsdf_eval(S, its, wo, nd) * fabsf(dot(its.ns, nd));
   float ppdf = L.pdfb * G2;
-  float J2 = S.shade[its2.tri].area / S.shade[its2.tri].area;
+  float J2 = ratio_self(S.shade[its2.tri].area);
   F3 beta2 = L.beta * f2 * G2 * J2 / ppdf;
   if (!(G2 > 0.0f)) beta2 = zero;
   if (its2.emitter >= 0) {
@@ -419,7 +424,7 @@ __device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const Ck
   L.tri = h.tri; L.u = h.u; L.v = h.v;
   L.beta = beta2;
   L.raydir = nd;
-  L.sb += 8u;  // b + 1
+  L.sb += 16u;  // b + 1
   if (kCkpt) {
     ckpt_put_vertex(ck, L.path, (int)L.b(), h.tri, h.u, h.v);
     meta += 1u;
@@ -506,16 +511,15 @@ __device__ void render_paths_regen(const SceneDev& S, const CameraDev& C, const 
       float beta0;
       {
         F3 cd = its.p - eye;
-        float dist = length(cd);
-        cd = cd / dist;
+        float dist;
+        cd = over_sqrt(cd, len2(cd), &dist);
+        L.raydir = cd;
         float cosy = dot(cd, cdir);
         float cosx = dot(-cd, its.ng);
         float G = fabsf(cosx) / (cosy * cosy * cosy * (dist * dist));
-        float area = S.shade[its.tri].area;
-        beta0 = (G / G) * (area / area);
+        beta0 = ratio_self(G) * ratio_self(S.shade[its.tri].area);
       }
       L.beta = F3{beta0, beta0, beta0};
-      L.raydir = normalize(its.p - eye);
       L.contrib = zero;
       if (its.emitter >= 0) {
         F3 Le = emitted(S, its.emitter, its.ng, -L.raydir);
@@ -533,18 +537,21 @@ __device__ void render_paths_regen(const SceneDev& S, const CameraDev& C, const 
       // next-event estimation of bounce b (Integrator.cpp:196-230) with the
       // traced shadow ray's outcome, then the BSDF-sampled ray's hit
       const F3 wo = -L.raydir;
-      const NeeGeo g = nee_geo(S, its, L.la, L.lb);
-      bool visible = g.ray && !trace_first_hit(L.ts);
+      const TriShade& lsh = S.shade[S.light_tri[L.li]];
+      const F3 ln{lsh.n[0], lsh.n[1], lsh.n[2]};
+      const float lpdf = S.light_pdf[L.li];
+      const F3 wi = L.d;
+      bool visible = (L.sb & 8u) != 0u && !trace_first_hit(L.ts);
       if (kCkpt && visible) meta |= 1u << (8u + L.b());
       float valid = visible ? 1.0f : 0.0f;
-      float Gl = fabsf(dot(g.ls.n, -g.wi)) / g.d2;
+      float Gl = fabsf(dot(ln, -wi)) / L.ld2;
       float pbs;
-      F3 f = bsdf_eval_pdf(S, its, wo, g.wi, &pbs) * fabsf(g.dsh);
-      F3 Le = emitted(S, g.ls.emitter, g.ls.n, -g.wi);
-      float JL = S.shade[g.ls.tri].area / S.shade[g.ls.tri].area;
-      F3 val = valid * L.beta * f * JL * Gl * Le / g.ls.pdf;
+      F3 f = bsdf_eval_pdf(S, its, wo, wi, &pbs) * fabsf(dot(its.ns, wi));
+      F3 Le = emitted(S, lsh.emitter, ln, -wi);
+      float JL = ratio_self(lsh.area);
+      F3 val = valid * L.beta * f * JL * Gl * Le / lpdf;
       float pb = pbs * Gl;
-      float mis = (g.ls.pdf * g.ls.pdf) / (g.ls.pdf * g.ls.pdf + pb * pb);
+      float mis = (lpdf * lpdf) / (lpdf * lpdf + pb * pb);
       val = val * mis;
       F3 ret = zero;
       ret = ret + val;
@@ -554,12 +561,12 @@ __device__ void render_paths_regen(const SceneDev& S, const CameraDev& C, const 
     // (Integrator.cpp:196-213 and 232-245; the draws of the reference's
     // loop in its order: light sample 1 + 2b, BSDF sample 2 + 2b)
     const Rnd4 rl = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b());
-    L.la = rl.a;
-    L.lb = rl.b;
     const NeeGeo g2 = nee_geo(S, its, rl.a, rl.b);
+    L.li = g2.ls.index;
+    L.ld2 = g2.d2;
     const Rnd4 rb = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b() + 1u);
     L.d2 = bsdf_sample(S, its, -L.raydir, rb.a, rb.b, &L.pdfb);
-    L.sb = (L.sb & ~7u) | kStageBounce | (L.pdfb > 0.0f ? 4u : 0u);
+    L.sb = (L.sb & ~15u) | kStageBounce | (L.pdfb > 0.0f ? 4u : 0u) | (g2.ray ? 8u : 0u);
     L.o = its.p;
     L.d = g2.wi;
     trace_begin_chain(L.ts, g2.ray ? g2.dist - kShadowEpsilon : -1.0f);

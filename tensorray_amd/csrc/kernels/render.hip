@@ -19,8 +19,6 @@ namespace trc {
 __device__ inline TraceCtx make_trace_ctx(uint32_t* lds, const LaunchCfg& L) {
   TraceCtx t;
   t.lds = lds + threadIdx.x;
-  t.lds_stride = kBlock;
-  t.lds_depth = kStackLds;
   t.leafq = lds + kStackLds * kBlock + threadIdx.x;
   t.spill = L.spill;
   t.spill_stride = L.grid * kBlock;

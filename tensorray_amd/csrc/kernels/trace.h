@@ -13,29 +13,34 @@ namespace trc {
 
 // Ray precomputation of the watertight test (Woop, Benthin, Wald, "Watertight
 // Ray/Triangle Intersection", JCGT 2(1), 2013): kz is the dominant axis of
-// the direction, kx / ky the other two (swapped when d[kz] < 0 to keep the
-// winding), S the shear constants.
+// the direction, kx / ky the two after it, S the shear constants.  The paper
+// swaps kx and ky when d[kz] < 0 to keep the winding; that only flips the
+// signs of U, V, W, of det and of T, so (t, u, v) are the same bits without
+// it, and the test below accepts either winding.
 struct RayPre {
   F3 o;
-  int kx, ky, kz;
+  int kz;
   float Sx, Sy, Sz;
 };
 
-TR_HD float comp(F3 v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : v.z); }
+TR_HD int ray_major(F3 d) {
+  float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
+  return (ax >= ay && ax >= az) ? 0 : (ay >= az ? 1 : 2);
+}
+// v rotated so that axis kz comes last.
+TR_HD F3 rotate_to(F3 v, int kz) {
+  return F3{kz == 2 ? v.x : (kz == 0 ? v.y : v.z), kz == 2 ? v.y : (kz == 0 ? v.z : v.x),
+            kz == 2 ? v.z : (kz == 0 ? v.x : v.y)};
+}
 
 TR_HD RayPre ray_pre(F3 o, F3 d) {
   RayPre r;
   r.o = o;
-  float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
-  int kz = (ax >= ay && ax >= az) ? 0 : (ay >= az ? 1 : 2);
-  int kx = kz == 2 ? 0 : kz + 1;
-  int ky = kx == 2 ? 0 : kx + 1;
-  float dz = comp(d, kz);
-  if (dz < 0.0f) { int t = kx; kx = ky; ky = t; }
-  r.kx = kx; r.ky = ky; r.kz = kz;
-  r.Sx = comp(d, kx) / dz;
-  r.Sy = comp(d, ky) / dz;
-  r.Sz = 1.0f / dz;
+  r.kz = ray_major(d);
+  const F3 k = rotate_to(d, r.kz);
+  r.Sx = k.x / k.z;
+  r.Sy = k.y / k.z;
+  r.Sz = 1.0f / k.z;
   return r;
 }
 
@@ -44,14 +49,13 @@ TR_HD RayPre ray_pre(F3 o, F3 d) {
 // applies the (tmin, tmax) interval.
 TR_HD bool tri_intersect(const RayPre& r, F3 p0, F3 p1, F3 p2, float* t_out, float* u_out,
                          float* v_out) {
-  F3 A = p0 - r.o, B = p1 - r.o, C = p2 - r.o;
-  float Akz = comp(A, r.kz), Bkz = comp(B, r.kz), Ckz = comp(C, r.kz);
-  float Ax = comp(A, r.kx) - r.Sx * Akz;
-  float Ay = comp(A, r.ky) - r.Sy * Akz;
-  float Bx = comp(B, r.kx) - r.Sx * Bkz;
-  float By = comp(B, r.ky) - r.Sy * Bkz;
-  float Cx = comp(C, r.kx) - r.Sx * Ckz;
-  float Cy = comp(C, r.ky) - r.Sy * Ckz;
+  const F3 A = rotate_to(p0 - r.o, r.kz), B = rotate_to(p1 - r.o, r.kz), C = rotate_to(p2 - r.o, r.kz);
+  float Ax = A.x - r.Sx * A.z;
+  float Ay = A.y - r.Sy * A.z;
+  float Bx = B.x - r.Sx * B.z;
+  float By = B.y - r.Sy * B.z;
+  float Cx = C.x - r.Sx * C.z;
+  float Cy = C.y - r.Sy * C.z;
   float U = Cx * By - Cy * Bx;
   float V = Ax * Cy - Ay * Cx;
   float W = Bx * Ay - By * Ax;
@@ -64,7 +68,7 @@ TR_HD bool tri_intersect(const RayPre& r, F3 p0, F3 p1, F3 p2, float* t_out, flo
   if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
   float det = U + V + W;
   if (det == 0.0f) return false;
-  float Az = r.Sz * Akz, Bz = r.Sz * Bkz, Cz = r.Sz * Ckz;
+  float Az = r.Sz * A.z, Bz = r.Sz * B.z, Cz = r.Sz * C.z;
   float T = U * Az + V * Bz + W * Cz;
   float inv = 1.0f / det;
   *t_out = T * inv;
@@ -78,26 +82,38 @@ struct Hit {
   float u, v, t;
 };
 
-// Conservative slab test factor 1 + 2*gamma(3) (gamma(n) = n eps / (1 - n eps),
-// eps = 2^-24): the far distance is inflated so rounding never culls a box
-// the exact ray enters.
-constexpr float kSlabScale = 1.0000003576278687f;
+// Slab test against the quantized planes, in units of the tree's scale (all
+// scalings are by powers of two).  With i = rcp(d) along an axis, the plane at
+// offset h from the node's origin g is met at t = (g + h - o) i, evaluated as
+// fma(h, i, b) over b = (g - o) i.  In units of e = 2^-24: i is off by at
+// most 2 e (v_rcp_f32), b by 2 e more relative to (g - o) / d, and the fma
+// rounds once, so t is off by at most 3 e |h i| + 5 e |b| (+ second order).
+// The stored offsets are widened by 16 e of themselves; kSlabWiden (8 e)
+// moves b towards the ray's start for near planes and away for far ones, its
+// own rounding included: rounding never culls a box the exact ray enters.
+constexpr float kSlabWiden = 4.76837158203125e-7f;
 
-TR_HD float safe_inv(float d) {
-  return fabsf(d) > 1e-30f ? 1.0f / d : (d >= 0.0f ? 1e30f : -1e30f);
+// 1 / d to within an ulp; a direction component of (nearly) zero counts as 1e-30.
+__device__ inline float slab_rcp(float d) {
+  return fabsf(d) > 1e-30f ? __builtin_amdgcn_rcpf(d) : (d >= 0.0f ? 1e30f : -1e30f);
 }
 
-// Per-thread traversal context: LDS part of the stack (stride = block size,
-// lane-interleaved so consecutive lanes use consecutive banks) and an HBM
-// spill slice for deeper entries.
+// The half-precision number in the low (i = 0) or high (i = 1) half of w; an
+// fma on it becomes one v_fma_mix_f32.
+__device__ inline float half_of(uint32_t w, uint32_t i) {
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  return (float)__builtin_bit_cast(half2_t, w)[i];
+}
+
+// Per-thread traversal context: the LDS part of the stack (kStackLds entries,
+// stride kBlock: lane-interleaved so consecutive lanes use consecutive banks)
+// and an HBM spill slice for deeper entries.
 struct TraceCtx {
   uint32_t* lds;        // &lds_stack[threadIdx.x]
-  uint32_t* leafq;      // postponed-leaf queue of this lane (kLeafQueue entries, stride lds_stride)
-  int lds_stride;       // blockDim.x
-  int lds_depth;        // entries held in LDS
+  uint32_t* leafq;      // postponed-leaf queue of this lane (kLeafQueue entries)
   uint32_t* spill;      // the grid's spill buffer [depth][grid threads] (wave-uniform)
   int spill_stride;     // total threads of the grid
-  int cap;              // total stack capacity (lds_depth + spill depth)
+  int cap;              // total stack capacity (kStackLds + spill depth)
   // this lane's result slots in LDS for the wave-wide leaf tests of
   // trace_run<true> (best hit key, its barycentrics); null where unused
   unsigned long long* slot_key;
@@ -109,17 +125,23 @@ struct TraceCtx {
 
 // This thread's column of the spill buffer, computed where it is used so
 // that no per-lane pointer stays live through the traversal.
-__device__ inline uint32_t spill_lane() { return blockIdx.x * blockDim.x + threadIdx.x; }
+__device__ inline uint32_t spill_lane() { return blockIdx.x * (uint32_t)kBlock + threadIdx.x; }
+
+// The stack's LDS part through an LDS pointer: a load that is either from
+// LDS or from the spill buffer would otherwise become one flat load, which
+// waits on both memories for every entry popped.
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+__device__ inline lds_u32* lds_ptr(uint32_t* p) { return (lds_u32*)p; }
 
 __device__ inline void stack_push(TraceCtx& c, int& sp, uint32_t v) {
-  if (sp < c.lds_depth) c.lds[sp * c.lds_stride] = v;
-  else c.spill[(size_t)(sp - c.lds_depth) * c.spill_stride + spill_lane()] = v;
+  if (sp < kStackLds) lds_ptr(c.lds)[sp * kBlock] = v;
+  else c.spill[(size_t)(sp - kStackLds) * c.spill_stride + spill_lane()] = v;
   ++sp;
 }
 __device__ inline uint32_t stack_pop(TraceCtx& c, int& sp) {
   --sp;
-  return sp < c.lds_depth ? c.lds[sp * c.lds_stride]
-                          : c.spill[(size_t)(sp - c.lds_depth) * c.spill_stride + spill_lane()];
+  if (sp < kStackLds) return lds_ptr(c.lds)[sp * kBlock];
+  return c.spill[(size_t)(sp - kStackLds) * c.spill_stride + spill_lane()];
 }
 
 __device__ inline F3 tri_vertex(const float* v) { return F3{v[0], v[1], v[2]}; }
@@ -136,6 +158,7 @@ struct TraceState {
                        // chain (14), second (15), first query hit (16)
 };
 constexpr uint32_t kNoHit = 0xFFFFFFFFu;
+constexpr uint32_t kNoChild = 0xFFFFFFFFu;  // sort key of a child slot without a hit inner child
 constexpr uint32_t kTsInnerDone = 1u << 12;
 constexpr uint32_t kTsFound = 1u << 13;
 // A chained pair of queries from one origin: an any-hit query (a shadow
@@ -217,7 +240,7 @@ __device__ inline void flush_wave(const SceneDev& S, TraceCtx& ctx, const RayPre
   int pre = 0, total = 0;
 #pragma unroll
   for (int bit = 0; bit < 4; ++bit) {
-    const uint64_t m = __ballot((nq >> bit) & 1);
+    const uint64_t m = __builtin_amdgcn_ballot_w64(((nq >> bit) & 1) != 0);
     pre += __popcll(m & below) << bit;
     total += __popcll(m) << bit;
   }
@@ -230,9 +253,9 @@ __device__ inline void flush_wave(const SceneDev& S, TraceCtx& ctx, const RayPre
   // wavefront fences keep the compiler from moving the slot accesses across
   // the rounds
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  const int kxyz = rp.kx | (rp.ky << 2) | (rp.kz << 4) | (any ? 64 : 0);
+  const int kz_any = rp.kz | (any ? 4 : 0);
   const uint32_t* leafq_w = ctx.leafq - lane;
-  const int qs = ctx.lds_stride;
+  constexpr int qs = kBlock;
   for (int base = 0; base < total; base += 64) {
     const int k = base + lane;
     // owner: the number of lanes whose items all lie below k
@@ -247,37 +270,25 @@ __device__ inline void flush_wave(const SceneDev& S, TraceCtx& ctx, const RayPre
     r.Sx = __shfl(rp.Sx, owner);
     r.Sy = __shfl(rp.Sy, owner);
     r.Sz = __shfl(rp.Sz, owner);
-    const int kk = __shfl(kxyz, owner);
-    r.kx = kk & 3;
-    r.ky = (kk >> 2) & 3;
-    r.kz = (kk >> 4) & 3;
-    const bool any_o = (kk & 64) != 0;
+    const int kk = __shfl(kz_any, owner);
+    r.kz = kk & 3;
+    const bool any_o = (kk & 4) != 0;
     const float bt_o = __shfl(best_t, owner);
     const uint32_t bid_o = (uint32_t)__shfl((int)best_id, owner);
     unsigned long long bkey = ~0ull;
     float bu = 0.0f, bv = 0.0f;
     if (k < total) {
-      const uint32_t c = leafq_w[owner + qi * qs];
-      uint32_t cur = leaf_first(c);
-      for (uint32_t left = leaf_count(c); left > 0u; --left, ++cur) {
-        ctx.n_tris++;
-        const TriRecord& tr = S.tris[cur];
-        float4 a = *reinterpret_cast<const float4*>(tr.v0);
-        float4 b = *reinterpret_cast<const float4*>(tr.v1);
-        float4 e = *reinterpret_cast<const float4*>(tr.v2);
-        float tt, uu, vv;
-        if (!tri_intersect(r, F3{a.x, a.y, a.z}, F3{b.x, b.y, b.z}, F3{e.x, e.y, e.z}, &tt, &uu, &vv)) continue;
+      ctx.n_tris++;
+      const TriRecord& tr = S.tris[leafq_w[owner + qi * qs]];
+      const float4 a = *reinterpret_cast<const float4*>(tr.v0);
+      const float4 b = *reinterpret_cast<const float4*>(tr.v1);
+      const float4 e = *reinterpret_cast<const float4*>(tr.v2);
+      float tt;
+      if (tri_intersect(r, F3{a.x, a.y, a.z}, F3{b.x, b.y, b.z}, F3{e.x, e.y, e.z}, &tt, &bu, &bv)) {
         const uint32_t id = __float_as_uint(a.w);
         // inside (tmin, tmax) and better than the owner's hit so far
-        if (!(tt > tmin)) continue;
         const bool ok = any_o ? tt < bt_o : (tt < bt_o || (tt == bt_o && bid_o != kNoHit && id < bid_o));
-        if (!ok) continue;
-        const unsigned long long key = ((unsigned long long)__float_as_uint(tt) << 32) | id;
-        if (key < bkey) {
-          bkey = key;
-          bu = uu;
-          bv = vv;
-        }
+        if (tt > tmin && ok) bkey = ((unsigned long long)__float_as_uint(tt) << 32) | id;
       }
     }
     if (bkey != ~0ull) {
@@ -335,7 +346,7 @@ __device__ inline void trace_run(const SceneDev& S, TraceCtx& ctx, F3 o, F3 d, F
   const F3 dq = (keep & kTsSecond) ? d2 : d;
   bool anyq = any && !(keep & kTsSecond);
   RayPre rp = ray_pre(o, dq);
-  float ix = safe_inv(dq.x), iy = safe_inv(dq.y), iz = safe_inv(dq.z);
+  float ix = slab_rcp(dq.x), iy = slab_rcp(dq.y), iz = slab_rcp(dq.z);
   float best_t = st.best_t, hu = st.u, hv = st.v;
   uint32_t best_id = st.best_id;
   uint32_t node = st.node;
@@ -343,18 +354,22 @@ __device__ inline void trace_run(const SceneDev& S, TraceCtx& ctx, F3 o, F3 d, F
   int nq = (int)((st.bits >> 8) & 0xFu);
   bool inner_done = (st.bits & kTsInnerDone) != 0u;
   bool found = (st.bits & kTsFound) != 0u;
+  bool chain = (keep & kTsChain) != 0u;
   int n_keep = 0;
-  if (keep64 > 0) n_keep = (__popcll(__ballot(!inner_done || nq > 0 || (keep & kTsChain))) * keep64) >> 6;
-  const int qs = ctx.lds_stride;
+  if (keep64 > 0) n_keep = (__popcll(__builtin_amdgcn_ballot_w64(!inner_done || nq > 0 || chain)) * keep64) >> 6;
+  constexpr int qs = kBlock;
+  lds_u32* const stack = lds_ptr(ctx.lds);
+  lds_u32* const leafq = lds_ptr(ctx.leafq);
   for (;;) {
     // ---- the first query of a chained pair has ended: start the second ----
-    if ((keep & kTsChain) && inner_done && nq == 0) {
+    if (chain && inner_done && nq == 0) {
+      chain = false;
       keep = kTsSecond | (best_id != kNoHit ? kTsFirstHit : 0u);
       anyq = false;
       rp = ray_pre(o, d2);
-      ix = safe_inv(d2.x);
-      iy = safe_inv(d2.y);
-      iz = safe_inv(d2.z);
+      ix = slab_rcp(d2.x);
+      iy = slab_rcp(d2.y);
+      iz = slab_rcp(d2.z);
       best_t = tmax2;
       hu = 0.0f;
       hv = 0.0f;
@@ -367,54 +382,70 @@ __device__ inline void trace_run(const SceneDev& S, TraceCtx& ctx, F3 o, F3 d, F
     // ---- visit one inner node (lanes with room in their leaf queue) ----
     if (!inner_done && nq <= kLeafQueue - 4) {
       ctx.n_nodes++;
-      const float4* np = reinterpret_cast<const float4*>(S.nodes + node);
-      float4 lox = np[0], loy = np[1], loz = np[2], hix = np[3], hiy = np[4], hiz = np[5];
-      uint4 ch = reinterpret_cast<const uint4*>(np)[6];
-      float lo_x[4] = {lox.x, lox.y, lox.z, lox.w}, lo_y[4] = {loy.x, loy.y, loy.z, loy.w};
-      float lo_z[4] = {loz.x, loz.y, loz.z, loz.w}, hi_x[4] = {hix.x, hix.y, hix.z, hix.w};
-      float hi_y[4] = {hiy.x, hiy.y, hiy.z, hiy.w}, hi_z[4] = {hiz.x, hiz.y, hiz.z, hiz.w};
-      uint32_t cid[4] = {ch.x, ch.y, ch.z, ch.w};
-      float kt[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
-      uint32_t kc[4] = {kEmpty, kEmpty, kEmpty, kEmpty};
+      const uint4* np = reinterpret_cast<const uint4*>(S.qnodes + node);
+      const uint4 n0 = np[0], qx = np[1], qy = np[2], qz = np[3];
+      // offsets of the node's origin, widened for near and far planes
+      const float bx = fmaf(-o.x, S.qinv_scale, __uint_as_float(n0.x & 0xFFFFF800u)) * ix;
+      const float by =
+          fmaf(-o.y, S.qinv_scale, __uint_as_float(__builtin_amdgcn_alignbit(n0.x, n0.y, 11) & 0xFFFFF800u)) * iy;
+      const float bz = fmaf(-o.z, S.qinv_scale, __uint_as_float((n0.y << 10) & 0xFFFFF800u)) * iz;
+      const float bnx = fmaf(-kSlabWiden, fabsf(bx), bx), bfx = fmaf(kSlabWiden, fabsf(bx), bx);
+      const float bny = fmaf(-kSlabWiden, fabsf(by), by), bfy = fmaf(kSlabWiden, fabsf(by), by);
+      const float bnz = fmaf(-kSlabWiden, fabsf(bz), bz), bfz = fmaf(kSlabWiden, fabsf(bz), bz);
+      // near and far planes by the direction's signs
+      const bool px = ix >= 0.0f, py = iy >= 0.0f, pz = iz >= 0.0f;
+      const uint32_t nx[2] = {px ? qx.x : qx.z, px ? qx.y : qx.w}, fx[2] = {px ? qx.z : qx.x, px ? qx.w : qx.y};
+      const uint32_t ny[2] = {py ? qy.x : qy.z, py ? qy.y : qy.w}, fy[2] = {py ? qy.z : qy.x, py ? qy.w : qy.y};
+      const uint32_t nz[2] = {pz ? qz.x : qz.z, pz ? qz.y : qz.w}, fz[2] = {pz ? qz.z : qz.x, pz ? qz.w : qz.y};
+      const float tmin_q = tmin * S.qinv_scale, tmax_q = best_t * S.qinv_scale;
+      const uint32_t ni = n0.z >> kQCountShift, nc = ni + (n0.w >> kQCountShift);
+      const uint32_t child0 = n0.z & kQIndexMask;
+      const uint32_t leaf0 = (n0.w & kQIndexMask) - ni;  // slot s >= ni: triangle record leaf0 + s
+      // hit inner children as sort keys: the entry distance's bits (t > 0
+      // sorts as an integer) with the slot in the two lowest
+      uint32_t key[4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        float t0x = (lo_x[s] - o.x) * ix, t1x = (hi_x[s] - o.x) * ix;
-        float t0y = (lo_y[s] - o.y) * iy, t1y = (hi_y[s] - o.y) * iy;
-        float t0z = (lo_z[s] - o.z) * iz, t1z = (hi_z[s] - o.z) * iz;
-        float tn = fmaxf(fmaxf(fminf(t0x, t1x), fminf(t0y, t1y)), fmaxf(fminf(t0z, t1z), tmin));
-        float tf = fminf(fminf(fmaxf(t0x, t1x), fmaxf(t0y, t1y)), fminf(fmaxf(t0z, t1z), best_t));
-        uint32_t c = cid[s];
-        bool hit = c != kEmpty && tn <= tf * kSlabScale;
-        if (hit && (c & kLeafBit)) {
-          ctx.leafq[nq * qs] = c;
-          ++nq;
-        }
-        if (hit && !(c & kLeafBit)) {
-          kt[s] = tn;
-          kc[s] = c;
-        }
+      for (uint32_t s = 0; s < 4; ++s) {
+        const float tx = fmaf(half_of(nx[s >> 1], s & 1u), ix, bnx), ux = fmaf(half_of(fx[s >> 1], s & 1u), ix, bfx);
+        const float ty = fmaf(half_of(ny[s >> 1], s & 1u), iy, bny), uy = fmaf(half_of(fy[s >> 1], s & 1u), iy, bfy);
+        const float tz = fmaf(half_of(nz[s >> 1], s & 1u), iz, bnz), uz = fmaf(half_of(fz[s >> 1], s & 1u), iz, bfz);
+        const float tn = fmaxf(fmaxf(tx, ty), fmaxf(tz, tmin_q));
+        const float tf = fminf(fminf(ux, uy), fminf(uz, tmax_q));
+        const bool hit = tn <= tf;
+        const bool inner = s < ni;
+        key[s] = hit && inner ? (__float_as_uint(tn) & ~3u) | s : kNoChild;
+        // the entry behind the last is written anyway and counts only for a
+        // hit leaf (kLeafQueue - 4 entries at most are queued here)
+        leafq[nq * qs] = leaf0 + s;
+        nq += hit && !inner && s < nc ? 1 : 0;
       }
       // 4-element sorting network, near to far
 #define TR_CSWAP(i, j)                                                   \
-      if (kt[j] < kt[i]) {                                               \
-        float _t = kt[i]; kt[i] = kt[j]; kt[j] = _t;                     \
-        uint32_t _c = kc[i]; kc[i] = kc[j]; kc[j] = _c;                  \
+      {                                                                  \
+        const uint32_t _a = key[i], _b = key[j];                         \
+        key[i] = _a < _b ? _a : _b;                                      \
+        key[j] = _a < _b ? _b : _a;                                      \
       }
       TR_CSWAP(0, 1) TR_CSWAP(2, 3) TR_CSWAP(0, 2) TR_CSWAP(1, 3) TR_CSWAP(1, 2)
 #undef TR_CSWAP
-      if (kc[0] != kEmpty) {
-        int npush = (kc[1] != kEmpty) + (kc[2] != kEmpty) + (kc[3] != kEmpty);
-        if (sp + npush > ctx.cap) {
-          // unreachable: the host refuses a launch whose BVH needs more than
-          // `cap` entries (stack_need, computed at build time); this branch
-          // only keeps the stack in bounds
-          inner_done = true;
-        } else {
-          if (kc[3] != kEmpty) stack_push(ctx, sp, kc[3]);
-          if (kc[2] != kEmpty) stack_push(ctx, sp, kc[2]);
-          if (kc[1] != kEmpty) stack_push(ctx, sp, kc[1]);
-          node = kc[0];
+      if (__builtin_amdgcn_ballot_w64(sp > kStackLds - 3) == 0ull) {
+        // room in LDS for three more entries on every lane: the far children
+        // are written unconditionally and the top moves past the hit ones
+#pragma unroll
+        for (int j = 3; j > 0; --j) {
+          stack[sp * qs] = child0 + (key[j] & 3u);
+          sp += key[j] != kNoChild ? 1 : 0;
         }
+      } else {
+        // sp < cap always holds: the host refuses a launch whose BVH needs
+        // more than `cap` entries (stack_need, computed at build time); the
+        // test only keeps the stack in bounds
+#pragma unroll
+        for (int j = 3; j > 0; --j)
+          if (key[j] != kNoChild && sp < ctx.cap) stack_push(ctx, sp, child0 + (key[j] & 3u));
+      }
+      if (key[0] != kNoChild) {
+        node = child0 + (key[0] & 3u);
       } else if (sp > 0) {
         node = stack_pop(ctx, sp);
       } else {
@@ -423,18 +454,18 @@ __device__ inline void trace_run(const SceneDev& S, TraceCtx& ctx, F3 o, F3 d, F
     }
     // ---- decide, wave-wide, whether queued leaves are tested now ----
     const bool pend = nq > 0;
-    const bool live = !inner_done || pend || (keep & kTsChain);
-    const uint64_t m_live = __ballot(live);
+    const bool live = !inner_done || pend || chain;
+    const uint64_t m_live = __builtin_amdgcn_ballot_w64(live);
     if (m_live == 0ull) break;
     if (__popcll(m_live) <= n_keep) break;
-    const uint64_t m_pend = __ballot(pend);
-    const uint64_t m_urgent = __ballot(pend && (inner_done || nq > kLeafQueue - 4));
+    const uint64_t m_pend = __builtin_amdgcn_ballot_w64(pend);
+    const uint64_t m_urgent = __builtin_amdgcn_ballot_w64(pend && (inner_done || nq > kLeafQueue - 4));
     bool flush;
     if constexpr (kWave) {
       // a wave-wide flush costs one round for up to 64 leaves: wait until
       // kWaveStall64/64 of the live lanes are stalled on their queue,
       // kWavePend64/64 have leaves queued, or no lane can visit a node
-      const uint64_t m_visit = __ballot(!inner_done && nq <= kLeafQueue - 4);
+      const uint64_t m_visit = __builtin_amdgcn_ballot_w64(!inner_done && nq <= kLeafQueue - 4);
       flush = m_visit == 0ull || __popcll(m_urgent) * 64 >= kWaveStall64 * __popcll(m_live) ||
               __popcll(m_pend) * 64 >= kWavePend64 * __popcll(m_live);
     } else {
@@ -447,20 +478,9 @@ __device__ inline void trace_run(const SceneDev& S, TraceCtx& ctx, F3 o, F3 d, F
         if (found) inner_done = true;
       }
     } else if (flush && pend) {
-      int qi = 0;
-      uint32_t cur = 0u, left = 0u;
-      for (;;) {
-        if (left == 0u) {
-          if (qi == nq) break;
-          const uint32_t c = ctx.leafq[qi * qs];
-          ++qi;
-          cur = leaf_first(c);
-          left = leaf_count(c);
-        }
+      for (int qi = 0; qi < nq; ++qi) {
         ctx.n_tris++;
-        const TriRecord& tr = S.tris[cur];
-        ++cur;
-        --left;
+        const TriRecord& tr = S.tris[leafq[qi * qs]];
         float4 a = *reinterpret_cast<const float4*>(tr.v0);
         float4 b = *reinterpret_cast<const float4*>(tr.v1);
         float4 e = *reinterpret_cast<const float4*>(tr.v2);

@@ -30,6 +30,7 @@
 #include <cfloat>
 
 #include "../trc_internal.h"
+#include "../common/tr_bsdf.h"
 
 namespace trc {
 
@@ -136,7 +137,7 @@ __global__ void k_vertex_normals(const TriShade* shade, const uint32_t* off, con
 
 // One lane: the emitter table is a handful of triangles.
 __global__ void k_light_table(const TriShade* shade, const int32_t* light_tri, const float* emit_rad, float* light_f,
-                              float* light_cdf, int32_t NL, UpdateScalars* out) {
+                              float* light_cdf, float* light_pdf, int32_t NL, UpdateScalars* out) {
   if (blockIdx.x != 0 || threadIdx.x != 0) return;
   float integral = 0.0f;
   if (NL > 0) {
@@ -155,6 +156,7 @@ __global__ void k_light_table(const TriShade* shade, const int32_t* light_tri, c
     integral = light_cdf[NL - 1];
     if (integral > 0.0f)
       for (int32_t i = 0; i < NL; ++i) light_cdf[i] = light_cdf[i] / integral;
+    for (int32_t i = 0; i < NL; ++i) light_pdf[i] = light_area_pdf(light_f[i], integral, NL, shade[light_tri[i]].area);
   }
   out->light_integral = integral;
 }
@@ -325,9 +327,10 @@ __global__ void k_tri_records(const float* pos, const uint32_t* idx, TriRecord* 
 }
 
 // One level of the refit: every node's child boxes from its leaves'
-// triangles or its children's (unpadded) boxes of the level below; nbox
-// keeps each node's unpadded box for its parent.
-__global__ void k_refit_level(Bvh4Node* nodes, float* nbox, const TriRecord* tris, const uint32_t* level_nodes,
+// triangles or its children's (unpadded) boxes of the level below, and the
+// quantized node the traversal reads; nbox keeps each node's unpadded box
+// for its parent.
+__global__ void k_refit_level(Bvh4Node* nodes, QNode* qnodes, float inv_scale, float* nbox, const TriRecord* tris, const uint32_t* level_nodes,
                               uint32_t count) {
   const uint32_t j = blockIdx.x * kUpdBlock + threadIdx.x;
   if (j >= count) return;
@@ -361,6 +364,7 @@ __global__ void k_refit_level(Bvh4Node* nodes, float* nbox, const TriRecord* tri
     n.hiz[s] = pad_hi(cb.hi[2]);
     all.grow(cb);
   }
+  qnodes[ni] = quantize_node(n, inv_scale);
   float* o = nbox + 6 * (size_t)ni;
   for (int k = 0; k < 3; ++k) {
     o[k] = all.lo[k];
@@ -445,7 +449,8 @@ hipError_t launch_scene_update(const SceneDev& S, const SceneUpdateDev& U, hipSt
     hipLaunchKernelGGL(k_vertex_normals, dim3(blocks_for(V)), dim3(kUpdBlock), 0, st, (const TriShade*)shade,
                        U.vs_off, U.vs_list, const_cast<float*>(S.vnrm), V);
   hipLaunchKernelGGL(k_light_table, dim3(1), dim3(1), 0, st, (const TriShade*)shade, S.light_tri, S.emit_rad,
-                     const_cast<float*>(S.light_f), const_cast<float*>(S.light_cdf), S.n_light, U.scal);
+                     const_cast<float*>(S.light_f), const_cast<float*>(S.light_cdf),
+                     const_cast<float*>(S.light_pdf), S.n_light, U.scal);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (U.n_edges > 0) {
@@ -459,8 +464,9 @@ hipError_t launch_scene_update(const SceneDev& S, const SceneUpdateDev& U, hipSt
   for (size_t l = 0; l + 1 < U.level_off.size(); ++l) {
     const uint32_t a = U.level_off[l], n = U.level_off[l + 1] - a;
     if (n == 0) continue;
-    hipLaunchKernelGGL(k_refit_level, dim3(blocks_for(n)), dim3(kUpdBlock), 0, st, nodes, U.nbox,
-                       (const TriRecord*)tris, U.refit_nodes + a, n);
+    hipLaunchKernelGGL(k_refit_level, dim3(blocks_for(n)), dim3(kUpdBlock), 0, st, nodes,
+                       const_cast<QNode*>(S.qnodes), S.qinv_scale, U.nbox, (const TriRecord*)tris, U.refit_nodes + a,
+                       n);
   }
   hipLaunchKernelGGL(k_zero_sah, dim3(1), dim3(1), 0, st, U.scal);
   hipLaunchKernelGGL(k_sah, dim3(blocks_for(U.n_nodes)), dim3(kUpdBlock), 0, st, (const Bvh4Node*)nodes, U.n_nodes,
