@@ -97,7 +97,8 @@ GradCopies make_grad_copies(int n_verts, hipStream_t st) {
 }
 
 // Words of a stream's spill buffer: the traversal stacks' spill area, then
-// the forward's tile counter (kTileCtrWords words, one used).
+// the launches' tile counters (kTileCtrWords words: one for the forward's
+// camera rays and for the other kernels, one for its bounces).
 constexpr size_t kTileCtrWords = 64;
 static size_t spill_words(int max_grid) { return (size_t)kSpillDepth * (size_t)max_grid * kBlock; }
 
@@ -790,6 +791,7 @@ static std::vector<JobDev> prepare_batch(trc_ctx* ctx, const trc_job* jobs, int3
     d.spp = J.opt.spp;
     d.first = J.first_path;
     d.count = J.num_paths;
+    d.range = adjoint ? PathRange{d.first, d.count, d.count, 0u, 0u} : path_range(C, d.first, d.count);
     d.paths = J.paths;
     d.ckpt = J.ckpt;
     d.dLdI = J.dLdI;
@@ -868,7 +870,7 @@ static uint64_t assign_tiles(std::vector<JobDev>& jd, uint64_t tile) {
   uint64_t ntiles = 0;
   for (JobDev& d : jd) {
     d.tile0 = ntiles;
-    if (!d.solo) ntiles += (d.count + tile - 1) / tile;
+    if (!d.solo) ntiles += (d.range.slots + tile - 1) / tile;
   }
   return ntiles;
 }

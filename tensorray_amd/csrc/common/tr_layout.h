@@ -245,6 +245,29 @@ struct CameraDev {
   int32_t width, height;
 };
 
+// Paths of a launch in its order of slots: path indices first .. first +
+// count, or (blocked, whole samples only) the 8 x 8 pixel blocks of the image
+// sample by sample, 64 slots each, some of them empty at the ragged edges.
+struct PathRange {
+  uint64_t first, count;  // paths
+  uint64_t slots;
+  uint32_t blocked;
+  uint32_t pad;
+};
+// Blocks keep the rays and bounces of a wave closer together than a row of 64
+// pixels does; not where the edges would leave more than an eighth of the
+// slots empty.
+inline PathRange path_range(const CameraDev& C, uint64_t first, uint64_t count) {
+  PathRange r{first, count, count, 0u, 0u};
+  const uint64_t W = (uint64_t)C.width, H = (uint64_t)C.height, wh = W * H;
+  const uint64_t slots = count / wh * (((W + 7) / 8) * ((H + 7) / 8) * 64);
+  if (first % wh == 0 && count % wh == 0 && slots * 8 <= count * 9) {
+    r.slots = slots;
+    r.blocked = 1u;
+  }
+  return r;
+}
+
 struct SceneDev {
   const float* pos;
   const uint32_t* idx;

@@ -262,25 +262,33 @@ __device__ F3 path_forward(const SceneDev& S, const CameraDev& C, const PathPara
 }
 
 // ---------------------------------------------------------------------------
-// Forward paths as a per-lane state machine with path regeneration.
+// Forward paths in two passes.
 //
-// path_forward runs one path to completion per lane, so a wave waits for its
-// longest path and every traversal is entered by whichever lanes still live.
-// Here each loop iteration advances one query per lane -- the camera ray, or
-// the two rays of a bounce (the NEE shadow ray, then the BSDF-sampled ray,
-// as one chained query from the vertex) -- and shades the lanes whose query
-// has finished; a lane whose path ends takes the next path of its wave's
-// chunk (ballot + popcount hand-out, no global atomics).  A query that is
-// still running when most of the wave's have finished keeps its traversal
-// state and continues in the next iteration.  Each path evaluates the same
-// expressions in the same order as path_forward<false>, so the per-path
-// radiance is identical.
+// The primary pass (trace_primary) traces the camera rays of 64 neighbouring
+// paths per wave and leaves each path's first hit where its radiance will go.
+// The bounce pass (render_bounces) runs the surviving paths as a per-lane
+// state machine with path regeneration: each loop iteration traces the two
+// rays of a bounce per lane (the NEE shadow ray, then the BSDF-sampled ray, as
+// one chained query from the vertex) and shades the lanes whose query has
+// finished; a lane whose path ends takes the next surviving path of its
+// wave's tiles and joins the others at the next bounce's set-up.  A query
+// that is still running when most of the wave's have finished keeps its
+// traversal state and continues in the next iteration.  Each path evaluates
+// the same expressions in the same order as path_forward<false>, so the
+// per-path radiance is identical.
+//
+// One pass whose lanes trace either a camera ray or a bounce shades both
+// kinds in every iteration, each at the lanes of its kind (about half), and
+// carries the camera rays that miss.
 // ---------------------------------------------------------------------------
-enum PathStage : uint32_t { kStageIdle = 0, kStageCamera = 1, kStageBounce = 2 };
+enum PathStage : uint32_t { kStageIdle = 0, kStageBounce = 1 };
 
 // Fraction (of 64) of a wave's queries still unfinished at which the wave
 // stops traversing and shades the finished ones.
-constexpr int kTraceKeep64 = 16;
+// (closed room / 512 x 512 step / large-mesh step / eight views at 16: 1.25 /
+// 3.38 / 5.27 / 1.73 ms, at 20: 1.24 / 3.35 / 5.18 / 1.74, at 24 and 5 waves
+// per SIMD: 1.42 / 3.42 / 5.11 / 1.82 against 1.40 / 3.44 / 5.25 / 1.79 at 16)
+constexpr int kTraceKeep64 = 20;
 
 struct PathLane {
   uint64_t path;
@@ -299,9 +307,9 @@ struct PathLane {
   int32_t li;
   float ld2;
   float pdfb;            // pdf of the BSDF direction d2 of bounce b
-  // query of this iteration from o (tmin = kShadowEpsilon): the camera ray
-  // along d, or the bounce's shadow ray along d (any hit) chained with its
-  // BSDF-sampled ray along d2; the traversal state holds the far bound
+  // query of this iteration from o (tmin = kShadowEpsilon): the bounce's
+  // shadow ray along d (any hit) chained with its BSDF-sampled ray along d2;
+  // the traversal state holds the far bound
   F3 o, d, d2;
   TraceState ts;
 };
@@ -327,37 +335,46 @@ __device__ inline NeeGeo nee_geo(const SceneDev& S, const Its& its, float la, fl
   return g;
 }
 
-// The path ranges a wave renders: tiles t, t + step, ... (below tile `tend`)
-// of `tile` paths each, tile k covering [base + k*tile, ...) clipped to
-// `limit`.  The wave moves to its next tile as soon as the current one is
-// handed out, without waiting for its lanes to drain.  All fields are
-// wave-uniform.
+// How the slots of a launch are cut into tiles: `nbig` tiles of `big` slots,
+// then tiles of `tile`.  One counter serves an atomic every 11.5 ns (65,536
+// tiles of 64 paths: 0.755 ms, whatever the paths cost), so most slots go out
+// in big tiles and the last ones in small ones, which let the waves finish
+// together.
+struct TileDeal {
+  uint64_t slots, nbig, ntiles;
+  uint32_t big, tile;
+};
+
+// The path ranges a wave renders: its tiles of a range of slots that starts at
+// tile t0 of the launch.  The wave moves to its next tile as soon as the
+// current one is handed out, without waiting for its lanes to drain.  All
+// fields are wave-uniform.
 struct TileSupply {
-  uint64_t next, end;            // paths not yet handed out of the current tile
+  uint64_t next, end;            // slots not yet handed out of the current tile
   uint64_t t, tend, step;        // tile cursor
-  uint64_t base, limit, tile, t0;
+  uint64_t t0;
+  TileDeal deal;
   // tile counter: when set, the wave's tiles after its first (tile t, one
   // per wave: tiles 0 .. step-1 of the launch are dealt so) are step + the
   // counter's next value, taken as the wave needs one; otherwise t,
   // t + step, ...  Tile numbers count over the whole launch.
   uint32_t* ctr;
   __device__ void load() {
-    next = base + (t - t0) * tile;
-    end = next + tile < limit ? next + tile : limit;
+    const uint64_t k = t - t0;
+    next = k < deal.nbig ? k * deal.big : deal.nbig * deal.big + (k - deal.nbig) * deal.tile;
+    end = next + (k < deal.nbig ? deal.big : deal.tile);
+    end = end < deal.slots ? end : deal.slots;
   }
-  // Starts at tile t; tiles t0.. map to paths base..limit.
-  __device__ static TileSupply make(uint64_t t, uint64_t tend, uint64_t step, uint64_t t0, uint64_t base,
-                                    uint64_t limit, uint64_t tile) {
+  // Starts at tile t.
+  __device__ static TileSupply make(uint64_t t, uint64_t step, uint64_t t0, const TileDeal& deal, uint32_t* ctr) {
     TileSupply s;
     s.t = t;
-    s.tend = tend;
+    s.tend = t0 + deal.ntiles;
     s.step = step;
     s.t0 = t0;
-    s.base = base;
-    s.limit = limit;
-    s.tile = tile;
-    s.ctr = nullptr;
-    if (t < tend) s.load();
+    s.deal = deal;
+    s.ctr = ctr;
+    if (t < s.tend) s.load();
     else s.next = s.end = 0;
     return s;
   }
@@ -384,13 +401,83 @@ struct TileSupply {
   }
 };
 
+// The first hit of a path between the passes, in the three words of its
+// radiance: (triangle + 1, u, v); zero for a camera ray that missed, whose
+// radiance that is.
+__device__ inline void put_first_hit(float* w, const Hit& h) {
+  w[0] = __uint_as_float((uint32_t)(h.tri + 1));
+  w[1] = h.u;
+  w[2] = h.v;
+}
+
+// 64 slots of a range.  All fields are wave-uniform.
+struct PathGroup {
+  uint64_t base;     // path of offset 0
+  uint32_t cols, rows;  // blocked: pixels of the block inside the image; else cols = paths, rows = 0
+  uint32_t width;
+  __device__ static PathGroup linear(uint64_t first, uint64_t end) {
+    PathGroup g;
+    g.base = first;
+    g.cols = end - first < 64u ? (uint32_t)(end - first) : 64u;
+    g.rows = 0u;
+    g.width = 0u;
+    return g;
+  }
+  // block `k` of the blocks of all samples from path `first` on (a multiple of W * H)
+  __device__ static PathGroup block(const CameraDev& C, uint64_t first, uint64_t k) {
+    const uint32_t W = (uint32_t)C.width, H = (uint32_t)C.height;
+    const uint32_t bx = (W + 7u) / 8u, nb = bx * ((H + 7u) / 8u);
+    const uint64_t s = k / nb;
+    const uint32_t r = (uint32_t)(k - s * nb), by = r / bx, x = (r - by * bx) * 8u, y = by * 8u;
+    PathGroup g;
+    g.base = first + s * ((uint64_t)W * H) + (uint64_t)y * W + x;
+    g.cols = W - x < 8u ? W - x : 8u;
+    g.rows = H - y < 8u ? H - y : 8u;
+    g.width = W;
+    return g;
+  }
+  // the group of slots i .. i + 63 (i a multiple of 64)
+  __device__ static PathGroup at(const CameraDev& C, const PathRange& R, uint64_t i) {
+    return R.blocked ? block(C, R.first, i >> 6) : linear(R.first + i, R.first + R.count);
+  }
+  __device__ bool has(uint32_t j) const { return rows ? (j & 7u) < cols && (j >> 3) < rows : j < cols; }
+  __device__ uint64_t path(uint32_t j) const { return base + (rows ? (j >> 3) * width + (j & 7u) : j); }
+};
+
+// The primary pass over one group: camera rays of the box filter (the sample
+// stays inside its pixel) and first hits, from the group's 64 lanes at once.
+// `paths` points at the words of path `paths_first`.
+template <bool kCkpt>
+__device__ inline void trace_primary(const SceneDev& S, const CameraDev& C, const PathParams& P, TraceCtx& tc, const PathGroup& g,
+                                     const CkptDev& ck, float* paths, uint64_t paths_first) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const bool has = g.has(lane);
+  const uint64_t path = has ? g.path(lane) : g.base;
+  const uint32_t pix = (uint32_t)(path % ((uint32_t)C.width * (uint32_t)C.height));
+  const uint32_t px = pix % (uint32_t)C.width, py = pix / (uint32_t)C.width;
+  const Rnd4 rc = rng4(P.seed, kRngInterior, path, 0u);
+  const F3 eye{C.eye[0], C.eye[1], C.eye[2]};
+  const F3 d = camera_dir(C, (float)px + rc.a, (float)py + rc.b);
+  TraceState ts;
+  if (has) trace_begin(ts, 1e32f);
+  else trace_none(ts);
+  trace_run<true>(S, tc, eye, d, d, 1e32f, kShadowEpsilon, false, ts, 0);
+  const Hit h = trace_hit(ts);
+  if (!has) return;
+  put_first_hit(paths + 3 * (path - paths_first), h);
+  if (kCkpt) {
+    ck.meta[path] = h.tri < 0 ? 0u : 1u;
+    if (h.tri >= 0) ckpt_put_vertex(ck, path, 0, h.tri, h.u, h.v);
+  }
+}
+
 // The BSDF-sampled ray of bounce b from `its` came back with hit `h`:
 // MIS-weighted emission, throughput update and the move to the next vertex,
 // or the end of the path (Integrator.cpp:232-293).  ret: the bounce's NEE
-// contribution.  Returns true, with `its` replaced by the new vertex
-// x_{b+1}, when the path continues.
+// contribution.  Returns true when the path continues from the new vertex
+// x_{b+1} (L.tri, L.u, L.v).
 template <bool kCkpt, class Finish>
-__device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const CkptDev& ck, Its& its, F3 wo,
+__device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const CkptDev& ck, const Its& its, F3 wo,
                                 const Hit& h, F3 ret, PathLane& L, uint32_t& meta, Finish& finish) {
   const F3 zero{0.0f, 0.0f, 0.0f};
   bool ok = h.tri >= 0 && L.pdfb > 0.0f && bsdf_dir_valid(S, its, L.d2);
@@ -435,107 +522,43 @@ __device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const Ck
     L.set_stage(kStageIdle);
     return false;
   }
-  its = its2;
   return true;
 }
 
-// The wave renders the paths of its tile supply.  A bounce is two ray
-// queries, the shadow ray of next-event estimation and the BSDF-sampled
-// ray, traced as one chained query and shaded together.
+// The bounce pass: the wave renders the surviving paths of its tile supply,
+// which counts slots of the launch's order of paths R.  A bounce is
+// two ray queries, the shadow ray of next-event estimation and the
+// BSDF-sampled ray, traced as one chained query and shaded together.
 template <bool kCkpt, class Finish>
-__device__ void render_paths_regen(const SceneDev& S, const CameraDev& C, const PathParams& P, TraceCtx& tc,
-                                   TileSupply& sup, const CkptDev& ck, Finish finish) {
+__device__ void render_bounces(const SceneDev& S, const CameraDev& C, const PathParams& P, TraceCtx& tc,
+                               TileSupply& sup, const PathRange& R, const CkptDev& ck, const float* paths,
+                               uint64_t paths_first, Finish finish) {
   const F3 zero{0.0f, 0.0f, 0.0f};
-  const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
   const F3 eye{C.eye[0], C.eye[1], C.eye[2]};
   const F3 cdir{C.dir[0], C.dir[1], C.dir[2]};
-  const int lane = (int)(threadIdx.x & 63u);
+  const uint32_t lane = threadIdx.x & 63u;
   PathLane L;
   L.sb = kStageIdle;
   trace_none(L.ts);
   uint32_t meta = 0u;  // checkpoint meta word of the current path
+  // the current group's surviving paths, not yet handed out from `pool_next`
+  // on: lane r holds the offset of the r-th
+  PathGroup group{};
+  uint32_t pool = 0u, pool_next = 0u, pool_n = 0u;
   for (;;) {
-    // ---- regenerate: idle lanes take the next paths of the wave's tiles ----
-    if (sup.next >= sup.end) sup.more();
-    const uint64_t next = sup.next, end = sup.end;
-    const bool idle = L.stage() == kStageIdle;
-    const uint64_t idle_mask = __ballot(idle);
-    if (idle) {
-      const uint64_t rank = (uint64_t)__popcll(idle_mask & ((1ull << lane) - 1ull));
-      if (next + rank < end) {
-        L.path = next + rank;
-        const uint32_t pix = (uint32_t)(L.path % WH);
-        const uint32_t px = pix % (uint32_t)C.width, py = pix / (uint32_t)C.width;
-        Rnd4 rc = rng4(P.seed, kRngInterior, L.path, 0u);
-        L.sb = kStageCamera;  // b = 0
-        L.o = eye;
-        L.d = camera_dir(C, (float)px + rc.a, (float)py + rc.b);
-        trace_begin(L.ts, 1e32f);
-      }
-    }
-    {
-      const uint64_t n_idle = (uint64_t)__popcll(idle_mask);
-      sup.next = next + n_idle < end ? next + n_idle : end;
-    }
-    if (__ballot(L.stage() != kStageIdle) == 0ull) break;
-    // ---- one query per lane ----
+    // ---- one chained query per lane ----
     // The wave leaves the traversal loop once at most kTraceKeep64 / 64 of
     // its queries are unfinished; those lanes skip shading and resume their
     // query in the next iteration, beside the new rays of the others.
     // (a BSDF direction of pdf 0 ends the path whatever it hits: its query
     // is given an empty interval)
-    trace_run<true>(S, tc, L.o, L.d, L.d2, (L.sb & 4u) ? 1e32f : -1.0f, kShadowEpsilon,
-                    L.stage() == kStageBounce, L.ts, kTraceKeep64);
-    if (!trace_finished(L.ts)) continue;
-    const Hit h = trace_hit(L.ts);
-    // ---- shade ----
-    // Both stages start from one surface interaction -- the first vertex for
-    // a camera ray, the current vertex x_b for a bounce -- and end with the
-    // next bounce's set-up (light sample, shadow ray, BSDF direction), each
-    // evaluated once for the whole wave.
-    const uint32_t stage = L.stage();
-    if (stage == kStageIdle) continue;  // no path left for this lane
-    const bool cam = stage == kStageCamera;
-    if (cam && h.tri < 0) {
-      if (kCkpt) ck.meta[L.path] = 0u;
-      finish(L.path, zero);
-      L.set_stage(kStageIdle);
-      continue;
-    }
-    Its its = post_intersect(S, cam ? h.tri : L.tri, cam ? h.u : L.u, cam ? h.v : L.v);
-    if (cam) {
-      if (kCkpt) {
-        ckpt_put_vertex(ck, L.path, 0, h.tri, h.u, h.v);
-        meta = 1u;
-      }
-      float beta0;
-      {
-        F3 cd = its.p - eye;
-        float dist;
-        cd = over_sqrt(cd, len2(cd), &dist);
-        L.raydir = cd;
-        float cosy = dot(cd, cdir);
-        float cosx = dot(-cd, its.ng);
-        float G = fabsf(cosx) / (cosy * cosy * cosy * (dist * dist));
-        beta0 = ratio_self(G) * ratio_self(S.shade[its.tri].area);
-      }
-      L.beta = F3{beta0, beta0, beta0};
-      L.contrib = zero;
-      if (its.emitter >= 0) {
-        F3 Le = emitted(S, its.emitter, its.ng, -L.raydir);
-        F3 e0 = L.beta * Le;
-        if (finite3(e0)) L.contrib = L.contrib + e0;
-      }
-      L.tri = h.tri; L.u = h.u; L.v = h.v;
-      if (P.max_bounces <= 0) {
-        if (kCkpt) ck.meta[L.path] = meta;
-        finish(L.path, L.contrib);
-        L.set_stage(kStageIdle);
-        continue;
-      }
-    } else {
-      // next-event estimation of bounce b (Integrator.cpp:196-230) with the
-      // traced shadow ray's outcome, then the BSDF-sampled ray's hit
+    trace_run<true>(S, tc, L.o, L.d, L.d2, (L.sb & 4u) ? 1e32f : -1.0f, kShadowEpsilon, true, L.ts, kTraceKeep64);
+    bool setup = false;  // the lane stands at a vertex whose bounce is to be set up
+    if (L.stage() == kStageBounce && trace_finished(L.ts)) {
+      // ---- shade: next-event estimation of bounce b (Integrator.cpp:196-230)
+      // with the traced shadow ray's outcome, then the BSDF-sampled ray's hit
+      const Hit h = trace_hit(L.ts);
+      const Its its = post_intersect(S, L.tri, L.u, L.v);
       const F3 wo = -L.raydir;
       const TriShade& lsh = S.shade[S.light_tri[L.li]];
       const F3 ln{lsh.n[0], lsh.n[1], lsh.n[2]};
@@ -555,21 +578,92 @@ __device__ void render_paths_regen(const SceneDev& S, const CameraDev& C, const 
       val = val * mis;
       F3 ret = zero;
       ret = ret + val;
-      if (!bsdf_hit<kCkpt>(S, P, ck, its, wo, h, ret, L, meta, finish)) continue;
+      setup = bsdf_hit<kCkpt>(S, P, ck, its, wo, h, ret, L, meta, finish);
     }
-    // ---- bounce b at `its`: light sample, shadow ray and BSDF direction ----
-    // (Integrator.cpp:196-213 and 232-245; the draws of the reference's
-    // loop in its order: light sample 1 + 2b, BSDF sample 2 + 2b)
-    const Rnd4 rl = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b());
-    const NeeGeo g2 = nee_geo(S, its, rl.a, rl.b);
-    L.li = g2.ls.index;
-    L.ld2 = g2.d2;
-    const Rnd4 rb = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b() + 1u);
-    L.d2 = bsdf_sample(S, its, -L.raydir, rb.a, rb.b, &L.pdfb);
-    L.sb = (L.sb & ~15u) | kStageBounce | (L.pdfb > 0.0f ? 4u : 0u) | (g2.ray ? 8u : 0u);
-    L.o = its.p;
-    L.d = g2.wi;
-    trace_begin_chain(L.ts, g2.ray ? g2.dist - kShadowEpsilon : -1.0f);
+    // ---- regenerate: idle lanes take the next surviving paths ----
+    const uint64_t idle_mask = __builtin_amdgcn_ballot_w64(L.stage() == kStageIdle);
+    if (idle_mask != 0ull) {
+      while (pool_next == pool_n) {
+        if (sup.next >= sup.end && !sup.more()) break;
+        group = PathGroup::at(C, R, sup.next);
+        sup.next += 64u;
+        const bool live = group.has(lane) && __float_as_uint(paths[3 * (group.path(lane) - paths_first)]) != 0u;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(live);
+        // lane r of the list: the r-th live lane (dead lanes write behind it)
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        pool_n = (uint32_t)__popcll(m);
+        pool_next = 0u;
+        pool = (uint32_t)__builtin_amdgcn_ds_permute((int)((live ? below : pool_n + lane - below) << 2), (int)lane);
+      }
+      const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle_mask >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)idle_mask, 0u));
+      const uint32_t off = (uint32_t)__shfl((int)pool, (int)((pool_next + rank) & 63u));
+      const bool take = L.stage() == kStageIdle && pool_next + rank < pool_n;
+      const uint32_t n_idle = (uint32_t)__popcll(idle_mask);
+      pool_next = pool_next + n_idle < pool_n ? pool_next + n_idle : pool_n;
+      if (take) {
+        L.path = group.path(off);
+        const float* w = paths + 3 * (L.path - paths_first);
+        L.tri = (int32_t)(__float_as_uint(w[0]) - 1u);
+        L.u = w[1];
+        L.v = w[2];
+        L.sb = kStageBounce;  // b = 0
+        meta = 1u;
+        setup = true;
+      }
+      if (__builtin_amdgcn_ballot_w64(L.stage() != kStageIdle) == 0ull) break;  // the supply is used up
+    }
+    if (setup) {
+      // The vertex is evaluated here, once for the lanes that continue and
+      // those that start, rather than kept from the shading above: its
+      // frame would be live through the hand-out.
+      const Its its = post_intersect(S, L.tri, L.u, L.v);
+      if (L.b() == 0u) {
+        // the first vertex (Integrator.cpp:55-73)
+        float beta0;
+        {
+          F3 cd = its.p - eye;
+          float dist;
+          cd = over_sqrt(cd, len2(cd), &dist);
+          L.raydir = cd;
+          float cosy = dot(cd, cdir);
+          float cosx = dot(-cd, its.ng);
+          float G = fabsf(cosx) / (cosy * cosy * cosy * (dist * dist));
+          beta0 = ratio_self(G) * ratio_self(S.shade[its.tri].area);
+        }
+        L.beta = F3{beta0, beta0, beta0};
+        L.contrib = zero;
+        if (its.emitter >= 0) {
+          F3 Le = emitted(S, its.emitter, its.ng, -L.raydir);
+          F3 e0 = L.beta * Le;
+          if (finite3(e0)) L.contrib = L.contrib + e0;
+        }
+      }
+      if (P.max_bounces <= 0) {
+        // no bounce: the path ends at its first vertex, and the lane takes
+        // another one in the next iteration
+        if (kCkpt) ck.meta[L.path] = meta;
+        finish(L.path, L.contrib);
+        L.set_stage(kStageIdle);
+        trace_none(L.ts);
+        continue;
+      }
+      // ---- bounce b at `its`: light sample, shadow ray and BSDF direction ----
+      // (Integrator.cpp:196-213 and 232-245; the draws of the reference's
+      // loop in its order: light sample 1 + 2b, BSDF sample 2 + 2b)
+      const Rnd4 rl = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b());
+      const NeeGeo g2 = nee_geo(S, its, rl.a, rl.b);
+      L.li = g2.ls.index;
+      L.ld2 = g2.d2;
+      const Rnd4 rb = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b() + 1u);
+      L.d2 = bsdf_sample(S, its, -L.raydir, rb.a, rb.b, &L.pdfb);
+      L.sb = (L.sb & ~15u) | kStageBounce | (L.pdfb > 0.0f ? 4u : 0u) | (g2.ray ? 8u : 0u);
+      L.o = its.p;
+      L.d = g2.wi;
+      trace_begin_chain(L.ts, g2.ray ? g2.dist - kShadowEpsilon : -1.0f);
+    }
+    // a lane without a path or query must not look live to the traversal
+    if (L.stage() == kStageIdle) trace_none(L.ts);
   }
 }
 

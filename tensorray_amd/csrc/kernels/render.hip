@@ -55,24 +55,39 @@ __global__ void __launch_bounds__(kBlock) k_intersect(SceneDev S, LaunchCfg L, c
   }
 }
 
+// Camera rays: a wave takes 64 slots at a time from the launch's counter.
 template <bool kCkpt>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWaves))) k_render_paths(SceneDev S, CameraDev C, PathParams P, LaunchCfg L,
-                                                         uint64_t first, uint64_t count, uint32_t tile, float* paths,
-                                                         uint64_t paths_first, CkptDev ck) {
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWaves)))
+k_primary(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, TileDeal deal, float* paths,
+          uint64_t paths_first, CkptDev ck) {
   __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
   TraceCtx tc = make_trace_ctx_wave(lds_stack, L);
-  // paths [first, first + count) in tiles of `tile` paths, dealt to the waves round-robin
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
   const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-  const uint64_t ntiles = (count + tile - 1) / tile;
-  TileSupply sup = TileSupply::make(wave, ntiles, nwaves, 0, first, first + count, tile);
-  sup.ctr = L.tiles;
-  render_paths_regen<kCkpt>(S, C, P, tc, sup, ck, [&](uint64_t p, F3 c) {
-    const uint64_t q = p - paths_first;
-    paths[3 * q] = c.x;
-    paths[3 * q + 1] = c.y;
-    paths[3 * q + 2] = c.z;
-  });
+  TileSupply sup = TileSupply::make(wave, nwaves, 0, deal, L.tiles);
+  while (sup.next < sup.end) {
+    trace_primary<kCkpt>(S, C, P, tc, PathGroup::at(C, R, sup.next), ck, paths, paths_first);
+    sup.next += 64u;
+    if (sup.next >= sup.end) sup.more();
+  }
+}
+
+template <bool kCkpt>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBounceWaves)))
+k_bounces(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, TileDeal deal, float* paths,
+          uint64_t paths_first, CkptDev ck) {
+  __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
+  TraceCtx tc = make_trace_ctx_wave(lds_stack, L);
+  const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
+  const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+  TileSupply sup = TileSupply::make(wave, nwaves, 0, deal, L.tiles ? L.tiles + 1 : nullptr);
+  render_bounces<kCkpt>(S, C, P, tc, sup, R, ck, paths, paths_first,
+                        [&](uint64_t p, F3 c) {
+                          const uint64_t q = p - paths_first;
+                          paths[3 * q] = c.x;
+                          paths[3 * q + 1] = c.y;
+                          paths[3 * q + 2] = c.z;
+                        });
 }
 
 // Work statistics of the forward paths: counters[0..3] += (paths, queries,
@@ -346,8 +361,37 @@ __device__ inline int job_of_tile(const JobDev* jobs, int njobs, uint64_t t) {
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWaves))) k_render_batch_fwd(const JobDev* __restrict__ jobs, int njobs, uint64_t ntiles,
-                                                             uint32_t tile, LaunchCfg L) {
+// Camera rays of the batch's jobs: a wave takes a tile at a time from the
+// launch's counter.
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWaves)))
+k_batch_primary(const JobDev* __restrict__ jobs, int njobs, uint64_t ntiles, uint32_t tile, LaunchCfg L) {
+  __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
+  TraceCtx tc = make_trace_ctx_wave(lds_stack, L);
+  const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
+  const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+  for (uint64_t t = wave; t < ntiles;) {
+    const int j = job_of_tile(jobs, njobs, t);
+    const SceneDev& S = jobs[j].S;
+    const CameraDev& C = jobs[j].C;
+    const PathParams P{jobs[j].seed, jobs[j].max_bounces, jobs[j].spp, 0u};
+    const PathRange R = jobs[j].range;
+    const uint64_t npaths = (uint64_t)P.spp * (uint64_t)C.width * (uint64_t)C.height;
+    const CkptDev ck = ckpt_view(jobs[j].ckpt, npaths, P.max_bounces);
+    const uint64_t i0 = (t - jobs[j].tile0) * tile, i1 = i0 + tile < R.slots ? i0 + tile : R.slots;
+    for (uint64_t i = i0; i < i1; i += 64)
+      trace_primary<true>(S, C, P, tc, PathGroup::at(C, R, i), ck, jobs[j].paths, 0);
+    if (L.tiles) {
+      uint32_t v = 0u;
+      if ((threadIdx.x & 63u) == 0u) v = atomicAdd(L.tiles, 1u);
+      t = nwaves + (uint64_t)(uint32_t)__shfl((int)v, 0);
+    } else {
+      t += nwaves;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBounceWaves)))
+k_batch_bounces(const JobDev* __restrict__ jobs, int njobs, uint64_t ntiles, uint32_t tile, LaunchCfg L) {
   __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
   TraceCtx tc = make_trace_ctx_wave(lds_stack, L);
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
@@ -359,15 +403,15 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFw
     const SceneDev& S = jobs[j].S;
     const CameraDev& C = jobs[j].C;
     const PathParams P{jobs[j].seed, jobs[j].max_bounces, jobs[j].spp, 0u};
-    const uint64_t first = jobs[j].first, count = jobs[j].count, t0 = jobs[j].tile0;
+    const PathRange& R = jobs[j].range;
+    const uint64_t t0 = jobs[j].tile0, slots = R.slots;
     const uint64_t npaths = (uint64_t)P.spp * (uint64_t)C.width * (uint64_t)C.height;
     const CkptDev ck = ckpt_view(jobs[j].ckpt, npaths, P.max_bounces);
     float* paths = jobs[j].paths;
     // the wave's tiles of this job, rendered without draining between them
-    const uint64_t tend = t0 + (count + tile - 1) / tile;
-    TileSupply sup = TileSupply::make(t, tend, nwaves, t0, first, first + count, tile);
-    sup.ctr = L.tiles;
-    render_paths_regen<true>(S, C, P, tc, sup, ck, [&](uint64_t p, F3 c) {
+    const TileDeal deal{slots, 0, (slots + tile - 1) / tile, 0u, tile};
+    TileSupply sup = TileSupply::make(t, nwaves, t0, deal, L.tiles ? L.tiles + 1 : nullptr);
+    render_bounces<true>(S, C, P, tc, sup, R, ck, paths, 0, [&](uint64_t p, F3 c) {
       paths[3 * p] = c.x;
       paths[3 * p + 1] = c.y;
       paths[3 * p + 2] = c.z;
@@ -502,9 +546,10 @@ hipError_t launch_render_batch(const JobDev* jobs_dev, const JobDev* jobs_host, 
   if (e != hipSuccess) return e;
   if (!adjoint) {
     if (ntiles == 0) return hipSuccess;
-    const LaunchCfg Lk = fit_grid(k_render_batch_fwd, L);
-    if (Lk.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Lk.tiles), 1, st)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_render_batch_fwd, dim3(Lk.grid), dim3(kBlock), 0, st, jobs_dev, njobs, ntiles, tile, Lk);
+    const LaunchCfg Lp = fit_grid(k_batch_primary, L), Lb = fit_grid(k_batch_bounces, L);
+    if (L.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2, st)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_batch_primary, dim3(Lp.grid), dim3(kBlock), 0, st, jobs_dev, njobs, ntiles, tile, Lp);
+    hipLaunchKernelGGL(k_batch_bounces, dim3(Lb.grid), dim3(kBlock), 0, st, jobs_dev, njobs, ntiles, tile, Lb);
     return hipGetLastError();
   }
   if (ntiles > 0) {
@@ -537,28 +582,43 @@ hipError_t launch_intersect(const SceneDev& S, const LaunchCfg& L, const float* 
   return hipGetLastError();
 }
 
-// About four tiles per wave of the grid, 64..4096 paths each.
-// Paths per tile: with the tile counter, small tiles taken as waves need
-// them (kDynTile); dealt statically, about four tiles per wave.
-constexpr uint32_t kDynTile = 64;
-static uint32_t forward_tile(uint64_t npaths, int grid, bool dynamic) {
-  if (dynamic) return kDynTile;
+// With the tile counter: big tiles, and small ones for the last slots (about
+// kDealTail per wave); dealt statically, about four tiles per wave, 64..4096
+// slots each.  512 x 512 step / 384 x 384 x 64 spp step with big tiles of 64:
+// 3.70 / 5.27 ms, 256 with a tail of 2: 3.48 / 5.22, of 4: 3.41 / 5.23, 512
+// with a tail of 2: 3.47 / 5.60.
+constexpr uint32_t kDealBig = 256, kDealTail = 4;
+static TileDeal deal_tiles(uint64_t slots, int grid, bool dynamic) {
   const uint64_t waves = (uint64_t)grid * (kBlock / 64);
-  const uint64_t t = npaths / (waves * 4) / 64 * 64;
-  return (uint32_t)(t < 64 ? 64 : (t > 4096 ? 4096 : t));
+  TileDeal d{slots, 0, 0, kDealBig, 64};
+  if (!dynamic) {
+    const uint64_t t = slots / (waves * 4) / 64 * 64;
+    d.tile = (uint32_t)(t < 64 ? 64 : (t > 4096 ? 4096 : t));
+    d.ntiles = (slots + d.tile - 1) / d.tile;
+    return d;
+  }
+  // big tiles only where each wave gets some of them
+  const uint64_t tail = waves * 64 * kDealTail;
+  while (d.big > 64 && slots < tail + waves * d.big * 2) d.big /= 2;
+  d.nbig = slots > tail ? (slots - tail) / d.big : 0;
+  d.ntiles = d.nbig + (slots - d.nbig * d.big + d.tile - 1) / d.tile;
+  return d;
 }
 
 template <bool kCkpt>
 static hipError_t launch_paths(const SceneDev& S, const CameraDev& C, const PathParams& P, const LaunchCfg& L,
                                uint64_t first, uint64_t count, float* paths, uint64_t paths_first, const CkptDev& ck,
                                hipStream_t st) {
-  const LaunchCfg Lk = fit_grid(k_render_paths<kCkpt>, L);
-  if (Lk.tiles) {
-    const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(Lk.tiles), 1, st);
+  const LaunchCfg Lp = fit_grid(k_primary<kCkpt>, L), Lb = fit_grid(k_bounces<kCkpt>, L);
+  if (L.tiles) {
+    const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2, st);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_render_paths<kCkpt>), dim3(Lk.grid), dim3(kBlock), 0, st, S, C, P, Lk, first,
-                     count, forward_tile(count, Lk.grid, Lk.tiles != nullptr), paths, paths_first, ck);
+  const PathRange R = path_range(C, first, count);
+  hipLaunchKernelGGL((k_primary<kCkpt>), dim3(Lp.grid), dim3(kBlock), 0, st, S, C, P, Lp, R,
+                     deal_tiles(R.slots, Lp.grid, L.tiles != nullptr), paths, paths_first, ck);
+  hipLaunchKernelGGL((k_bounces<kCkpt>), dim3(Lb.grid), dim3(kBlock), 0, st, S, C, P, Lb, R,
+                     deal_tiles(R.slots, Lb.grid, L.tiles != nullptr), paths, paths_first, ck);
   return hipGetLastError();
 }
 

@@ -120,6 +120,11 @@ constexpr int kBlock = 128;
 // going from 4 to 5 waves, 6.38 ms at 6; adjoint 2.15 -> 1.86 ms going from
 // 2 to 3.
 constexpr int kFwdWaves = 5;
+// The bounce pass holds a path and its shading: 4 waves (128 VGPRs) instead
+// of 5 (96, 176 B of scratch per lane): closed room 1.40 -> 1.25 ms, 512 x 512
+// step 3.44 -> 3.39 ms, eight views 1.79 -> 1.73 ms, 392k-triangle mesh 5.24 ->
+// 5.29 ms.
+constexpr int kBounceWaves = 4;
 constexpr int kAdjWaves = 3;
 // The boundary (edge) kernels: 5 waves; primary / pixel / indirect edge
 // terms at 512^2 x 4 spp on the metric scene: 2.35 / 2.53 / 3.09 ms at their
@@ -142,7 +147,7 @@ struct LaunchCfg {
   uint32_t* spill;      // spill buffer [depth][grid*kBlock]
   int cap;              // stack capacity
   int cus;              // compute units of the device
-  uint32_t* tiles;      // the forward's tile counter (one word, zeroed per launch); null: tiles dealt statically
+  uint32_t* tiles;      // tile counters (two words, zeroed per launch); null: tiles dealt statically
 };
 
 // A persistent grid-stride kernel should not launch more blocks than can be
@@ -216,6 +221,7 @@ struct JobDev {
   int32_t max_bounces, spp;
   int32_t solo;            // launched on its own (single-request kernels over its range), no tiles
   uint64_t first, count;   // path range of the job
+  PathRange range;         // its order of slots (forward)
   uint64_t tile0;          // first tile of the job in the batch
   float* paths;
   void* ckpt;
