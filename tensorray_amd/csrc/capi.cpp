@@ -1135,21 +1135,26 @@ trc_status trc_adam_uniform_step(trc_ctx* ctx, float* x, const float* grad, floa
 struct trc_lsolver {
   trc_ctx* ctx = nullptr;
   int n = 0;
-  int* row = nullptr;
+  float lambda = 0.0f;
+  int* len = nullptr;
+  int* off = nullptr;
   int* col = nullptr;
-  float* val = nullptr;
-  float* work = nullptr;      // r, p, ap: 3 x [n][3]
+  float* work = nullptr;      // r, p0, p1, ap: 4 x [n][3]
   CgScalars* scal = nullptr;
-  CsrDev dev() const { return CsrDev{n, row, col, val}; }
+  uint32_t* done = nullptr;   // pinned: the number of the last solve the device has finished iterating
+  uint32_t seq = 0;
+  LaplaceDev dev() const { return LaplaceDev{n, lambda, len, off, col}; }
 };
 
 namespace {
 void lsolver_free(trc_lsolver* s) {
-  for (void* p : {(void*)s->row, (void*)s->col, (void*)s->val, (void*)s->work, (void*)s->scal})
+  for (void* p : {(void*)s->len, (void*)s->off, (void*)s->col, (void*)s->work, (void*)s->scal})
     if (p) hipFree(p);
-  s->row = s->col = nullptr;
-  s->val = s->work = nullptr;
+  if (s->done) hipHostFree(s->done);
+  s->len = s->off = s->col = nullptr;
+  s->work = nullptr;
   s->scal = nullptr;
+  s->done = nullptr;
 }
 }  // namespace
 
@@ -1161,7 +1166,7 @@ trc_status trc_lsolver_create(trc_ctx* ctx, const uint32_t* faces, int32_t nf, i
     if (ctx->device < 0) throw Fail(TRC_ERR_STATE, "host-only context cannot run kernels");
     if (nv <= 0 || nf < 0 || (nf > 0 && !faces)) throw Fail(TRC_ERR_INVALID, "bad mesh");
     if (!(lambda >= 0.0f)) throw Fail(TRC_ERR_INVALID, "lambda must be >= 0");
-    // undirected edges of the triangles, then CSR rows with the diagonal
+    // undirected edges of the triangles, then rows with the diagonal, sliced
     std::vector<std::pair<int, int>> e;
     e.reserve(6 * (size_t)nf);
     for (int32_t f = 0; f < nf; ++f)
@@ -1174,44 +1179,48 @@ trc_status trc_lsolver_create(trc_ctx* ctx, const uint32_t* faces, int32_t nf, i
       }
     std::sort(e.begin(), e.end());
     e.erase(std::unique(e.begin(), e.end()), e.end());
-    std::vector<int> row((size_t)nv + 1, 0), col;
-    std::vector<float> val;
-    col.reserve(e.size() + (size_t)nv);
-    val.reserve(e.size() + (size_t)nv);
+    std::vector<int> len((size_t)nv, 1), off(((size_t)nv + 63) / 64), col;
+    for (const auto& p : e) ++len[(size_t)p.first];
+    size_t columns = 0;
+    for (size_t sl = 0; sl < off.size(); ++sl) {
+      int width = 0;
+      for (size_t i = 64 * sl; i < std::min<size_t>(64 * sl + 64, (size_t)nv); ++i) width = std::max(width, len[i]);
+      off[sl] = (int)columns;
+      columns += (size_t)width;
+    }
+    if (columns > (size_t)INT32_MAX) throw Fail(TRC_ERR_INVALID, "mesh too large");
+    col.assign(columns * 64, 0);
     size_t k = 0;
     for (int i = 0; i < nv; ++i) {
-      size_t k0 = k;
-      while (k < e.size() && e[k].first == i) ++k;
-      const int deg = (int)(k - k0);
+      int* c = &col[(size_t)off[(size_t)i / 64] * 64 + (size_t)i % 64];
       bool diag_done = false;
-      for (size_t q = k0; q < k; ++q) {
-        if (!diag_done && e[q].second > i) {
-          col.push_back(i);
-          val.push_back(1.0f + lambda * (float)deg);
+      for (; k < e.size() && e[k].first == i; ++k) {
+        if (!diag_done && e[k].second > i) {
+          *c = i;
+          c += 64;
           diag_done = true;
         }
-        col.push_back(e[q].second);
-        val.push_back(-lambda);
+        *c = e[k].second;
+        c += 64;
       }
-      if (!diag_done) {
-        col.push_back(i);
-        val.push_back(1.0f + lambda * (float)deg);
-      }
-      row[(size_t)i + 1] = (int)col.size();
+      if (!diag_done) *c = i;
     }
     std::unique_ptr<trc_lsolver> s(new trc_lsolver);
     s->ctx = ctx;
     s->n = nv;
+    s->lambda = lambda;
     try {
       hip_check(hipSetDevice(ctx->device), "hipSetDevice");
-      hip_check(hipMalloc((void**)&s->row, row.size() * sizeof(int)), "hipMalloc(csr)");
-      hip_check(hipMalloc((void**)&s->col, col.size() * sizeof(int)), "hipMalloc(csr)");
-      hip_check(hipMalloc((void**)&s->val, val.size() * sizeof(float)), "hipMalloc(csr)");
-      hip_check(hipMalloc((void**)&s->work, 9 * (size_t)nv * sizeof(float)), "hipMalloc(cg)");
+      hip_check(hipMalloc((void**)&s->len, len.size() * sizeof(int)), "hipMalloc(matrix)");
+      hip_check(hipMalloc((void**)&s->off, off.size() * sizeof(int)), "hipMalloc(matrix)");
+      hip_check(hipMalloc((void**)&s->col, col.size() * sizeof(int)), "hipMalloc(matrix)");
+      hip_check(hipMalloc((void**)&s->work, 12 * (size_t)nv * sizeof(float)), "hipMalloc(cg)");
       hip_check(hipMalloc((void**)&s->scal, sizeof(CgScalars)), "hipMalloc(cg)");
-      hip_check(hipMemcpy(s->row, row.data(), row.size() * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
+      hip_check(hipHostMalloc((void**)&s->done, sizeof(uint32_t), hipHostMallocDefault), "hipHostMalloc(cg)");
+      *s->done = 0u;
+      hip_check(hipMemcpy(s->len, len.data(), len.size() * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
+      hip_check(hipMemcpy(s->off, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
       hip_check(hipMemcpy(s->col, col.data(), col.size() * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
-      hip_check(hipMemcpy(s->val, val.data(), val.size() * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
     } catch (...) {
       lsolver_free(s.get());
       throw;
@@ -1224,7 +1233,7 @@ trc_status trc_lsolver_apply(trc_lsolver* s, const float* x, float* y, trc_strea
   if (!s) return TRC_ERR_INVALID;
   return guarded(s->ctx, [&] {
     if (!x || !y || x == y) throw Fail(TRC_ERR_INVALID, "bad vectors");
-    hip_check(launch_csr_spmv3(s->dev(), x, y, (hipStream_t)stream), "k_csr_spmv3");
+    hip_check(launch_laplace_apply(s->dev(), x, y, (hipStream_t)stream), "k_laplace_apply");
   });
 }
 
@@ -1234,10 +1243,17 @@ trc_status trc_lsolver_solve(trc_lsolver* s, const float* b, float* x, int32_t m
   return guarded(s->ctx, [&] {
     if (!b || !x || b == x) throw Fail(TRC_ERR_INVALID, "bad vectors");
     if (max_iter < 0 || !(tol > 0.0f && tol < 1.0f)) throw Fail(TRC_ERR_INVALID, "bad solver limits");
-    float* r = s->work;
-    float* p = r + 3 * (size_t)s->n;
-    float* ap = p + 3 * (size_t)s->n;
-    hip_check(launch_cg(s->dev(), b, x, r, p, ap, s->scal, max_iter, tol, (hipStream_t)stream), "k_cg");
+    const size_t nv3 = 3 * (size_t)s->n;
+    float *r = s->work, *p0 = r + nv3, *p1 = p0 + nv3, *ap = p1 + nv3;
+    // under capture every iteration is recorded: a replay may need them all
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const bool plain =
+        hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+    if (!plain) (void)hipGetLastError();
+    uint32_t* done = plain ? s->done : nullptr;
+    if (++s->seq == 0u) s->seq = 1u;
+    hip_check(launch_cg(s->dev(), b, x, r, p0, p1, ap, s->scal, max_iter, tol, done, s->seq, (hipStream_t)stream),
+              "k_cg");
   });
 }
 
@@ -1248,7 +1264,8 @@ trc_status trc_lsolver_status(trc_lsolver* s, int32_t* iters, float rel_residual
     hip_check(hipMemcpy(&h, s->scal, sizeof(h), hipMemcpyDeviceToHost), "hipMemcpy");
     if (iters) *iters = (int32_t)h.iters;
     if (rel_residual)
-      for (int c = 0; c < 3; ++c) rel_residual[c] = h.rr0[c] > 0.0f ? std::sqrt(h.rr[c] / h.rr0[c]) : 0.0f;  // |r| / |b|
+      for (int c = 0; c < 3; ++c)
+        rel_residual[c] = h.rr0[c] > 0.0f ? std::sqrt(h.rr[h.last & 1u][c] / h.rr0[c]) : 0.0f;  // |r| / |b|
   });
 }
 

@@ -100,17 +100,27 @@ hipError_t launch_adam_uniform(float* x, const float* g, float* m, float* v, uin
 
 // ---------------------------------------------------------------------------
 // Conjugate gradients for M x = b with M = I + lambda L symmetric positive
-// definite (CSR), three right-hand sides at once in the [V][3] layout of the
+// definite, three right-hand sides at once in the [V][3] layout of the
 // vertex buffers.  Scalars live on the device (CgScalars); every kernel
 // returns at once when all three columns have converged, so the host can
-// queue max_iter iterations without reading anything back.  A dot product
-// is a partial per block (no atomics: the partials are summed in block order
-// by every kernel that needs the total, so all of them see the same bits).
+// queue iterations without waiting for anything.  A dot product is a partial
+// per block (no atomics: the partials are summed in block order by every
+// kernel that needs the total, so all of them see the same bits).
+//
+// An iteration is two kernels.  k_cg_matvec forms the search direction p = r
+// + beta p_old of a row's neighbours where it gathers them (the direction of
+// one iteration is the other buffer of the last) and the new direction's
+// product; k_cg_update moves x and r.  With a kernel each for the product,
+// the update, the direction and the scalars, a mesh of 100,002 vertices (4-5 us
+// of work per iteration) was bound by queueing launches: 1,600 per call of 400
+// iterations, 8-12 ms for a LargeSteps step of two calls.  The word `done` in
+// host memory tells the host, which is still queueing, to stop; it never
+// waits for it.
 // ---------------------------------------------------------------------------
 constexpr int kCgThreads = 256;
 
 // The block's sum of (a, b, c) into part[blockIdx.x], in a fixed order.
-__device__ inline void block_partial3(float a, float b, float c, float (*part)[3]) {
+__device__ inline void block_partial3(float a, float b, float c, float4* part) {
   __shared__ float w[kCgThreads / 64][3];
   for (int o = 32; o > 0; o >>= 1) {
     a += __shfl_xor(a, o);
@@ -130,22 +140,28 @@ __device__ inline void block_partial3(float a, float b, float c, float (*part)[3
       s1 += w[k][1];
       s2 += w[k][2];
     }
-    part[blockIdx.x][0] = s0;
-    part[blockIdx.x][1] = s1;
-    part[blockIdx.x][2] = s2;
+    part[blockIdx.x] = make_float4(s0, s1, s2, 0.0f);
   }
 }
 
 // Sum of part[0 .. nb) per column, the same bits in every block: the first
-// wave sums a fixed subset per lane, then reduces across lanes.
-__device__ inline void sum_partials3(const float (*part)[3], int nb, float out[3]) {
+// wave sums a fixed subset per lane, then reduces across lanes.  The loads go
+// out together (their latency is most of a small solve's kernels).
+__device__ inline void sum_partials3(const float4* part, int nb, float out[3]) {
   __shared__ float tot[3];
   if (threadIdx.x < 64u) {
+    float4 v[kCgBlocks / 64];
+#pragma unroll
+    for (int j = 0; j < kCgBlocks / 64; ++j) {
+      const int k = (int)threadIdx.x + 64 * j;
+      v[j] = k < nb ? part[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
     float a = 0.0f, b = 0.0f, c = 0.0f;
-    for (int k = (int)threadIdx.x; k < nb; k += 64) {
-      a += part[k][0];
-      b += part[k][1];
-      c += part[k][2];
+#pragma unroll
+    for (int j = 0; j < kCgBlocks / 64; ++j) {
+      a += v[j].x;
+      b += v[j].y;
+      c += v[j].z;
     }
     for (int o = 32; o > 0; o >>= 1) {
       a += __shfl_xor(a, o);
@@ -164,130 +180,158 @@ __device__ inline void sum_partials3(const float (*part)[3], int nb, float out[3
   out[2] = tot[2];
 }
 
-__device__ inline bool cg_done(const CgScalars* s) { return s->active == 0u; }
+// y_i = sum over row i's columns j, in ascending order, of M_ij x_j; x(j)
+// gives a vector's row.
+template <class X>
+__device__ inline F3 row_product(const LaplaceDev& M, int i, X&& x) {
+  const int len = M.len[i];
+  const float diag = 1.0f + M.lambda * (float)(len - 1);
+  const int* col = M.col + (size_t)M.off[i >> 6] * 64u + (i & 63);
+  F3 a{0.0f, 0.0f, 0.0f};
+  for (int k = 0; k < len; ++k) {
+    const int j = col[(size_t)k * 64u];
+    a = a + (j == i ? diag : -M.lambda) * x(j);
+  }
+  return a;
+}
+__device__ inline F3 row3(const float* v, int i) { return F3{v[3 * (size_t)i], v[3 * (size_t)i + 1], v[3 * (size_t)i + 2]}; }
+__device__ inline void put_row3(float* v, int i, F3 a) {
+  v[3 * (size_t)i] = a.x;
+  v[3 * (size_t)i + 1] = a.y;
+  v[3 * (size_t)i + 2] = a.z;
+}
 
-// y = M x (and, with with_dot, the partials of x_c . y_c)
-__global__ void __launch_bounds__(kCgThreads) k_csr_spmv3(CsrDev M, const float* x, float* y, CgScalars* s,
-                                                          int use_flag, int with_dot) {
-  if (use_flag && cg_done(s)) return;
-  float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f;
+// y = M x
+__global__ void __launch_bounds__(kCgThreads) k_laplace_apply(LaplaceDev M, const float* x, float* y) {
+  const int stride = gridDim.x * blockDim.x;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < M.n; i += stride)
+    put_row3(y, i, row_product(M, i, [&](int j) { return row3(x, j); }));
+}
+
+// r = b - M x; partials of r.r and b.b
+__global__ void __launch_bounds__(kCgThreads) k_cg_init(LaplaceDev M, const float* b, const float* x, float* r,
+                                                        CgScalars* s) {
+  F3 d{0.0f, 0.0f, 0.0f}, e{0.0f, 0.0f, 0.0f};
   const int stride = gridDim.x * blockDim.x;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < M.n; i += stride) {
-    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-    for (int k = M.row[i]; k < M.row[i + 1]; ++k) {
-      const float w = M.val[k];
-      const float* xj = x + 3 * (size_t)M.col[k];
-      a0 = a0 + w * xj[0];
-      a1 = a1 + w * xj[1];
-      a2 = a2 + w * xj[2];
-    }
-    y[3 * (size_t)i] = a0;
-    y[3 * (size_t)i + 1] = a1;
-    y[3 * (size_t)i + 2] = a2;
-    if (with_dot) {
-      d0 = d0 + x[3 * (size_t)i] * a0;
-      d1 = d1 + x[3 * (size_t)i + 1] * a1;
-      d2 = d2 + x[3 * (size_t)i + 2] * a2;
-    }
+    const F3 bi = row3(b, i);
+    const F3 ri = bi - row_product(M, i, [&](int j) { return row3(x, j); });
+    put_row3(r, i, ri);
+    d = d + ri * ri;
+    e = e + bi * bi;
   }
-  if (with_dot) block_partial3(d0, d1, d2, s->part_pap);
-}
-
-// r = b - Mx (Mx in r on entry), p = r; partials of r.r and b.b
-__global__ void __launch_bounds__(kCgThreads) k_cg_init(const float* b, float* r, float* p, int n, CgScalars* s) {
-  float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f, e0 = 0.0f, e1 = 0.0f, e2 = 0.0f;
-  const int stride = gridDim.x * blockDim.x;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    for (int c = 0; c < 3; ++c) {
-      const size_t j = 3 * (size_t)i + c;
-      const float ri = b[j] - r[j];
-      r[j] = ri;
-      p[j] = ri;
-    }
-    d0 = d0 + r[3 * (size_t)i] * r[3 * (size_t)i];
-    d1 = d1 + r[3 * (size_t)i + 1] * r[3 * (size_t)i + 1];
-    d2 = d2 + r[3 * (size_t)i + 2] * r[3 * (size_t)i + 2];
-    e0 = e0 + b[3 * (size_t)i] * b[3 * (size_t)i];
-    e1 = e1 + b[3 * (size_t)i + 1] * b[3 * (size_t)i + 1];
-    e2 = e2 + b[3 * (size_t)i + 2] * b[3 * (size_t)i + 2];
-  }
-  block_partial3(d0, d1, d2, s->part_rr);
+  block_partial3(d.x, d.y, d.z, s->part_rr);
   __syncthreads();  // block_partial3's LDS is reused
-  block_partial3(e0, e1, e2, s->part_b);
+  block_partial3(e.x, e.y, e.z, s->part_b);
 }
 
-// x += alpha p, r -= alpha Ap; partials of the new r.r   (alpha = rr / pAp)
-__global__ void __launch_bounds__(kCgThreads) k_cg_update(float* x, float* r, const float* p, const float* ap, int n,
-                                                          CgScalars* s) {
-  if (cg_done(s)) return;
-  float pap[3];
-  sum_partials3(s->part_pap, (int)gridDim.x, pap);
-  float alpha[3];
-  for (int c = 0; c < 3; ++c) alpha[c] = ((s->active >> c) & 1u) && pap[c] > 0.0f ? s->rr[c] / pap[c] : 0.0f;
-  float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f;
-  const int stride = gridDim.x * blockDim.x;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    for (int c = 0; c < 3; ++c) {
-      const size_t j = 3 * (size_t)i + c;
-      x[j] = x[j] + alpha[c] * p[j];
-      r[j] = r[j] - alpha[c] * ap[j];
-    }
-    d0 = d0 + r[3 * (size_t)i] * r[3 * (size_t)i];
-    d1 = d1 + r[3 * (size_t)i + 1] * r[3 * (size_t)i + 1];
-    d2 = d2 + r[3 * (size_t)i + 2] * r[3 * (size_t)i + 2];
-  }
-  block_partial3(d0, d1, d2, s->part_rr);
-}
-
-// p = r + beta p  (beta = rr_new / rr per column)
-__global__ void __launch_bounds__(kCgThreads) k_cg_direction(const float* r, float* p, int n, CgScalars* s) {
-  if (cg_done(s)) return;
-  float rr_new[3];
-  sum_partials3(s->part_rr, (int)gridDim.x, rr_new);
-  float beta[3];
-  for (int c = 0; c < 3; ++c) beta[c] = s->rr[c] > 0.0f ? rr_new[c] / s->rr[c] : 0.0f;
-  const int stride = gridDim.x * blockDim.x;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    for (int c = 0; c < 3; ++c) {
-      const size_t j = 3 * (size_t)i + c;
-      p[j] = r[j] + beta[c] * p[j];
-    }
-}
-
-// One block: rr = the summed r.r partials (rr0 = b.b at the start), retire
-// converged columns.
-__global__ void __launch_bounds__(kCgThreads) k_cg_scalars(CgScalars* s, float tol2, int first, int nb) {
-  if (!first && cg_done(s)) return;
-  float rr[3];
+// Scalars of iteration `it` from the partials the last kernels left: rr = r.r
+// and the columns still active.  Every block computes them; block 0 stores
+// them at parity (it + 1) & 1 (others still read parity it & 1).
+__device__ inline uint32_t cg_scalars(CgScalars* s, int it, float tol2, float rr[3], float beta[3], uint32_t* done,
+                                      uint32_t seq) {
+  const int nb = (int)gridDim.x;
   sum_partials3(s->part_rr, nb, rr);
-  if (first) {
+  uint32_t active = 0u;
+  if (it == 0) {
     float b2[3];
     __syncthreads();  // sum_partials3's LDS is reused
     sum_partials3(s->part_b, nb, b2);
-    if (threadIdx.x != 0u) return;
-    s->active = 0u;
     for (int c = 0; c < 3; ++c) {
-      s->rr[c] = rr[c];
-      s->rr0[c] = b2[c];
-      s->pap[c] = s->rr_new[c] = 0.0f;
-      if (rr[c] > tol2 * b2[c] && rr[c] > 0.0f) s->active |= 1u << c;
+      beta[c] = 0.0f;
+      if (rr[c] > tol2 * b2[c] && rr[c] > 0.0f) active |= 1u << c;
     }
-    s->iters = 0u;
-    return;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+      for (int c = 0; c < 3; ++c) s->rr0[c] = b2[c];
+  } else {
+    active = s->active[it & 1];
+    for (int c = 0; c < 3; ++c) {
+      const float old = s->rr[it & 1][c];
+      beta[c] = old > 0.0f ? rr[c] / old : 0.0f;
+      if (!(rr[c] > tol2 * s->rr0[c])) active &= ~(1u << c);
+    }
   }
-  if (threadIdx.x != 0u) return;
-  s->iters += 1u;
-  for (int c = 0; c < 3; ++c) {
-    s->rr[c] = rr[c];
-    s->rr_new[c] = rr[c];
-    if (!(rr[c] > tol2 * s->rr0[c])) s->active &= ~(1u << c);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int c = 0; c < 3; ++c) s->rr[(it + 1) & 1][c] = rr[c];
+    s->active[(it + 1) & 1] = active;
+    s->iters = (uint32_t)it;
+    s->last = (uint32_t)((it + 1) & 1);
+    if (active == 0u && done) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
+  return active;
+}
+// A converged solve: the state is handed on to the other parity unchanged.
+__device__ inline bool cg_done(CgScalars* s, int it) {
+  if (it == 0 || s->active[it & 1] != 0u) return false;
+  if (blockIdx.x == 0 && threadIdx.x == 0) s->active[(it + 1) & 1] = 0u;
+  return true;
 }
 
-__global__ void k_cg_reset(CgScalars* s) {
-  for (int c = 0; c < 3; ++c) s->rr[c] = s->rr_new[c] = s->pap[c] = s->rr0[c] = 0.0f;
-  s->active = 7u;
-  s->iters = 0u;
+// p = r + beta p_old (it = 0: r), ap = M p; partials of p.ap.  r.r of the last
+// update decides whether any column still iterates.
+__global__ void __launch_bounds__(kCgThreads) k_cg_matvec(LaplaceDev M, const float* r, const float* p_old, float* p,
+                                                          float* ap, CgScalars* s, int it, float tol2, uint32_t* done,
+                                                          uint32_t seq) {
+  if (cg_done(s, it)) return;
+  float rr[3], beta[3];
+  if (cg_scalars(s, it, tol2, rr, beta, done, seq) == 0u) return;
+  F3 dot3{0.0f, 0.0f, 0.0f};
+  const F3 bt{beta[0], beta[1], beta[2]};
+  const int stride = gridDim.x * blockDim.x;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < M.n; i += stride) {
+    F3 pi, y;
+    if (it == 0) {
+      pi = row3(r, i);
+      y = row_product(M, i, [&](int j) { return row3(r, j); });
+    } else {
+      pi = row3(r, i) + bt * row3(p_old, i);
+      y = row_product(M, i, [&](int j) { return row3(r, j) + bt * row3(p_old, j); });
+    }
+    put_row3(p, i, pi);
+    put_row3(ap, i, y);
+    dot3 = dot3 + pi * y;
+  }
+  block_partial3(dot3.x, dot3.y, dot3.z, s->part_pap);
+}
+
+// x += alpha p, r -= alpha Ap (alpha = rr / pAp); partials of the new r.r
+__global__ void __launch_bounds__(kCgThreads) k_cg_update(float* x, float* r, const float* p, const float* ap, int n,
+                                                          CgScalars* s, int it) {
+  const uint32_t active = s->active[(it + 1) & 1];
+  if (active == 0u) return;
+  float pap[3];
+  sum_partials3(s->part_pap, (int)gridDim.x, pap);
+  float al[3];
+  for (int c = 0; c < 3; ++c)
+    al[c] = ((active >> c) & 1u) && pap[c] > 0.0f ? s->rr[(it + 1) & 1][c] / pap[c] : 0.0f;
+  const F3 alpha{al[0], al[1], al[2]};
+  F3 d{0.0f, 0.0f, 0.0f};
+  const int stride = gridDim.x * blockDim.x;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    put_row3(x, i, row3(x, i) + alpha * row3(p, i));
+    const F3 ri = row3(r, i) - alpha * row3(ap, i);
+    put_row3(r, i, ri);
+    d = d + ri * ri;
+  }
+  block_partial3(d.x, d.y, d.z, s->part_rr);
+}
+
+// The scalars after the last update (one block standing for the grid of nb).
+__global__ void __launch_bounds__(kCgThreads) k_cg_finish(CgScalars* s, int it, float tol2, int nb) {
+  if (it > 0 && s->active[it & 1] == 0u) return;  // the last k_cg_matvec stored them
+  float rr[3], b2[3];
+  sum_partials3(s->part_rr, nb, rr);
+  if (it == 0) {
+    __syncthreads();  // sum_partials3's LDS is reused
+    sum_partials3(s->part_b, nb, b2);
+  }
+  if (threadIdx.x != 0u) return;
+  for (int c = 0; c < 3; ++c) {
+    s->rr[0][c] = rr[c];
+    if (it == 0) s->rr0[c] = b2[c];
+  }
+  s->iters = (uint32_t)it;
+  s->last = 0u;
 }
 
 static int cg_grid(int n) {
@@ -295,27 +339,27 @@ static int cg_grid(int n) {
   return g < 1 ? 1 : (g > kCgBlocks ? kCgBlocks : g);
 }
 
-hipError_t launch_csr_spmv3(const CsrDev& M, const float* x, float* y, hipStream_t st) {
-  hipLaunchKernelGGL(k_csr_spmv3, dim3(cg_grid(M.n)), dim3(kCgThreads), 0, st, M, x, y, (CgScalars*)nullptr, 0, 0);
+hipError_t launch_laplace_apply(const LaplaceDev& M, const float* x, float* y, hipStream_t st) {
+  hipLaunchKernelGGL(k_laplace_apply, dim3(cg_grid(M.n)), dim3(kCgThreads), 0, st, M, x, y);
   return hipGetLastError();
 }
 
-hipError_t launch_cg(const CsrDev& M, const float* b, float* x, float* r, float* p, float* ap, CgScalars* s,
-                     int max_iter, float tol, hipStream_t st) {
+hipError_t launch_cg(const LaplaceDev& M, const float* b, float* x, float* r, float* p0, float* p1, float* ap,
+                     CgScalars* s, int max_iter, float tol, uint32_t* done, uint32_t seq, hipStream_t st) {
   const int n = M.n;
   const int nb = cg_grid(n);
   const dim3 g(nb), blk(kCgThreads);
   const float tol2 = tol * tol;
-  hipLaunchKernelGGL(k_cg_reset, dim3(1), dim3(1), 0, st, s);
-  hipLaunchKernelGGL(k_csr_spmv3, g, blk, 0, st, M, x, r, s, 0, 0);  // r = M x
-  hipLaunchKernelGGL(k_cg_init, g, blk, 0, st, b, r, p, n, s);
-  hipLaunchKernelGGL(k_cg_scalars, dim3(1), blk, 0, st, s, tol2, 1, nb);
-  for (int it = 0; it < max_iter; ++it) {
-    hipLaunchKernelGGL(k_csr_spmv3, g, blk, 0, st, M, p, ap, s, 1, 1);
-    hipLaunchKernelGGL(k_cg_update, g, blk, 0, st, x, r, p, ap, n, s);
-    hipLaunchKernelGGL(k_cg_direction, g, blk, 0, st, r, p, n, s);
-    hipLaunchKernelGGL(k_cg_scalars, dim3(1), blk, 0, st, s, tol2, 0, nb);
+  float* p[2] = {p0, p1};
+  hipLaunchKernelGGL(k_cg_init, g, blk, 0, st, M, b, (const float*)x, r, s);
+  int it = 0;
+  for (; it < max_iter; ++it) {
+    if (done && __atomic_load_n(done, __ATOMIC_RELAXED) == seq) break;
+    hipLaunchKernelGGL(k_cg_matvec, g, blk, 0, st, M, (const float*)r, (const float*)p[(it + 1) & 1], p[it & 1], ap, s,
+                       it, tol2, done, seq);
+    hipLaunchKernelGGL(k_cg_update, g, blk, 0, st, x, r, (const float*)p[it & 1], (const float*)ap, n, s, it);
   }
+  hipLaunchKernelGGL(k_cg_finish, dim3(1), blk, 0, st, s, it, tol2, nb);
   return hipGetLastError();
 }
 

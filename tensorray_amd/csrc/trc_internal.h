@@ -186,31 +186,36 @@ hipError_t launch_adam(float* x, const float* g, float* m, float* v, uint64_t n,
 // vmax_bits: one device word of scratch
 hipError_t launch_adam_uniform(float* x, const float* g, float* m, float* v, uint64_t n, float lr, float b1, float b2,
                                float bc1, float bc2, unsigned int* vmax_bits, hipStream_t st);
-// Sparse symmetric matrix (CSR) and the device scalars of a 3-column
-// conjugate-gradient solve.
-struct CsrDev {
+// I + lambda L of a mesh: the columns of each row (its neighbours and itself,
+// ascending) in slices of 64 rows, column k of a slice's rows side by side, so
+// that a wave reads them with one coalesced load.  The values follow from the
+// pattern: 1 + lambda (len - 1) on the diagonal, -lambda elsewhere.
+struct LaplaceDev {
   int n;
-  const int* row;    // [n + 1]
-  const int* col;    // [nnz]
-  const float* val;  // [nnz]
+  float lambda;
+  const int* len;  // [n] entries of each row
+  const int* off;  // [ceil(n / 64)] first 64-wide column of each slice
+  const int* col;  // [columns][64]
 };
 // Blocks of the conjugate-gradient kernels (grid-stride over the rows); each
 // writes its share of a dot product to a partial, and the partials are
 // summed in block order, so the solve is deterministic.
 constexpr int kCgBlocks = 1024;
-struct CgScalars {
-  float rr[3], rr_new[3], pap[3], rr0[3];  // rr0: |b|^2 per column
-  unsigned int active;  // bit c: column c not converged
-  unsigned int iters;
-  float part_pap[kCgBlocks][3];  // p . Ap
-  float part_rr[kCgBlocks][3];   // r . r
-  float part_b[kCgBlocks][3];    // b . b
+struct alignas(16) CgScalars {
+  float rr[2][3], rr0[3];   // r.r (by parity of the iteration) and |b|^2 per column
+  unsigned int active[2];   // bit c: column c not converged
+  unsigned int iters, last; // updates made; which rr is the last
+  float4 part_pap[kCgBlocks];  // p . Ap
+  float4 part_rr[kCgBlocks];   // r . r
+  float4 part_b[kCgBlocks];    // b . b
 };
-hipError_t launch_csr_spmv3(const CsrDev& M, const float* x, float* y, hipStream_t st);
+hipError_t launch_laplace_apply(const LaplaceDev& M, const float* x, float* y, hipStream_t st);
 // M x = b for the three columns of [n][3] b, x (x: initial guess on entry);
-// r, p, ap: [n][3] work vectors; stops a column once |r| <= tol |b|.
-hipError_t launch_cg(const CsrDev& M, const float* b, float* x, float* r, float* p, float* ap, CgScalars* s,
-                     int max_iter, float tol, hipStream_t st);
+// r, p0, p1, ap: [n][3] work vectors; stops a column once |r| <= tol |b|.
+// done (or null): host memory the device sets to seq once every column has
+// stopped; the call queues no further iterations when it sees that.
+hipError_t launch_cg(const LaplaceDev& M, const float* b, float* x, float* r, float* p0, float* p1, float* ap,
+                     CgScalars* s, int max_iter, float tol, uint32_t* done, uint32_t seq, hipStream_t st);
 hipError_t launch_grad_reduce(const GradCopies& g, float* dpos, hipStream_t st);
 
 // One job of a batched launch (device copy of trc_job).
