@@ -75,12 +75,21 @@ constexpr int kQCountShift = 27;
 constexpr uint32_t kQIndexMask = (1u << kQCountShift) - 1u;
 // Relative widening of the plane offsets: covers the rounding of the
 // traversal's t = h i + b in its h i part (3 x 2^-24 of it).
-constexpr double kQWiden = 1.0 / 1048576.0;
+constexpr float kQWiden = 1.0f / 1048576.0f;
 
-// Bits of the half-precision number at or below (up = false) or at or above
-// (up = true) x >= 0; beyond the largest one 65504 or infinity, 0 or infinity
-// for NaN.
-TR_HD uint32_t half_bits(double x, bool up) {
+// Bits of a half-precision number at or below (up = false) or at or above
+// (up = true) x >= 0; beyond the largest one 65504 or infinity.  The device
+// converts with v_cvt_pkrtz_f16_f32 (towards zero).
+#if defined(__HIP_DEVICE_COMPILE__)
+TR_HD uint32_t half_bits(float x, bool up) {
+  x = x > 0.0f ? x : 0.0f;
+  uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, 0.0f)) & 0xFFFFu;
+  if (up && (float)__builtin_bit_cast(_Float16, (uint16_t)h) < x) ++h;
+  return h;
+}
+#else
+TR_HD uint32_t half_bits(float xf, bool up) {
+  const double x = (double)xf;
   if (!(x < 65504.0)) return up ? 0x7C00u : (x >= 65504.0 ? 0x7BFFu : 0u);
   if (!(x > 0.0)) return 0u;
   int e = 0;
@@ -90,6 +99,7 @@ TR_HD uint32_t half_bits(double x, bool up) {
   const uint32_t k = (uint32_t)(up ? ceil(m) : floor(m));
   return ((uint32_t)(e + 13) << 10) + k;  // a normal number's leading 1024 carries into the exponent
 }
+#endif
 
 // The scale of a tree of extent `ext`: offsets up to 2^14 steps, which leaves
 // room for a refit to grow the boxes fourfold (beyond that the upper planes
@@ -102,40 +112,51 @@ TR_HD float quant_scale(float ext) {
 }
 
 // The QNode of `n`, whose slots are laid out as described at Bvh4Node.  The
-// differences to the origin are taken in double (exact, or within 2^-53 of
-// coordinates whose boxes were padded by 2^-20), so the planes never lie
-// inside the padded boxes.
+// scaling is exact; the difference to the origin and the widening round by
+// 2^-24 each, well inside the widening, so the planes never lie inside the
+// padded boxes.
 TR_HD QNode quantize_node(const Bvh4Node& n, float inv_scale) {
   QNode q;
-  uint32_t ni = 0u, nl = 0u;
-  const float* lo[3] = {n.lox, n.loy, n.loz};
-  const float* hi[3] = {n.hix, n.hiy, n.hiz};
+  uint32_t ni = 0u, nl = 0u, leaf = 0u;
+#pragma unroll
   for (int s = 0; s < 4; ++s) {
     if (n.child[s] == kEmpty) continue;
-    if (n.child[s] & kLeafBit) ++nl;
-    else ++ni;
+    if (n.child[s] & kLeafBit) {
+      if (nl == 0u) leaf = leaf_first(n.child[s]);
+      ++nl;
+    } else {
+      ++ni;
+    }
   }
+  const uint32_t nc = ni + nl;
+  const float* lo[3] = {n.lox, n.loy, n.loz};
+  const float* hi[3] = {n.hix, n.hiy, n.hiz};
   uint32_t org[3];
+#pragma unroll
   for (int k = 0; k < 3; ++k) {
     float o = lo[k][0];
-    for (uint32_t s = 1; s < ni + nl; ++s) o = lo[k][s] < o ? lo[k][s] : o;
+#pragma unroll
+    for (uint32_t s = 1; s < 4; ++s) o = s < nc && lo[k][s] < o ? lo[k][s] : o;
     union { float f; uint32_t u; } c;
     c.f = o * inv_scale;
     if (c.u & 0x80000000u) c.u += 0x7FFu;  // towards minus infinity
     c.u &= ~0x7FFu;
     org[k] = c.u >> 11;
-    for (uint32_t j = 0; j < 4; ++j) q.w[4 + 4 * k + j] = 0u;
-    for (uint32_t s = 0; s < ni + nl; ++s) {
-      const double a = (double)lo[k][s] * (double)inv_scale - (double)c.f;
-      const double b = (double)hi[k][s] * (double)inv_scale - (double)c.f;
-      q.w[4 + 4 * k + (s >> 1)] |= half_bits(a * (1.0 - kQWiden), false) << (16u * (s & 1u));
-      q.w[6 + 4 * k + (s >> 1)] |= half_bits(b * (1.0 + kQWiden), true) << (16u * (s & 1u));
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (uint32_t s = 0; s < 4; ++s) {
+      if (s >= nc) continue;
+      const float a = lo[k][s] * inv_scale - c.f, b = hi[k][s] * inv_scale - c.f;
+      w[s >> 1] |= half_bits(a * (1.0f - kQWiden), false) << (16u * (s & 1u));
+      w[2 + (s >> 1)] |= half_bits(b * (1.0f + kQWiden), true) << (16u * (s & 1u));
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q.w[4 + 4 * k + j] = w[j];
   }
   q.w[0] = org[0] << 11 | org[1] >> 10;
   q.w[1] = org[1] << 22 | org[2] << 1;
   q.w[2] = (ni ? n.child[0] : 0u) | ni << kQCountShift;
-  q.w[3] = (nl ? leaf_first(n.child[ni]) : 0u) | nl << kQCountShift;
+  q.w[3] = leaf | nl << kQCountShift;
   return q;
 }
 

@@ -575,16 +575,48 @@ __global__ void k_guide_poly(GuideDev G) {
   }
 }
 
-// part[c] = sequential sum of chunk c of v[0, n).
-__global__ void k_chunk_sums(const float* v, int n, float* part) {
-  const int nc = (n + kSumChunk - 1) / kSumChunk;
-  const int stride = gridDim.x * blockDim.x;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += stride) {
-    const int lo = c * kSumChunk, hi = min(n, lo + kSumChunk);
-    float acc = 0.0f;
-    for (int i = lo; i < hi; ++i) acc = acc + v[i];
-    part[c] = acc;
+// One wave per chunk of kSumChunk values: the lanes stage the chunk in LDS and
+// one lane runs the dependent additions from there (reading the chunk from
+// memory, one lane each, k_chunk_sums took 70 us and k_chunk_prefix 129 us for
+// 12,000 leaves).  Returns (lane 0) the sequential sum;
+// with `prefix` the inclusive prefix of every value is left in v.
+__device__ inline float chunk_sum(float* v, const float* src, int m, bool prefix) {
+  for (int i = (int)threadIdx.x; i < kSumChunk; i += 64) v[i] = i < m ? src[i] : 0.0f;
+  __syncthreads();
+  float acc = 0.0f;
+  if (threadIdx.x == 0u) {
+    int i = 0;
+    for (; i + 16 <= m; i += 16) {
+      float4 q[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) q[k] = reinterpret_cast<const float4*>(v + i)[k];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        q[k].x = acc = acc + q[k].x;
+        q[k].y = acc = acc + q[k].y;
+        q[k].z = acc = acc + q[k].z;
+        q[k].w = acc = acc + q[k].w;
+      }
+      if (prefix) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) reinterpret_cast<float4*>(v + i)[k] = q[k];
+      }
+    }
+    for (; i < m; ++i) {
+      acc = acc + v[i];
+      if (prefix) v[i] = acc;
+    }
   }
+  __syncthreads();
+  return acc;
+}
+
+// part[c] = sequential sum of chunk c of v[0, n).
+__global__ void __launch_bounds__(64) k_chunk_sums(const float* v, int n, float* part) {
+  __shared__ __align__(16) float s[kSumChunk];
+  const int lo = (int)blockIdx.x * kSumChunk;
+  const float acc = chunk_sum(s, v + lo, min(n - lo, kSumChunk), false);
+  if (threadIdx.x == 0u) part[blockIdx.x] = acc;
 }
 
 // One thread: part[c] becomes the exclusive prefix of the chunk sums,
@@ -614,18 +646,12 @@ __global__ void k_guide_weights(const float* sec_cdf, GuideDev G, const float* t
 }
 
 // cdf_i = (blocked inclusive prefix of f) / n, from the chunk offsets.
-__global__ void k_chunk_prefix(float* v, int n, const float* part, float inv) {
-  const int nc = (n + kSumChunk - 1) / kSumChunk;
-  const int stride = gridDim.x * blockDim.x;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += stride) {
-    const int lo = c * kSumChunk, hi = min(n, lo + kSumChunk);
-    float local = 0.0f;
-    const float off = part[c];
-    for (int i = lo; i < hi; ++i) {
-      local = local + v[i];
-      v[i] = (off + local) * inv;
-    }
-  }
+__global__ void __launch_bounds__(64) k_chunk_prefix(float* v, int n, const float* part, float inv) {
+  __shared__ __align__(16) float s[kSumChunk];
+  const int lo = (int)blockIdx.x * kSumChunk, m = min(n - lo, kSumChunk);
+  const float off = part[blockIdx.x];
+  chunk_sum(s, v + lo, m, true);
+  for (int i = (int)threadIdx.x; i < m; i += 64) v[lo + i] = (off + s[i]) * inv;
 }
 
 // fsum = total of f; cdf_i /= cdf_{n-1} (the integral) when it is positive.
@@ -930,15 +956,14 @@ hipError_t launch_guide_build(const SceneDev& S, const LaunchCfg& L, uint32_t se
   if (e != hipSuccess) return e;
   const int n = g.n, nc = (n + kSumChunk - 1) / kSumChunk;
   const int gl = (n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096;  // grid over leaves
-  const int gc = (nc + 63) / 64;                                     // grid over chunks
   float* total = g.part + nc;
   hipLaunchKernelGGL(k_guide_poly, dim3(gl), dim3(256), 0, st, g);
-  hipLaunchKernelGGL(k_chunk_sums, dim3(gc), dim3(64), 0, st, g.poly, n, g.part);
+  hipLaunchKernelGGL(k_chunk_sums, dim3(nc), dim3(64), 0, st, g.poly, n, g.part);
   hipLaunchKernelGGL(k_chunk_scan, dim3(1), dim3(64), 0, st, g.part, nc);
   hipLaunchKernelGGL(k_guide_weights, dim3(gl), dim3(256), 0, st, S.sec.cdf, g, total);
-  hipLaunchKernelGGL(k_chunk_sums, dim3(gc), dim3(64), 0, st, g.cdf, n, g.part);
+  hipLaunchKernelGGL(k_chunk_sums, dim3(nc), dim3(64), 0, st, g.cdf, n, g.part);
   hipLaunchKernelGGL(k_chunk_scan, dim3(1), dim3(64), 0, st, g.part, nc);
-  hipLaunchKernelGGL(k_chunk_prefix, dim3(gc), dim3(64), 0, st, g.cdf, n, g.part, 1.0f / (float)n);
+  hipLaunchKernelGGL(k_chunk_prefix, dim3(nc), dim3(64), 0, st, g.cdf, n, g.part, 1.0f / (float)n);
   hipLaunchKernelGGL(k_guide_normalize, dim3(gl), dim3(256), 0, st, g, total);
   hipLaunchKernelGGL(k_guide_normalize_last, dim3(1), dim3(64), 0, st, g);
   return hipGetLastError();
