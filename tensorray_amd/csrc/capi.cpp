@@ -195,6 +195,15 @@ void upload_scene(trc_scene* s, hipStream_t st) {
   d.uv_idx = upload(s, h.uv_idx, st);
   d.shade = upload(s, h.shade, st);
   d.tris = upload(s, h.tris, st);
+  std::vector<TriVerts> verts((size_t)h.num_triangles());
+  for (size_t t = 0; t < verts.size(); ++t) {
+    float* v[3] = {verts[t].v0, verts[t].v1, verts[t].v2};
+    for (int j = 0; j < 3; ++j) {
+      std::memcpy(v[j], &h.pos[3 * (size_t)h.idx[3 * t + j]], 12);
+      std::memcpy(v[j] + 3, &h.idx[3 * t + j], 4);
+    }
+  }
+  d.verts = upload(s, verts, st);
   d.nodes = upload(s, h.nodes, st);
   float ext = 0.0f;
   {

@@ -30,18 +30,31 @@ TR_HD F3 to_world(const Its& s, F3 l) { return l.x * s.t + l.y * s.b + l.z * s.n
 
 TR_HD F3 load3(const float* p, uint32_t i) { return F3{p[3 * i], p[3 * i + 1], p[3 * i + 2]}; }
 
+struct TriCorners {
+  F3 p0, p1, p2;
+  uint32_t i0, i1, i2;
+};
+TR_HD TriCorners tri_corners(const SceneDev& S, int32_t tri) {
+  const float4* q = reinterpret_cast<const float4*>(S.verts + tri);
+  const float4 a = q[0], b = q[1], c = q[2];
+  union { float f; uint32_t u; } i0, i1, i2;
+  i0.f = a.w;
+  i1.f = b.w;
+  i2.f = c.w;
+  return TriCorners{F3{a.x, a.y, a.z}, F3{b.x, b.y, b.z}, F3{c.x, c.y, c.z}, i0.u, i1.u, i2.u};
+}
+
 // Scene::PostIntersect (Scene.cpp:668-730) for triangle `tri` and
 // barycentrics (u, v).
 TR_HD Its post_intersect(const SceneDev& S, int32_t tri, float u, float v) {
   Its s;
-  uint32_t i0 = S.idx[3 * tri], i1 = S.idx[3 * tri + 1], i2 = S.idx[3 * tri + 2];
-  F3 p0 = load3(S.pos, i0), p1 = load3(S.pos, i1), p2 = load3(S.pos, i2);
+  const TriCorners q = tri_corners(S, tri);
   float w = 1.0f - u - v;
-  s.p = w * p0 + u * p1 + v * p2;
+  s.p = w * q.p0 + u * q.p1 + v * q.p2;
   const TriShade& sh = S.shade[tri];
   s.ng = F3{sh.n[0], sh.n[1], sh.n[2]};
   if (sh.flags & kTriSmooth) {
-    F3 n0 = load3(S.vnrm, i0), n1 = load3(S.vnrm, i1), n2 = load3(S.vnrm, i2);
+    F3 n0 = load3(S.vnrm, q.i0), n1 = load3(S.vnrm, q.i1), n2 = load3(S.vnrm, q.i2);
     s.ns = w * n0 + u * n1 + v * n2;
   } else {
     s.ns = s.ng;
@@ -386,8 +399,8 @@ TR_HD LightSample light_sample(const SceneDev& S, float u0, float u1) {
   float bv = t * u1;
   float bw = 1.0f - bu - bv;
   int32_t tri = S.light_tri[i];
-  F3 q0 = load3(S.pos, S.idx[3 * tri]), q1 = load3(S.pos, S.idx[3 * tri + 1]), q2 = load3(S.pos, S.idx[3 * tri + 2]);
-  ls.p = bw * q0 + bu * q1 + bv * q2;
+  const TriCorners q = tri_corners(S, tri);
+  ls.p = bw * q.p0 + bu * q.p1 + bv * q.p2;
   const TriShade& sh = S.shade[tri];
   ls.n = F3{sh.n[0], sh.n[1], sh.n[2]};
   ls.pdf = S.light_pdf[i];

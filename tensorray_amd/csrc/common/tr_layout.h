@@ -8,6 +8,7 @@
 //   vnrm     float[V][3]      vertex normals (smooth-shaded meshes only)
 //   shade    TriShade[T]      per-triangle face normal, area, material, emitter
 //   tris     TriRecord[T]     triangle vertices in BVH leaf order (48 B)
+//   verts    TriVerts[T]      vertices and their indices by triangle id (48 B)
 //   nodes    Bvh4Node[N]      4-wide BVH with float child boxes (refit, SAH cost)
 //   qnodes   QNode[N]         the same tree as the traversal reads it, 64 B per node
 //   mats     Material[M]
@@ -177,6 +178,16 @@ struct alignas(16) TriRecord {
   float v2[4];
 };
 
+// A triangle's vertices by triangle id, the index of vertex j in vj.w: shading
+// and the adjoint read one 48-byte record where idx and then pos would be two
+// dependent gathers of twelve words (the checkpointed adjoint waits on memory
+// for three quarters of its wave cycles).
+struct alignas(16) TriVerts {
+  float v0[4];
+  float v1[4];
+  float v2[4];
+};
+
 // Per-triangle shading data (Scene::PostIntersect inputs, Scene.cpp:668-730).
 struct alignas(16) TriShade {
   float n[3];        // geometric (face) normal, normalize(cross(p1-p0, p2-p0))
@@ -297,6 +308,7 @@ struct SceneDev {
   const uint32_t* uv_idx;   // uint32[T][3] or null
   const TriShade* shade;
   const TriRecord* tris;
+  const TriVerts* verts;
   const Bvh4Node* nodes;
   const QNode* qnodes;
   const Material* mats;

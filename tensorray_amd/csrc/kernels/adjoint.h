@@ -391,16 +391,18 @@ template <class Sink>
 __device__ inline void tri_flush(const SceneDev& S, int32_t tri, const TriAdj& a, Sink& sk) {
   if (tri < 0) return;
   if (!(S.shade[tri].flags & kTriDiff)) return;
-  uint32_t v[3] = {S.idx[3 * tri], S.idx[3 * tri + 1], S.idx[3 * tri + 2]};
+  const TriCorners q = tri_corners(S, tri);
+  uint32_t v[3] = {q.i0, q.i1, q.i2};
   F3 aa[3] = {a.a0, a.a1, a.a2};
 #pragma unroll
   for (int j = 0; j < 3; ++j) sk.pos(v[j], aa[j]);
 }
 
 __device__ inline void tri_verts(const SceneDev& S, int32_t tri, F3& p0, F3& p1, F3& p2) {
-  p0 = load3(S.pos, S.idx[3 * tri]);
-  p1 = load3(S.pos, S.idx[3 * tri + 1]);
-  p2 = load3(S.pos, S.idx[3 * tri + 2]);
+  const TriCorners q = tri_corners(S, tri);
+  p0 = q.p0;
+  p1 = q.p1;
+  p2 = q.p2;
 }
 
 // Backward sweep over a recorded path.  g = dL/dI of the pixel times 1/spp;
@@ -559,9 +561,9 @@ __device__ void path_backward(const SceneDev& S, const CameraDev& C, const PathP
       adj_ng += adj_ns;  // flat shading: ns = ng
     } else if (sk.has_vn() && (tflags & kTriDiff)) {
       // ns = w n0 + u n1 + v n2 (vertex normals, not renormalized)
-      const uint32_t k0 = S.idx[3 * ti], k1 = S.idx[3 * ti + 1], k2 = S.idx[3 * ti + 2];
+      const TriCorners q = tri_corners(S, ti);
       const F3 c[3] = {w * adj_ns, u * adj_ns, v * adj_ns};
-      const uint32_t ks[3] = {k0, k1, k2};
+      const uint32_t ks[3] = {q.i0, q.i1, q.i2};
 #pragma unroll
       for (int j = 0; j < 3; ++j) sk.vn(ks[j], c[j]);
     }

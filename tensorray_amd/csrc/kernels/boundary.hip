@@ -266,21 +266,21 @@ __device__ inline F3 dLdI_at(const float* dLdI, uint32_t WH, int32_t pix) {
 template <class Sink>
 __device__ void scatter_xdn(const SceneDev& S, int32_t tri, F3 org, F3 through, F3 n, float w, const EdgeDev* edge,
                             float et, int32_t ef0, int32_t otri, float ou, float ov, Sink& sk) {
-  F3 P0, P1, P2;
-  tri_verts(S, tri, P0, P1, P2);
-  XdnAdj a = x_dot_n_vjp(P0, P1, P2, org, through, n, w);
-  vtx_add(S, S.idx[3 * tri], tri, a.P0, sk);
-  vtx_add(S, S.idx[3 * tri + 1], tri, a.P1, sk);
-  vtx_add(S, S.idx[3 * tri + 2], tri, a.P2, sk);
+  const TriCorners q = tri_corners(S, tri);
+  XdnAdj a = x_dot_n_vjp(q.p0, q.p1, q.p2, org, through, n, w);
+  vtx_add(S, q.i0, tri, a.P0, sk);
+  vtx_add(S, q.i1, tri, a.P1, sk);
+  vtx_add(S, q.i2, tri, a.P2, sk);
   if (edge) {
     vtx_add(S, edge->v0, ef0, (1.0f - et) * a.through, sk);
     vtx_add(S, edge->v1, ef0, et * a.through, sk);
   }
   if (otri >= 0) {
     float ow = 1.0f - ou - ov;
-    vtx_add(S, S.idx[3 * otri], otri, ow * a.org, sk);
-    vtx_add(S, S.idx[3 * otri + 1], otri, ou * a.org, sk);
-    vtx_add(S, S.idx[3 * otri + 2], otri, ov * a.org, sk);
+    const TriCorners oq = tri_corners(S, otri);
+    vtx_add(S, oq.i0, otri, ow * a.org, sk);
+    vtx_add(S, oq.i1, otri, ou * a.org, sk);
+    vtx_add(S, oq.i2, otri, ov * a.org, sk);
   }
 }
 

@@ -98,10 +98,15 @@ struct PrimPred {
   }
 };
 
-__global__ void k_face_normals(const float* pos, const uint32_t* idx, TriShade* shade, uint32_t T) {
+__global__ void k_face_normals(const float* pos, const uint32_t* idx, TriShade* shade, TriVerts* verts, uint32_t T) {
   const uint32_t t = blockIdx.x * kUpdBlock + threadIdx.x;
   if (t >= T) return;
-  const F3 p0 = pos3(pos, idx[3 * t]), p1 = pos3(pos, idx[3 * t + 1]), p2 = pos3(pos, idx[3 * t + 2]);
+  const uint32_t i0 = idx[3 * t], i1 = idx[3 * t + 1], i2 = idx[3 * t + 2];
+  const F3 p0 = pos3(pos, i0), p1 = pos3(pos, i1), p2 = pos3(pos, i2);
+  float4* q = reinterpret_cast<float4*>(verts + t);
+  q[0] = make_float4(p0.x, p0.y, p0.z, __uint_as_float(i0));
+  q[1] = make_float4(p1.x, p1.y, p1.z, __uint_as_float(i1));
+  q[2] = make_float4(p2.x, p2.y, p2.z, __uint_as_float(i2));
   const F3 c = cross(p1 - p0, p2 - p0);
   const float l = length(c);
   const F3 n = c / l;
@@ -324,18 +329,20 @@ __global__ void k_edge_cdf_norm(float* cdf, uint32_t cap, const EdgeCount* count
   cdf[i] = cdf[i] / integral;
 }
 
-// Triangle records in leaf order follow the new positions (the triangle id
-// stays in v0[3]).
-__global__ void k_tri_records(const float* pos, const uint32_t* idx, TriRecord* tris, uint32_t T) {
+// Triangle records in leaf order follow the new positions, read from the
+// records by id (the triangle id stays in v0[3]).
+__global__ void k_tri_records(const TriVerts* verts, TriRecord* tris, uint32_t T) {
   const uint32_t i = blockIdx.x * kUpdBlock + threadIdx.x;
   if (i >= T) return;
-  TriRecord& r = tris[i];
-  const uint32_t t = __float_as_uint(r.v0[3]);
-  for (int k = 0; k < 3; ++k) {
-    r.v0[k] = pos[3 * (size_t)idx[3 * t] + k];
-    r.v1[k] = pos[3 * (size_t)idx[3 * t + 1] + k];
-    r.v2[k] = pos[3 * (size_t)idx[3 * t + 2] + k];
-  }
+  float4* r = reinterpret_cast<float4*>(tris + i);
+  const float id = tris[i].v0[3];
+  const float4* q = reinterpret_cast<const float4*>(verts + __float_as_uint(id));
+  float4 a = q[0], b = q[1], c = q[2];
+  a.w = id;
+  b.w = c.w = 0.0f;
+  r[0] = a;
+  r[1] = b;
+  r[2] = c;
 }
 
 // One level of the refit: every node's child boxes from its leaves'
@@ -458,7 +465,8 @@ hipError_t launch_scene_update(const SceneDev& S, const SceneUpdateDev& U, hipSt
   const float* pos = S.pos;
   const uint32_t T = (uint32_t)S.n_tris, V = (uint32_t)S.n_verts;
   if (T == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_face_normals, dim3(blocks_for(T)), dim3(kUpdBlock), 0, st, pos, S.idx, shade, T);
+  hipLaunchKernelGGL(k_face_normals, dim3(blocks_for(T)), dim3(kUpdBlock), 0, st, pos, S.idx, shade,
+                     const_cast<TriVerts*>(S.verts), T);
   if (U.vs_off)
     hipLaunchKernelGGL(k_vertex_normals, dim3(blocks_for(V)), dim3(kUpdBlock), 0, st, (const TriShade*)shade,
                        U.vs_off, U.vs_list, const_cast<float*>(S.vnrm), V);
@@ -474,7 +482,7 @@ hipError_t launch_scene_update(const SceneDev& S, const SceneUpdateDev& U, hipSt
   }
   TriRecord* tris = const_cast<TriRecord*>(S.tris);
   Bvh4Node* nodes = const_cast<Bvh4Node*>(S.nodes);
-  hipLaunchKernelGGL(k_tri_records, dim3(blocks_for(T)), dim3(kUpdBlock), 0, st, pos, S.idx, tris, T);
+  hipLaunchKernelGGL(k_tri_records, dim3(blocks_for(T)), dim3(kUpdBlock), 0, st, S.verts, tris, T);
   for (size_t l = 0; l + 1 < U.level_off.size(); ++l) {
     const uint32_t a = U.level_off[l], n = U.level_off[l + 1] - a;
     if (n == 0) continue;
