@@ -96,6 +96,28 @@ GradCopies make_grad_copies(int n_verts, hipStream_t st) {
   return g;
 }
 
+// Stream-ordered scratch of the passes that trace their own checkpoint, in the
+// largest window (halved down to 32k paths) that can be allocated; null when
+// none can.
+struct ReplayScratch {
+  void* ptr = nullptr;
+  uint64_t window = 0;
+  hipStream_t st;
+  ReplayScratch(uint64_t npaths, int max_bounces, hipStream_t stream) : window(replay_window(npaths)), st(stream) {
+    while (hipMallocAsync(&ptr, (size_t)replay_bytes(window, max_bounces), st) != hipSuccess) {
+      (void)hipGetLastError();
+      ptr = nullptr;
+      if (window <= (32u << 10)) return;
+      window = (window / 2 + 63) / 64 * 64;
+    }
+  }
+  ~ReplayScratch() {
+    if (ptr) hipFreeAsync(ptr, st);
+  }
+  ReplayScratch(const ReplayScratch&) = delete;
+  ReplayScratch& operator=(const ReplayScratch&) = delete;
+};
+
 // Words of a stream's spill buffer: the traversal stacks' spill area, then
 // the launches' tile counters (kTileCtrWords words: one for the forward's
 // camera rays and for the other kernels, one for its bounces).
@@ -1428,8 +1450,9 @@ trc_status trc_render_deriv(trc_scene* s, const trc_camera* cam, const trc_optio
     float* tvn = nullptr;
     if (s->vn_adj)
       hip_check(hipMallocAsync((void**)&tvn, 3 * (size_t)s->dev.n_verts * sizeof(float), st), "hipMallocAsync(tvn)");
-    const hipError_t e = launch_render_deriv(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, tpos, tmat, tvn,
-                                             dimg, st);
+    ReplayScratch rs((uint64_t)np, opt->max_bounces, st);
+    const hipError_t e = !rs.ptr ? hipErrorOutOfMemory : launch_render_deriv(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, tpos, tmat, tvn,
+                                             dimg, rs.ptr, rs.window, st);
     if (tvn) hipFreeAsync(tvn, st);
     hip_check(e, "k_render_deriv");
   });
@@ -1445,8 +1468,11 @@ trc_status trc_render_adj(trc_scene* s, const trc_camera* cam, const trc_options
     long long np = (long long)opt->spp * C.width * C.height;
     LaunchCfg L = make_cfg(s->ctx, s, (hipStream_t)stream, np);
     GradCopies gc = make_grad_copies(s->dev.n_verts, (hipStream_t)stream);
-    hipError_t e = launch_render_adj(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, dLdI, dpos, dmat, dtex,
-                                     s->vn_adj, gc, (hipStream_t)stream);
+    hipError_t e = hipErrorOutOfMemory;
+    ReplayScratch rs((uint64_t)np, opt->max_bounces, (hipStream_t)stream);
+    if (rs.ptr)
+      e = launch_render_adj(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, dLdI, dpos, dmat, dtex, s->vn_adj, gc,
+                            rs.ptr, rs.window, (hipStream_t)stream);
     if (gc.base) hipFreeAsync(gc.base, (hipStream_t)stream);
     hip_check(e, "k_render_adj");
   });

@@ -68,6 +68,16 @@ TR_HD CkptDev ckpt_view(void* base, uint64_t npaths, int max_bounces) {
   c.nv = (int32_t)nv;
   return c;
 }
+// The checkpoint of paths first .. first + count alone, in as many bytes as
+// ckpt_bytes(count): its planes are addressed by path index like a whole one's.
+TR_HD CkptDev ckpt_window(void* base, uint64_t first, uint64_t count, int max_bounces) {
+  CkptDev c = ckpt_view(base, count, max_bounces);
+  c.meta -= first;
+  c.tri -= first;
+  c.u -= first;
+  c.v -= first;
+  return c;
+}
 __device__ inline void ckpt_put_vertex(const CkptDev& c, uint64_t path, int i, int32_t tri, float u, float v) {
   const uint64_t k = (uint64_t)i * c.npaths + path;
   c.tri[k] = tri;

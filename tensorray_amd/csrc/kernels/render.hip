@@ -1,10 +1,13 @@
 // HIP kernels of the interior integrator and the ray-query entry point.
 //
-//   k_intersect     one ray per thread (trc_intersect)
-//   k_render_paths  persistent megakernel: one path per thread iteration,
-//                   per-path radiance to HBM (forward of PathTracer::Radiance)
-//   k_film_reduce   deterministic per-pixel sum over samples
-//   k_render_adj    persistent megakernel: replay + backward sweep per path
+//   k_intersect        one ray per lane (trc_intersect)
+//   k_primary          camera rays of 64 neighbouring paths per wave, first hits
+//   k_bounces          the surviving paths as a per-lane state machine; per-path
+//                      radiance to HBM (forward of PathTracer::Radiance)
+//   k_film_reduce      deterministic per-pixel sum over samples
+//   k_render_adj_ckpt  backward sweep of the paths of a checkpoint
+//   k_render_deriv     the same sweep into a derivative image
+//   k_batch_*          the passes over the jobs of a batch
 //
 // All kernels use 128-thread blocks; the traversal short stack lives in LDS
 // (kStackLds entries per thread, lane-interleaved) and spills to an HBM
@@ -126,37 +129,8 @@ __global__ void k_film_reduce(const float* paths, int spp, int wh, float* film) 
   film[2 * wh + pix] = sz * inv;
 }
 
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) k_render_adj(SceneDev S, CameraDev C, PathParams P, LaunchCfg L,
-                                                       uint64_t npaths, const float* dLdI, float* dpos,
-                                                       float* dmat, float* adj_vn, float* dtex, GradCopies gc) {
-  if (gc.base) dpos = gc.base + (size_t)(blockIdx.x % gc.copies) * gc.n3;
-  __shared__ uint32_t lds_stack[kTraceLdsWords * kBlock];
-  __shared__ float mat_grad[kMaxMatGrad * kMatGradStride];
-  for (int i = threadIdx.x; i < kMaxMatGrad * kMatGradStride; i += kBlock) mat_grad[i] = 0.0f;
-  __syncthreads();
-  TraceCtx tc = make_trace_ctx(lds_stack, L);
-  const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
-  const float inv_spp = 1.0f / (float)P.spp;
-  const uint64_t stride = (uint64_t)L.grid * kBlock;
-  for (uint64_t p = (uint64_t)blockIdx.x * kBlock + threadIdx.x; p < npaths; p += stride) {
-    const uint32_t pix = (uint32_t)(p % WH);
-    F3 g{dLdI[pix] * inv_spp, dLdI[WH + pix] * inv_spp, dLdI[2 * WH + pix] * inv_spp};
-    if (g.x == 0.0f && g.y == 0.0f && g.z == 0.0f) continue;
-    PathRec R;
-    path_forward<true>(S, C, P, p, tc, &R);
-    GradSink sk{dpos, mat_grad, adj_vn, dtex};
-    path_backward(S, C, P, R, g, sk);
-  }
-  __syncthreads();
-  if (dmat) {
-    const int n = (S.n_mats < kMaxMatGrad ? S.n_mats : kMaxMatGrad) * kMatGradStride;
-    for (int i = threadIdx.x; i < n; i += kBlock)
-      if (mat_grad[i] != 0.0f) atomicAdd(&dmat[i], mat_grad[i]);
-  }
-}
-
 // Adjoint from a path checkpoint: the path is re-evaluated from its recorded
-// hits (no traversal), then swept backwards as in k_render_adj.  Blocks take
+// hits (no traversal), then swept backwards (path_backward).  Blocks take
 // chunks of kAdjChunk consecutive paths from a counter (the next free chunk,
 // so no block idles while another still has several) and order each chunk
 // in LDS by path length (longest first, camera misses and zero dL/dI
@@ -165,39 +139,40 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAd
 // consecutive paths runs 2.6 vertices where its paths average 1.1.
 // Measured there: 1.84 ms unsorted, 1.40 with 256-path chunks, 1.12 with
 // 1,024, 1.04 with 1,024 fetched from the counter (2,048: 1.19).
+// Launches that would leave blocks without a chunk use shorter ones.
 constexpr int kAdjSortR = 8;                   // paths per thread per chunk
 constexpr int kAdjChunk = kBlock * kAdjSortR;
 constexpr int kLenBuckets = kMaxBounces + 2;   // K + 1 in 0 .. max_bounces + 1
 constexpr uint64_t kAdjTail = 256;             // paths per chunk at the end of a launch
 
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) k_render_adj_ckpt(SceneDev S, CameraDev C, PathParams P, LaunchCfg L,
-                                                            uint64_t first, uint64_t count, CkptDev ck,
-                                                            const float* dLdI, float* dpos, float* dmat, float* adj_vn,
-                                                            float* dtex, GradCopies gc, uint32_t* chunk_ctr) {
-  if (gc.base) dpos = gc.base + (size_t)(blockIdx.x % gc.copies) * gc.n3;
-  __shared__ float mat_grad[kMaxMatGrad * kMatGradStride];
+// Calls sweep(p) for the paths of [first, first + count) that skip(pixel) does
+// not drop and whose camera ray hit something, sorted as above.
+template <class Skip, class Sweep>
+__device__ inline void for_each_sorted(uint64_t first, uint64_t count, uint32_t WH, const CkptDev& ck,
+                                       uint32_t* chunk_ctr, Skip&& skip, Sweep&& sweep) {
   __shared__ uint32_t s_ch;
   __shared__ uint16_t order[kAdjChunk];
   __shared__ uint32_t bcount[kLenBuckets], bnext[kLenBuckets];
-  for (int i = threadIdx.x; i < kMaxMatGrad * kMatGradStride; i += kBlock) mat_grad[i] = 0.0f;
-  const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
-  const float inv_spp = 1.0f / (float)P.spp;
   const uint64_t end = first + count;
+  // a few chunks per block, whole rows of the block's threads each
+  const uint64_t want = count / ((uint64_t)gridDim.x * 4u) / kBlock * kBlock;
+  const uint64_t big = want < (uint64_t)kBlock ? (uint64_t)kBlock : (want > (uint64_t)kAdjChunk ? (uint64_t)kAdjChunk : want);
+  const uint64_t small = big < kAdjTail ? big : kAdjTail;
   // the last paths come in chunks of kAdjTail, so that the blocks finish
   // together: an eighth of the paths, at most two such chunks per block
   // (metric scene: 0.91 ms with 1,024-path chunks only, 0.86 with this tail)
-  const uint64_t tail_max = (uint64_t)gridDim.x * 2u * kAdjTail;
+  const uint64_t tail_max = (uint64_t)gridDim.x * 2u * small;
   const uint64_t tail = count / 8u < tail_max ? count / 8u : tail_max;
-  const uint64_t nbig = (count - tail) / kAdjChunk;
-  const uint64_t nchunks = nbig + (count - nbig * kAdjChunk + kAdjTail - 1) / kAdjTail;
+  const uint64_t nbig = (count - tail) / big;
+  const uint64_t nchunks = nbig + (count - nbig * big + small - 1) / small;
   for (;;) {
     if (threadIdx.x == 0) s_ch = atomicAdd(chunk_ctr, 1u);
     if (threadIdx.x < kLenBuckets) bcount[threadIdx.x] = 0u;
     __syncthreads();
     const uint64_t ch = s_ch;
     if (ch >= nchunks) break;  // s_ch is the block's: every thread leaves together
-    const uint64_t base = ch < nbig ? first + ch * kAdjChunk : first + nbig * kAdjChunk + (ch - nbig) * kAdjTail;
-    const uint64_t cend0 = base + (ch < nbig ? kAdjChunk : kAdjTail);
+    const uint64_t base = ch < nbig ? first + ch * big : first + nbig * big + (ch - nbig) * small;
+    const uint64_t cend0 = base + (ch < nbig ? big : small);
     const uint64_t cend = cend0 < end ? cend0 : end;
     uint32_t kb[kAdjSortR];
 #pragma unroll
@@ -205,10 +180,8 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAd
       const uint64_t p = base + threadIdx.x + (uint64_t)r * kBlock;
       kb[r] = 0u;
       if (p < cend) {
-        const uint32_t pix = (uint32_t)(p % WH);
-        const bool zero = dLdI[pix] == 0.0f && dLdI[WH + pix] == 0.0f && dLdI[2 * WH + pix] == 0.0f;
         const uint32_t k1 = ck.meta[p] & 0xFFu;
-        kb[r] = zero ? 0u : (k1 < (uint32_t)kLenBuckets ? k1 : (uint32_t)kLenBuckets - 1u);
+        kb[r] = skip((uint32_t)(p % WH)) ? 0u : (k1 < (uint32_t)kLenBuckets ? k1 : (uint32_t)kLenBuckets - 1u);
         if (kb[r]) atomicAdd(&bcount[kb[r]], 1u);
       }
     }
@@ -227,19 +200,33 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAd
       if (kb[r]) order[atomicAdd(&bnext[kb[r]], 1u)] = (uint16_t)(threadIdx.x + r * kBlock);
     __syncthreads();
     const uint32_t nsweep = bcount[0];
-    for (uint32_t j = threadIdx.x; j < nsweep; j += kBlock) {
-      const uint64_t p = base + order[j];
-      const uint32_t pix = (uint32_t)(p % WH);
-      F3 g{dLdI[pix] * inv_spp, dLdI[WH + pix] * inv_spp, dLdI[2 * WH + pix] * inv_spp};
-      CkptSrc src{&ck, p, ck.meta[p]};
-      PathRec R;
-      path_forward<true>(S, C, P, p, src, &R);
-      GradSink sk{dpos, mat_grad, adj_vn, dtex};
-      path_backward(S, C, P, R, g, sk);
-    }
+    for (uint32_t j = threadIdx.x; j < nsweep; j += kBlock) sweep(base + order[j]);
     __syncthreads();  // order / bcount are reused by the next chunk
   }
   __syncthreads();
+}
+
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdjWaves)))
+k_render_adj_ckpt(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, uint64_t first, uint64_t count, CkptDev ck,
+                  const float* dLdI, float* dpos, float* dmat, float* adj_vn, float* dtex, GradCopies gc,
+                  uint32_t* chunk_ctr) {
+  if (gc.base) dpos = gc.base + (size_t)(blockIdx.x % gc.copies) * gc.n3;
+  __shared__ float mat_grad[kMaxMatGrad * kMatGradStride];
+  for (int i = threadIdx.x; i < kMaxMatGrad * kMatGradStride; i += kBlock) mat_grad[i] = 0.0f;
+  const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
+  const float inv_spp = 1.0f / (float)P.spp;
+  for_each_sorted(
+      first, count, WH, ck, chunk_ctr,
+      [&](uint32_t pix) { return dLdI[pix] == 0.0f && dLdI[WH + pix] == 0.0f && dLdI[2 * WH + pix] == 0.0f; },
+      [&](uint64_t p) {
+        const uint32_t pix = (uint32_t)(p % WH);
+        F3 g{dLdI[pix] * inv_spp, dLdI[WH + pix] * inv_spp, dLdI[2 * WH + pix] * inv_spp};
+        CkptSrc src{&ck, p, ck.meta[p]};
+        PathRec R;
+        path_forward<true>(S, C, P, p, src, &R);
+        GradSink sk{dpos, mat_grad, adj_vn, dtex};
+        path_backward(S, C, P, R, g, sk);
+      });
   if (dmat) {
     const int n = (S.n_mats < kMaxMatGrad ? S.n_mats : kMaxMatGrad) * kMatGradStride;
     for (int i = threadIdx.x; i < n; i += kBlock)
@@ -250,31 +237,31 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAd
 // Derivative image of the interior integrator along one parameter tangent
 // (the reference's export_deriv: GradiantImageHandler::AccumulateDeriv,
 // Integrator.cpp:338-373, the forward-mode derivative of every path's
-// contribution): each path is replayed once and swept backwards three
-// times, with the seeds e_r, e_g, e_b / spp, into a TangentSink; the sums
-// are the derivatives of the path's RGB contribution and go to
-// dimg[c][pixel].  Non-finite derivatives are dropped, as the reference
+// contribution): each path is re-evaluated once from its checkpoint and swept
+// backwards three times, with the seeds e_r, e_g, e_b / spp, into a
+// TangentSink; the sums are the derivatives of the path's RGB contribution and
+// go to dimg[c][pixel].  Non-finite derivatives are dropped, as the reference
 // filters its derivative images (Integrator.cpp:364-367).
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) k_render_deriv(SceneDev S, CameraDev C, PathParams P, LaunchCfg L,
-                                                         uint64_t npaths, const float* tpos, const float* tmat,
-                                                         const float* tvn, float* dimg) {
-  __shared__ uint32_t lds_stack[kTraceLdsWords * kBlock];
-  TraceCtx tc = make_trace_ctx(lds_stack, L);
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdjWaves)))
+k_render_deriv(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, uint64_t first, uint64_t count, CkptDev ck,
+               const float* tpos, const float* tmat, const float* tvn, float* dimg, uint32_t* chunk_ctr) {
   const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
   const float inv_spp = 1.0f / (float)P.spp;
-  const uint64_t stride = (uint64_t)L.grid * kBlock;
-  for (uint64_t p = (uint64_t)blockIdx.x * kBlock + threadIdx.x; p < npaths; p += stride) {
-    const uint32_t pix = (uint32_t)(p % WH);
-    PathRec R;
-    path_forward<true>(S, C, P, p, tc, &R);
+  for_each_sorted(
+      first, count, WH, ck, chunk_ctr, [](uint32_t) { return false; },
+      [&](uint64_t p) {
+        const uint32_t pix = (uint32_t)(p % WH);
+        CkptSrc src{&ck, p, ck.meta[p]};
+        PathRec R;
+        path_forward<true>(S, C, P, p, src, &R);
 #pragma unroll 1
-    for (int c = 0; c < 3; ++c) {
-      const F3 g{c == 0 ? inv_spp : 0.0f, c == 1 ? inv_spp : 0.0f, c == 2 ? inv_spp : 0.0f};
-      TangentSink sk{tpos, tmat, tvn, 0.0f};
-      path_backward(S, C, P, R, g, sk);
-      if (sk.acc != 0.0f && isfinite(sk.acc)) atomicAdd(&dimg[(size_t)c * WH + pix], sk.acc);
-    }
-  }
+        for (int c = 0; c < 3; ++c) {
+          const F3 g{c == 0 ? inv_spp : 0.0f, c == 1 ? inv_spp : 0.0f, c == 2 ? inv_spp : 0.0f};
+          TangentSink sk{tpos, tmat, tvn, 0.0f};
+          path_backward(S, C, P, R, g, sk);
+          if (sk.acc != 0.0f && isfinite(sk.acc)) atomicAdd(&dimg[(size_t)c * WH + pix], sk.acc);
+        }
+      });
 }
 
 __global__ void __launch_bounds__(kBlock) k_vertex_normal_tangent(SceneDev S, const float* tpos, float* tvn) {
@@ -729,15 +716,48 @@ size_t noalloc_scratch_bytes() { return kNoAllocScratchBytes; }
 
 hipError_t noalloc_scratch_address(void** out) { return hipGetSymbolAddress(out, HIP_SYMBOL(scratch)); }
 
+// Paths per window of the passes that trace their own checkpoint: 248 MB of
+// scratch at 8 bounces.
+constexpr uint64_t kReplayWindow = 2u << 20;
+
+uint64_t replay_window(uint64_t npaths) { return npaths < kReplayWindow ? npaths : kReplayWindow; }
+uint64_t replay_bytes(uint64_t window, int max_bounces) { return 12ull * window + ckpt_bytes(window, max_bounces); }
+
+// Calls pass(first, count, checkpoint, chunk counter) for windows of the
+// request's paths, each traced into `scratch` (replay_bytes(window)) first.
+// One launch that re-traced a path and swept it backwards on the same lane
+// carried the adjoint's registers through the traversal (301 x 211 x 16 smooth
+// scene: 1.74 ms against 0.45 for the forward and 0.26 for the sweep).
+template <class Pass>
+static hipError_t replay_windows(const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
+                                 const LaunchCfg& L, void* scratch, uint64_t window, hipStream_t st, Pass&& pass) {
+  const uint64_t np = (uint64_t)spp * (uint64_t)C.width * (uint64_t)C.height;
+  if (!L.spill) return hipErrorInvalidValue;
+  for (uint64_t first = 0; first < np; first += window) {
+    const uint64_t count = first + window < np ? window : np - first;
+    float* paths = (float*)scratch;
+    const CkptDev ck = ckpt_window(paths + 3 * window, first, count, max_bounces);
+    hipError_t e = launch_paths<true>(S, C, PathParams{seed, max_bounces, spp, 0u}, L, first, count, paths, first, ck, st);
+    // the traversal is done with the stream's spill buffer: word 0 becomes the
+    // chunk counter of the sweep
+    if (e == hipSuccess) e = launch_fill_zero((float*)L.spill, 1, st);
+    if (e == hipSuccess) e = pass(first, count, ck);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t launch_render_adj(const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
                              const LaunchCfg& L, const float* dLdI, float* dpos, float* dmat, float* dtex,
-                             float* vn_adj, const GradCopies& gc, hipStream_t st) {
-  PathParams P{seed, max_bounces, spp, 0u};
-  uint64_t np = (uint64_t)spp * (uint64_t)C.width * (uint64_t)C.height;
-  const LaunchCfg Lk = fit_grid(k_render_adj, L);
-  hipLaunchKernelGGL(k_render_adj, dim3(Lk.grid), dim3(kBlock), 0, st, S, C, P, Lk, np, dLdI, dpos, dmat, vn_adj, dtex,
-                     gc);
-  hipError_t e = hipGetLastError();
+                             float* vn_adj, const GradCopies& gc, void* scratch, uint64_t window, hipStream_t st) {
+  const LaunchCfg Lk = fit_grid(k_render_adj_ckpt, L);
+  hipError_t e = replay_windows(
+      S, C, seed, max_bounces, spp, L, scratch, window, st, [&](uint64_t first, uint64_t count, const CkptDev& ck) {
+        hipLaunchKernelGGL(k_render_adj_ckpt, dim3(Lk.grid), dim3(kBlock), 0, st, S, C,
+                           (PathParams{seed, max_bounces, spp, 0u}), Lk, first, count, ck, dLdI, dpos, dmat, vn_adj,
+                           dtex, gc, L.spill);
+        return hipGetLastError();
+      });
   if (e == hipSuccess && gc.base) e = launch_grad_reduce(gc, dpos, st);
   if (e != hipSuccess || !vn_adj || S.n_verts == 0) return e;
   const int grid = (S.n_verts + kBlock - 1) / kBlock;
@@ -747,18 +767,19 @@ hipError_t launch_render_adj(const SceneDev& S, const CameraDev& C, uint32_t see
 
 hipError_t launch_render_deriv(const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
                                const LaunchCfg& L, const float* tpos, const float* tmat, float* tvn, float* dimg,
-                               hipStream_t st) {
-  const PathParams P{seed, max_bounces, spp, 0u};
-  const uint64_t np = (uint64_t)spp * (uint64_t)C.width * (uint64_t)C.height;
-  if (np == 0) return hipSuccess;
+                               void* scratch, uint64_t window, hipStream_t st) {
   if (tvn) {
     const unsigned nb = (unsigned)((S.n_verts + kBlock - 1) / kBlock);
     hipLaunchKernelGGL(k_vertex_normal_tangent, dim3(nb), dim3(kBlock), 0, st, S, tpos, tvn);
   }
   const LaunchCfg Lk = fit_grid(k_render_deriv, L);
-  hipLaunchKernelGGL(k_render_deriv, dim3(Lk.grid), dim3(kBlock), 0, st, S, C, P, Lk, np, tpos, tmat,
-                     (const float*)tvn, dimg);
-  return hipGetLastError();
+  return replay_windows(
+      S, C, seed, max_bounces, spp, L, scratch, window, st, [&](uint64_t first, uint64_t count, const CkptDev& ck) {
+        hipLaunchKernelGGL(k_render_deriv, dim3(Lk.grid), dim3(kBlock), 0, st, S, C,
+                           (PathParams{seed, max_bounces, spp, 0u}), Lk, first, count, ck, tpos, tmat,
+                           (const float*)tvn, dimg, L.spill);
+        return hipGetLastError();
+      });
 }
 
 }  // namespace trc

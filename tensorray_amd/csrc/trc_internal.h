@@ -313,11 +313,16 @@ hipError_t launch_boundary(int kind, const SceneDev& S, const CameraDev& C, uint
 // tangents when a differentiable mesh is smooth-shaded, else null.
 hipError_t launch_render_deriv(const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
                                const LaunchCfg& L, const float* tpos, const float* tmat, float* tvn, float* dimg,
-                               hipStream_t st);
+                               void* scratch, uint64_t window, hipStream_t st);
 // vn_adj: [V][3] zeroed scratch for smooth-shaded differentiable meshes or
 // null; it is folded into dpos and cleared again by a second kernel.
 hipError_t launch_render_adj(const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
                              const LaunchCfg& L, const float* dLdI, float* dpos, float* dmat, float* dtex,
-                             float* vn_adj, const GradCopies& gc, hipStream_t st);
+                             float* vn_adj, const GradCopies& gc, void* scratch, uint64_t window, hipStream_t st);
+// The replaying passes (launch_render_adj, launch_render_deriv) trace windows
+// of the request's paths into a checkpoint in `scratch`: the number of paths
+// per window for a request, and the bytes a window needs.
+uint64_t replay_window(uint64_t npaths);
+uint64_t replay_bytes(uint64_t window, int max_bounces);
 
 }  // namespace trc
