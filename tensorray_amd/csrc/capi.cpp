@@ -867,13 +867,19 @@ static void assign_grad_copies(std::vector<JobDev>& jd, float* base) {
   }
 }
 
-// Default tile: about four tiles per resident wave (waves take tiles
-// round-robin, so finer tiles even out paths of unequal length), at least
-// one path per lane, at most 4096 paths.
-static uint64_t default_tile(const trc_ctx* ctx, uint64_t total) {
+// Default tile.  Waves take tiles from a counter, which serves an atomic every
+// 11.5 ns: small tiles cost time there (and sort the adjoint's paths over few),
+// large ones leave waves behind at the end.  Forward: about three tiles per
+// wave of the launch, 64..256 paths; adjoint: about 8,192 tiles, 64..1024
+// paths.  2.2M paths in eight views, tiles of 64 / 128 / 256 / 512: forward
+// 1,215 / 1,153 / 1,353 / 1,833 us, adjoint 474 / 298 / 213 / 238; 59M paths in
+// 32 views, 64 / 256 / 1024: forward 26.8 / 21.0 / 21.6 ms, adjoint 11.3 / 4.0 /
+// 2.7; 63k paths in three views, 64 / 128: 170 / 261 and 86 / 91 us.
+static uint64_t default_tile(const trc_ctx* ctx, uint64_t total, int adjoint) {
   const uint64_t waves = (uint64_t)ctx->num_cus * kBlocksPerCU * (kBlock / 64);
-  uint64_t tile = total / (waves * 4) / 64 * 64;
-  return tile < 64 ? 64 : (tile > 4096 ? 4096 : tile);
+  const uint64_t tile = total / (adjoint ? 8192 : waves * 3) / 64 * 64;
+  const uint64_t top = adjoint ? 1024 : 256;
+  return tile < 64 ? 64 : (tile > top ? top : tile);
 }
 
 // In a batch that mixes scenes, jobs of at least this many paths (several
@@ -922,7 +928,7 @@ trc_status trc_render_batch(trc_ctx* ctx, const trc_job* jobs, int32_t n, int32_
     }
     LaunchCfg L = make_cfg(ctx, deepest, st, (long long)total);
     const uint64_t tiled = mark_solo(jd);
-    const uint64_t tile = default_tile(ctx, tiled);
+    const uint64_t tile = default_tile(ctx, tiled, adjoint);
     const uint64_t ntiles = assign_tiles(jd, tile);
     // job table: pinned staging -> device (stream-ordered), from a ring slot
     // whose previous batch has completed
@@ -1015,7 +1021,7 @@ trc_status trc_plan_create(trc_ctx* ctx, const trc_job* jobs, int32_t n, int32_t
       p->L.spill = p->spill;
       p->L.tiles = p->spill + words;
       p->tiled = mark_solo(p->jd);
-      plan_upload_tiles(p.get(), default_tile(ctx, p->tiled));
+      plan_upload_tiles(p.get(), default_tile(ctx, p->tiled, p->adjoint));
       hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     } catch (...) {
       plan_free(p.get());
@@ -1029,7 +1035,7 @@ trc_status trc_plan_set_tile(trc_plan* plan, uint32_t tile_paths) {
   if (!plan) return TRC_ERR_INVALID;
   return guarded(plan->ctx, [&] {
     if (tile_paths % 64 != 0) throw Fail(TRC_ERR_INVALID, "tile_paths must be a multiple of 64");
-    plan_upload_tiles(plan, tile_paths ? tile_paths : default_tile(plan->ctx, plan->tiled));
+    plan_upload_tiles(plan, tile_paths ? tile_paths : default_tile(plan->ctx, plan->tiled, plan->adjoint));
   });
 }
 
