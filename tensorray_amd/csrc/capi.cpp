@@ -119,9 +119,9 @@ struct ReplayScratch {
 };
 
 // Words of a stream's spill buffer: the traversal stacks' spill area, then
-// the launches' tile counters (kTileCtrWords words: one for the forward's
-// camera rays and for the other kernels, one for its bounces).
-constexpr size_t kTileCtrWords = 64;
+// the launches' tile counters (one set for the forward's camera rays and for
+// the other kernels, one for its bounces).
+constexpr size_t kTileCtrWords = 2 * kTileSet;
 static size_t spill_words(int max_grid) { return (size_t)kSpillDepth * (size_t)max_grid * kBlock; }
 
 // Launch shape for `work_items` items over scene `s`, with the spill buffer of
@@ -867,19 +867,14 @@ static void assign_grad_copies(std::vector<JobDev>& jd, float* base) {
   }
 }
 
-// Default tile.  Waves take tiles from a counter, which serves an atomic every
-// 11.5 ns: small tiles cost time there (and sort the adjoint's paths over few),
-// large ones leave waves behind at the end.  Forward: about three tiles per
-// wave of the launch, 64..256 paths; adjoint: about 8,192 tiles, 64..1024
-// paths.  2.2M paths in eight views, tiles of 64 / 128 / 256 / 512: forward
-// 1,215 / 1,153 / 1,353 / 1,833 us, adjoint 474 / 298 / 213 / 238; 59M paths in
-// 32 views, 64 / 256 / 1024: forward 26.8 / 21.0 / 21.6 ms, adjoint 11.3 / 4.0 /
-// 2.7; 63k paths in three views, 64 / 128: 170 / 261 and 86 / 91 us.
-static uint64_t default_tile(const trc_ctx* ctx, uint64_t total, int adjoint) {
-  const uint64_t waves = (uint64_t)ctx->num_cus * kBlocksPerCU * (kBlock / 64);
-  const uint64_t tile = total / (adjoint ? 8192 : waves * 3) / 64 * 64;
-  const uint64_t top = adjoint ? 1024 : 256;
-  return tile < 64 ? 64 : (tile > top ? top : tile);
+// Default tile.  Forward: 64 paths, a group of its blocked order.  Adjoint,
+// which sorts a tile's paths: about 8,192 tiles, 64..1024 paths.  Tiles of 64 /
+// 256 / 1024: 2.2M paths in eight views forward 1,068 / 1,345 / 2,933 us, adjoint
+// 232 / 181 / 338; 59M paths in 32 views 21.1 / 21.4 / 22.0 ms and 4.53 / 3.16 /
+// 2.94; 63k paths in three views 172 / 471 / 1,459 us and 81 / 114 / 240.
+static uint64_t default_tile(uint64_t total, int adjoint) {
+  const uint64_t tile = adjoint ? total / 8192 / 64 * 64 : 64;
+  return tile < 64 ? 64 : (tile > 1024 ? 1024 : tile);
 }
 
 // In a batch that mixes scenes, jobs of at least this many paths (several
@@ -928,7 +923,7 @@ trc_status trc_render_batch(trc_ctx* ctx, const trc_job* jobs, int32_t n, int32_
     }
     LaunchCfg L = make_cfg(ctx, deepest, st, (long long)total);
     const uint64_t tiled = mark_solo(jd);
-    const uint64_t tile = default_tile(ctx, tiled, adjoint);
+    const uint64_t tile = default_tile(tiled, adjoint);
     const uint64_t ntiles = assign_tiles(jd, tile);
     // job table: pinned staging -> device (stream-ordered), from a ring slot
     // whose previous batch has completed
@@ -1021,7 +1016,7 @@ trc_status trc_plan_create(trc_ctx* ctx, const trc_job* jobs, int32_t n, int32_t
       p->L.spill = p->spill;
       p->L.tiles = p->spill + words;
       p->tiled = mark_solo(p->jd);
-      plan_upload_tiles(p.get(), default_tile(ctx, p->tiled, p->adjoint));
+      plan_upload_tiles(p.get(), default_tile(p->tiled, p->adjoint));
       hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     } catch (...) {
       plan_free(p.get());

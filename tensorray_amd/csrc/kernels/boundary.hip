@@ -36,26 +36,19 @@ __device__ inline TraceCtx make_trace_ctx_b(uint32_t* lds, const LaunchCfg& L) {
 
 __device__ inline F3 cam_eye(const CameraDev& c) { return F3{c.eye[0], c.eye[1], c.eye[2]}; }
 
-// Calls f(i) for the items i of [first, end).  With a counter (zeroed before
-// the launch) a wave takes 64 consecutive items at a time as it finishes the
-// last ones, so no wave is left with a long tail of items dealt to it in
-// advance; without one, items are dealt grid-stride.  f returns to skip the
-// rest of an item.  All lanes of the wave must call it together.
+// Calls f(i) for the items i of [first, end), 64 consecutive ones per wave at
+// a time, taken from the launch's tile counters as waves need them (without
+// counters dealt round-robin).  f returns to skip the rest of an item.  All
+// lanes of the wave must call it together.
 template <class F>
-__device__ inline void for_each_item(uint64_t first, uint64_t end, uint32_t* ctr, const LaunchCfg& L, F&& f) {
-  if (ctr) {
-    const uint32_t lane = threadIdx.x & 63u;
-    for (;;) {
-      uint32_t c = 0u;
-      if (lane == 0u) c = atomicAdd(ctr, 1u);
-      c = (uint32_t)__shfl((int)c, 0);
-      const uint64_t i0 = first + (uint64_t)c * 64u;
-      if (i0 >= end) break;
-      if (i0 + lane < end) f(i0 + lane);
-    }
-  } else {
-    const uint64_t stride = (uint64_t)L.grid * kBlock;
-    for (uint64_t i = first + (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < end; i += stride) f(i);
+__device__ inline void for_each_item(uint64_t first, uint64_t end, const LaunchCfg& L, F&& f) {
+  const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
+  const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+  const uint32_t lane = threadIdx.x & 63u;
+  TileSupply sup = TileSupply::make(wave, nwaves, 0, end - first, 64, L.tiles);
+  while (sup.next < sup.end) {
+    if (sup.next + lane < sup.end) f(first + sup.next + lane);
+    sup.more();
   }
 }
 
@@ -369,7 +362,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
   const F3 eye = cam_eye(C);
   // no silhouette or boundary edge seen from this camera: no samples
   if ((E.dyn ? E.dyn->n : E.n) <= 0) return;
-  for_each_item(first, end, L.tiles, L, [&](uint64_t i) {
+  for_each_item(first, end, L, [&](uint64_t i) {
     bool keep = false;
     Hit h;
     SensorSample sd;
@@ -467,7 +460,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
   const float plx = 2.0f * C.ratio * C.tan_half, ply = 2.0f * C.tan_half;
   const F3 vdir = normalize(C.ay * U), hdir = normalize(C.ax * R);
   const uint64_t per_anti = N / 4;
-  for_each_item(0, N, L.tiles, L, [&](uint64_t i) {
+  for_each_item(0, N, L, [&](uint64_t i) {
     const uint64_t j = i % per_anti, anti = i / per_anti;
     float rr = rng4(P.seed, kRngPixelEdge, j, 0u).a;
     float rv;
@@ -529,7 +522,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
   TraceCtx tc = make_trace_ctx_b(lds_stack, L);
   const EdgeSet& E = S.sec;
   const uint64_t N = (uint64_t)G.n * (uint64_t)G.spp;
-  for_each_item(0, N, L.tiles, L, [&](uint64_t j) {
+  for_each_item(0, N, L, [&](uint64_t j) {
     const int32_t leaf = (int32_t)(j / (uint64_t)G.spp);
     Rnd4 r = rng4(seed, kRngGuide, j, 0u);
     const float x0 = leaf > 0 ? E.cdf[leaf - 1] : 0.0f, x1 = E.cdf[leaf];
@@ -676,7 +669,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
   __shared__ uint32_t lds_stack[kTraceLdsWords * kBlock];
   TraceCtx tc = make_trace_ctx_b(lds_stack, L);
   const EdgeSet& E = S.sec;
-  for_each_item(first, end, L.tiles, L, [&](uint64_t i) {
+  for_each_item(first, end, L, [&](uint64_t i) {
     bool keep = false;
     Hit h0, h;
     F3 K0, rdir, p, n;
@@ -804,7 +797,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
   __shared__ uint32_t lds_stack[kTraceLdsWords * kBlock];
   TraceCtx tc = make_trace_ctx_b(lds_stack, L);
   const EdgeSet& E = S.sec;
-  for_each_item(first, end, L.tiles, L, [&](uint64_t i) {
+  for_each_item(first, end, L, [&](uint64_t i) {
     bool keep = false;
     Hit he, hs;
     F3 dir, p, n;
@@ -948,7 +941,7 @@ hipError_t launch_guide_build(const SceneDev& S, const LaunchCfg& L, uint32_t se
                               hipStream_t st) {
   const LaunchCfg Lg = fit_grid(k_guide_eval, L);
   if (Lg.tiles) {
-    const hipError_t z = launch_fill_zero(reinterpret_cast<float*>(Lg.tiles), 1, st);
+    const hipError_t z = launch_fill_zero(reinterpret_cast<float*>(Lg.tiles), kTileSet, st);
     if (z != hipSuccess) return z;
   }
   hipLaunchKernelGGL(k_guide_eval, dim3(Lg.grid), dim3(kBlock), 0, st, S, Lg, seed, g);
@@ -984,7 +977,7 @@ static hipError_t launch_boundary_t(int kind, const SceneDev& S, const CameraDev
   if (kind == 1) {
     const LaunchCfg Lk = fit_grid(k_boundary_pixel<kTangent>, L);
     if (Lk.tiles) {
-      const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(Lk.tiles), 1, st);
+      const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(Lk.tiles), kTileSet, st);
       if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k_boundary_pixel<kTangent>, dim3(Lk.grid), dim3(kBlock), 0, st, S, C, P, Lk, N, dLdI, dpos,
@@ -1004,19 +997,19 @@ static hipError_t launch_boundary_t(int kind, const SceneDev& S, const CameraDev
     const BndQueue Q{counts + c, buf, cap};
     if (kind == 0) {
       const LaunchCfg Ls = fit_grid(k_bnd_primary_select, L), Le = fit_grid(k_bnd_primary_eval<kTangent>, L);
-      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), 1, st)) != hipSuccess) break;
+      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), kTileSet, st)) != hipSuccess) break;
       hipLaunchKernelGGL(k_bnd_primary_select, dim3(Ls.grid), dim3(kBlock), 0, st, S, C, P, Ls, prim, first, end, Q);
       hipLaunchKernelGGL(k_bnd_primary_eval<kTangent>, dim3(Le.grid), dim3(kBlock), 0, st, S, C, P, Le, prim, Q,
                          dLdI, dpos, tpos, dimg);
     } else if (kind == 2) {
       const LaunchCfg Ls = fit_grid(k_bnd_direct_select, L), Le = fit_grid(k_bnd_direct_eval<kTangent>, L);
-      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), 1, st)) != hipSuccess) break;
+      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), kTileSet, st)) != hipSuccess) break;
       hipLaunchKernelGGL(k_bnd_direct_select, dim3(Ls.grid), dim3(kBlock), 0, st, S, C, P, Ls, guide, first, end, Q);
       hipLaunchKernelGGL(k_bnd_direct_eval<kTangent>, dim3(Le.grid), dim3(kBlock), 0, st, S, C, P, Le, Q, dLdI, dpos,
                          tpos, dimg);
     } else {
       const LaunchCfg Ls = fit_grid(k_bnd_indirect_select, L), Le = fit_grid(k_bnd_indirect_eval<kTangent>, L);
-      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), 1, st)) != hipSuccess) break;
+      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), kTileSet, st)) != hipSuccess) break;
       hipLaunchKernelGGL(k_bnd_indirect_select, dim3(Ls.grid), dim3(kBlock), 0, st, S, C, P, Ls, first, end, Q);
       hipLaunchKernelGGL(k_bnd_indirect_eval<kTangent>, dim3(Le.grid), dim3(kBlock), 0, st, S, C, P, Le, Q, dLdI,
                          dpos, tpos, dimg);

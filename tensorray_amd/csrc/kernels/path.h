@@ -345,45 +345,42 @@ __device__ inline NeeGeo nee_geo(const SceneDev& S, const Its& its, float la, fl
   return g;
 }
 
-// How the slots of a launch are cut into tiles: `nbig` tiles of `big` slots,
-// then tiles of `tile`.  One counter serves an atomic every 11.5 ns (65,536
-// tiles of 64 paths: 0.755 ms, whatever the paths cost), so most slots go out
-// in big tiles and the last ones in small ones, which let the waves finish
-// together.
-struct TileDeal {
-  uint64_t slots, nbig, ntiles;
-  uint32_t big, tile;
-};
-
-// The path ranges a wave renders: its tiles of a range of slots that starts at
-// tile t0 of the launch.  The wave moves to its next tile as soon as the
-// current one is handed out, without waiting for its lanes to drain.  All
-// fields are wave-uniform.
+// The slots a wave works on: its tiles of `tile` slots of a range of `slots`
+// that starts at tile t0 of the launch.  The wave moves to its next tile as
+// soon as the current one is handed out, without waiting for its lanes to
+// drain.  All fields are wave-uniform.
+//
+// Tile counters: when set, the wave's tiles after its first (tile t, one per
+// wave: tiles 0 .. step-1 of the launch are dealt so) are taken as the wave
+// needs one; otherwise t, t + step, ...  One word serves an atomic every
+// 11.5 ns (65,536 tiles of 64 paths: 0.755 ms, whatever the paths cost), so
+// there are kTileCtrs of them, each in its own cache line, which share the
+// tiles evenly; a wave uses that of its block (blocks b and b + 8 run on one
+// XCD).  Tile numbers count over the whole launch.
 struct TileSupply {
-  uint64_t next, end;            // slots not yet handed out of the current tile
-  uint64_t t, tend, step;        // tile cursor
-  uint64_t t0;
-  TileDeal deal;
-  // tile counter: when set, the wave's tiles after its first (tile t, one
-  // per wave: tiles 0 .. step-1 of the launch are dealt so) are step + the
-  // counter's next value, taken as the wave needs one; otherwise t,
-  // t + step, ...  Tile numbers count over the whole launch.
+  uint64_t next, end;  // slots not yet handed out of the current tile
+  uint64_t t, tend, step;
+  uint64_t t0, slots;
+  uint32_t tile;
+  uint32_t q, nq;      // the wave's counter and how many there are
   uint32_t* ctr;
   __device__ void load() {
-    const uint64_t k = t - t0;
-    next = k < deal.nbig ? k * deal.big : deal.nbig * deal.big + (k - deal.nbig) * deal.tile;
-    end = next + (k < deal.nbig ? deal.big : deal.tile);
-    end = end < deal.slots ? end : deal.slots;
+    next = (t - t0) * tile;
+    end = next + tile < slots ? next + tile : slots;
   }
-  // Starts at tile t.
-  __device__ static TileSupply make(uint64_t t, uint64_t step, uint64_t t0, const TileDeal& deal, uint32_t* ctr) {
+  // Starts at tile t; ctr: the launch's counters or null.
+  __device__ static TileSupply make(uint64_t t, uint64_t step, uint64_t t0, uint64_t slots, uint32_t tile,
+                                    uint32_t* ctr) {
     TileSupply s;
     s.t = t;
-    s.tend = t0 + deal.ntiles;
     s.step = step;
     s.t0 = t0;
-    s.deal = deal;
-    s.ctr = ctr;
+    s.slots = slots;
+    s.tile = tile;
+    s.tend = t0 + (slots + tile - 1) / tile;
+    s.nq = gridDim.x < (uint32_t)kTileCtrs ? 1u : (uint32_t)kTileCtrs;
+    s.q = blockIdx.x % s.nq;
+    s.ctr = ctr ? ctr + s.q * (uint32_t)kTileCtrStride : nullptr;
     if (t < s.tend) s.load();
     else s.next = s.end = 0;
     return s;
@@ -395,19 +392,20 @@ struct TileSupply {
       next = end;
       return false;
     }
-    if (ctr) {
-      uint32_t v = 0u;
-      if ((threadIdx.x & 63u) == 0u) v = atomicAdd(ctr, 1u);
-      t = step + (uint64_t)(uint32_t)__shfl((int)v, 0);
-    } else {
-      t += step;
-    }
+    t = next_tile();
     if (t >= tend) {
       next = end;
       return false;
     }
     load();
     return true;
+  }
+  // The number of the wave's next tile.
+  __device__ uint64_t next_tile() const {
+    if (!ctr) return t + step;
+    uint32_t v = 0u;
+    if ((threadIdx.x & 63u) == 0u) v = atomicAdd(ctr, 1u);
+    return step + (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) * nq + q;
   }
 };
 

@@ -61,13 +61,13 @@ __global__ void __launch_bounds__(kBlock) k_intersect(SceneDev S, LaunchCfg L, c
 // Camera rays: a wave takes 64 slots at a time from the launch's counter.
 template <bool kCkpt>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWaves)))
-k_primary(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, TileDeal deal, float* paths,
+k_primary(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, uint32_t tile, float* paths,
           uint64_t paths_first, CkptDev ck) {
   __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
   TraceCtx tc = make_trace_ctx_wave(lds_stack, L);
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
   const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-  TileSupply sup = TileSupply::make(wave, nwaves, 0, deal, L.tiles);
+  TileSupply sup = TileSupply::make(wave, nwaves, 0, R.slots, tile, L.tiles);
   while (sup.next < sup.end) {
     trace_primary<kCkpt>(S, C, P, tc, PathGroup::at(C, R, sup.next), ck, paths, paths_first);
     sup.next += 64u;
@@ -77,13 +77,13 @@ k_primary(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, TileD
 
 template <bool kCkpt>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBounceWaves)))
-k_bounces(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, TileDeal deal, float* paths,
+k_bounces(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, uint32_t tile, float* paths,
           uint64_t paths_first, CkptDev ck) {
   __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
   TraceCtx tc = make_trace_ctx_wave(lds_stack, L);
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
   const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-  TileSupply sup = TileSupply::make(wave, nwaves, 0, deal, L.tiles ? L.tiles + 1 : nullptr);
+  TileSupply sup = TileSupply::make(wave, nwaves, 0, R.slots, tile, L.tiles ? L.tiles + kTileSet : nullptr);
   render_bounces<kCkpt>(S, C, P, tc, sup, R, ck, paths, paths_first,
                         [&](uint64_t p, F3 c) {
                           const uint64_t q = p - paths_first;
@@ -364,16 +364,10 @@ k_batch_primary(const JobDev* __restrict__ jobs, int njobs, uint64_t ntiles, uin
     const PathRange R = jobs[j].range;
     const uint64_t npaths = (uint64_t)P.spp * (uint64_t)C.width * (uint64_t)C.height;
     const CkptDev ck = ckpt_view(jobs[j].ckpt, npaths, P.max_bounces);
-    const uint64_t i0 = (t - jobs[j].tile0) * tile, i1 = i0 + tile < R.slots ? i0 + tile : R.slots;
-    for (uint64_t i = i0; i < i1; i += 64)
+    const TileSupply sup = TileSupply::make(t, nwaves, jobs[j].tile0, R.slots, tile, L.tiles);
+    for (uint64_t i = sup.next; i < sup.end; i += 64)
       trace_primary<true>(S, C, P, tc, PathGroup::at(C, R, i), ck, jobs[j].paths, 0);
-    if (L.tiles) {
-      uint32_t v = 0u;
-      if ((threadIdx.x & 63u) == 0u) v = atomicAdd(L.tiles, 1u);
-      t = nwaves + (uint64_t)(uint32_t)__shfl((int)v, 0);
-    } else {
-      t += nwaves;
-    }
+    t = sup.next_tile();
   }
 }
 
@@ -396,8 +390,7 @@ k_batch_bounces(const JobDev* __restrict__ jobs, int njobs, uint64_t ntiles, uin
     const CkptDev ck = ckpt_view(jobs[j].ckpt, npaths, P.max_bounces);
     float* paths = jobs[j].paths;
     // the wave's tiles of this job, rendered without draining between them
-    const TileDeal deal{slots, 0, (slots + tile - 1) / tile, 0u, tile};
-    TileSupply sup = TileSupply::make(t, nwaves, t0, deal, L.tiles ? L.tiles + 1 : nullptr);
+    TileSupply sup = TileSupply::make(t, nwaves, t0, slots, tile, L.tiles ? L.tiles + kTileSet : nullptr);
     render_bounces<true>(S, C, P, tc, sup, R, ck, paths, 0, [&](uint64_t p, F3 c) {
       paths[3 * p] = c.x;
       paths[3 * p + 1] = c.y;
@@ -505,13 +498,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAd
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    if (L.tiles) {
-      uint32_t v = 0u;
-      if (lane == 0) v = atomicAdd(L.tiles, 1u);
-      t = nwaves + (uint64_t)(uint32_t)__shfl((int)v, 0);
-    } else {
-      t += nwaves;
-    }
+    t = TileSupply::make(t, nwaves, t0, count, tile, L.tiles).next_tile();
   }
 }
 
@@ -534,14 +521,14 @@ hipError_t launch_render_batch(const JobDev* jobs_dev, const JobDev* jobs_host, 
   if (!adjoint) {
     if (ntiles == 0) return hipSuccess;
     const LaunchCfg Lp = fit_grid(k_batch_primary, L), Lb = fit_grid(k_batch_bounces, L);
-    if (L.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2, st)) != hipSuccess) return e;
+    if (L.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2 * kTileSet, st)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_batch_primary, dim3(Lp.grid), dim3(kBlock), 0, st, jobs_dev, njobs, ntiles, tile, Lp);
     hipLaunchKernelGGL(k_batch_bounces, dim3(Lb.grid), dim3(kBlock), 0, st, jobs_dev, njobs, ntiles, tile, Lb);
     return hipGetLastError();
   }
   if (ntiles > 0) {
     const LaunchCfg Lk = fit_grid(k_render_batch_adj, L);
-    if (Lk.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Lk.tiles), 1, st)) != hipSuccess) return e;
+    if (Lk.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Lk.tiles), kTileSet, st)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_render_batch_adj, dim3(Lk.grid), dim3(kBlock), 0, st, jobs_dev, njobs, ntiles, tile, Lk);
     e = hipGetLastError();
   }
@@ -569,27 +556,14 @@ hipError_t launch_intersect(const SceneDev& S, const LaunchCfg& L, const float* 
   return hipGetLastError();
 }
 
-// With the tile counter: big tiles, and small ones for the last slots (about
-// kDealTail per wave); dealt statically, about four tiles per wave, 64..4096
-// slots each.  512 x 512 step / 384 x 384 x 64 spp step with big tiles of 64:
-// 3.70 / 5.27 ms, 256 with a tail of 2: 3.48 / 5.22, of 4: 3.41 / 5.23, 512
-// with a tail of 2: 3.47 / 5.60.
-constexpr uint32_t kDealBig = 256, kDealTail = 4;
-static TileDeal deal_tiles(uint64_t slots, int grid, bool dynamic) {
+// Slots per tile: with the tile counters, small tiles taken as waves need them
+// (tiles of 64 / 256 from one counter: 512 x 512 step 3.70 / 3.48 ms); dealt
+// statically, about four tiles per wave, 64..4096 slots each.
+static uint32_t forward_tile(uint64_t slots, int grid, bool dynamic) {
+  if (dynamic) return 64u;
   const uint64_t waves = (uint64_t)grid * (kBlock / 64);
-  TileDeal d{slots, 0, 0, kDealBig, 64};
-  if (!dynamic) {
-    const uint64_t t = slots / (waves * 4) / 64 * 64;
-    d.tile = (uint32_t)(t < 64 ? 64 : (t > 4096 ? 4096 : t));
-    d.ntiles = (slots + d.tile - 1) / d.tile;
-    return d;
-  }
-  // big tiles only where each wave gets some of them
-  const uint64_t tail = waves * 64 * kDealTail;
-  while (d.big > 64 && slots < tail + waves * d.big * 2) d.big /= 2;
-  d.nbig = slots > tail ? (slots - tail) / d.big : 0;
-  d.ntiles = d.nbig + (slots - d.nbig * d.big + d.tile - 1) / d.tile;
-  return d;
+  const uint64_t t = slots / (waves * 4) / 64 * 64;
+  return (uint32_t)(t < 64 ? 64 : (t > 4096 ? 4096 : t));
 }
 
 template <bool kCkpt>
@@ -598,14 +572,14 @@ static hipError_t launch_paths(const SceneDev& S, const CameraDev& C, const Path
                                hipStream_t st) {
   const LaunchCfg Lp = fit_grid(k_primary<kCkpt>, L), Lb = fit_grid(k_bounces<kCkpt>, L);
   if (L.tiles) {
-    const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2, st);
+    const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2 * kTileSet, st);
     if (e != hipSuccess) return e;
   }
   const PathRange R = path_range(C, first, count);
   hipLaunchKernelGGL((k_primary<kCkpt>), dim3(Lp.grid), dim3(kBlock), 0, st, S, C, P, Lp, R,
-                     deal_tiles(R.slots, Lp.grid, L.tiles != nullptr), paths, paths_first, ck);
+                     forward_tile(R.slots, Lp.grid, L.tiles != nullptr), paths, paths_first, ck);
   hipLaunchKernelGGL((k_bounces<kCkpt>), dim3(Lb.grid), dim3(kBlock), 0, st, S, C, P, Lb, R,
-                     deal_tiles(R.slots, Lb.grid, L.tiles != nullptr), paths, paths_first, ck);
+                     forward_tile(R.slots, Lb.grid, L.tiles != nullptr), paths, paths_first, ck);
   return hipGetLastError();
 }
 

@@ -147,8 +147,11 @@ struct LaunchCfg {
   uint32_t* spill;      // spill buffer [depth][grid*kBlock]
   int cap;              // stack capacity
   int cus;              // compute units of the device
-  uint32_t* tiles;      // tile counters (two words, zeroed per launch); null: tiles dealt statically
+  uint32_t* tiles;      // two sets of tile counters (zeroed before a launch); null: tiles dealt statically
 };
+// A set of tile counters: kTileCtrs words in cache lines of their own.
+constexpr int kTileCtrs = 8, kTileCtrStride = 32;
+constexpr int kTileSet = kTileCtrs * kTileCtrStride;
 
 // A persistent grid-stride kernel should not launch more blocks than can be
 // resident at once: blocks beyond that only start when resident ones have
