@@ -1030,7 +1030,7 @@ trc_status trc_plan_set_tile(trc_plan* plan, uint32_t tile_paths) {
   if (!plan) return TRC_ERR_INVALID;
   return guarded(plan->ctx, [&] {
     if (tile_paths % 64 != 0) throw Fail(TRC_ERR_INVALID, "tile_paths must be a multiple of 64");
-    plan_upload_tiles(plan, tile_paths ? tile_paths : default_tile(plan->ctx, plan->tiled, plan->adjoint));
+    plan_upload_tiles(plan, tile_paths ? tile_paths : default_tile(plan->tiled, plan->adjoint));
   });
 }
 
