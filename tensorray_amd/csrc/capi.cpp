@@ -96,26 +96,33 @@ GradCopies make_grad_copies(int n_verts, hipStream_t st) {
   return g;
 }
 
-// Stream-ordered scratch of the passes that trace their own checkpoint, in the
-// largest window (halved down to 32k paths) that can be allocated; null when
-// none can.
-struct ReplayScratch {
+// Stream-ordered scratch of a pass that runs in windows of paths or samples:
+// bytes(window), for the largest window (halved down to 32k) that can be
+// allocated; null when none can.
+struct WindowScratch {
   void* ptr = nullptr;
   uint64_t window = 0;
   hipStream_t st;
-  ReplayScratch(uint64_t npaths, int max_bounces, hipStream_t stream) : window(replay_window(npaths)), st(stream) {
-    while (hipMallocAsync(&ptr, (size_t)replay_bytes(window, max_bounces), st) != hipSuccess) {
+  template <class Bytes>
+  WindowScratch(uint64_t first_window, hipStream_t stream, Bytes&& bytes) : window(first_window), st(stream) {
+    while (hipMallocAsync(&ptr, (size_t)bytes(window), st) != hipSuccess) {
       (void)hipGetLastError();
       ptr = nullptr;
       if (window <= (32u << 10)) return;
       window = (window / 2 + 63) / 64 * 64;
     }
   }
-  ~ReplayScratch() {
+  ~WindowScratch() {
     if (ptr) hipFreeAsync(ptr, st);
   }
-  ReplayScratch(const ReplayScratch&) = delete;
-  ReplayScratch& operator=(const ReplayScratch&) = delete;
+  WindowScratch(const WindowScratch&) = delete;
+  WindowScratch& operator=(const WindowScratch&) = delete;
+};
+// that of a pass which traces its own checkpoint
+struct ReplayScratch : WindowScratch {
+  ReplayScratch(uint64_t npaths, int max_bounces, hipStream_t stream)
+      : WindowScratch(replay_window(npaths), stream,
+                      [=](uint64_t window) { return replay_bytes(window, max_bounces); }) {}
 };
 
 // Words of a stream's spill buffer: the traversal stacks' spill area, then
@@ -1409,7 +1416,16 @@ static void boundary_call(trc_scene* s, const trc_camera* cam, const trc_options
     }
   }
   LaunchCfg L = make_cfg(s->ctx, s, st, N);
-  const size_t qb = (size_t)boundary_queue_bytes(kind, (uint64_t)N);
+  if (kind == 1) {
+    // of the call alone: pixel terms of one scene may run on several streams
+    WindowScratch q(kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes((uint64_t)N, chunk) + 4; });
+    hip_check(!q.ptr ? hipErrorOutOfMemory
+                     : launch_boundary(kind, s->dev, C, opt->seed, opt->max_bounces, spp, L, prim, guide, dLdI, dpos,
+                                       tpos, dimg, q.ptr, q.window, st),
+              "k_boundary");
+    return;
+  }
+  const size_t qb = (size_t)boundary_queue_bytes((uint64_t)N, kBndChunk);
   if (s->bq_buf.bytes < qb) {
     hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
     if (s->bq_buf.ptr) hipFree(s->bq_buf.ptr);
@@ -1419,7 +1435,7 @@ static void boundary_call(trc_scene* s, const trc_camera* cam, const trc_options
     s->bq_buf.bytes = qb;
   }
   hip_check(launch_boundary(kind, s->dev, C, opt->seed, opt->max_bounces, spp, L, prim, guide, dLdI, dpos, tpos,
-                            dimg, s->bq_buf.ptr, st),
+                            dimg, s->bq_buf.ptr, kBndChunk, st),
             "k_boundary");
 }
 

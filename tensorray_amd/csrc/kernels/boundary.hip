@@ -36,20 +36,46 @@ __device__ inline TraceCtx make_trace_ctx_b(uint32_t* lds, const LaunchCfg& L) {
 
 __device__ inline F3 cam_eye(const CameraDev& c) { return F3{c.eye[0], c.eye[1], c.eye[2]}; }
 
-// Calls f(i) for the items i of [first, end), 64 consecutive ones per wave at
-// a time, taken from the launch's tile counters as waves need them (without
-// counters dealt round-robin).  f returns to skip the rest of an item.  All
-// lanes of the wave must call it together.
+// Context with the slots of the wave-wide leaf tests (trace_run<true>).
+__device__ inline TraceCtx make_trace_ctx_bw(uint32_t* lds, const LaunchCfg& L) {
+  TraceCtx t = make_trace_ctx_b(lds, L);
+  uint32_t* slots = lds + kTraceLdsWords * kBlock;
+  t.slot_key = reinterpret_cast<unsigned long long*>(slots) + threadIdx.x;
+  t.slot_uv = reinterpret_cast<float2*>(slots + 2 * kBlock) + threadIdx.x;
+  return t;
+}
+
+// One ray per lane with `has`, the whole wave together.
+__device__ inline Hit trace_wave(const SceneDev& S, TraceCtx& tc, bool has, F3 o, F3 d, float tmax, bool any) {
+  TraceState ts;
+  if (has) trace_begin(ts, tmax);
+  else trace_none(ts);
+  trace_run<true>(S, tc, o, d, d, tmax, kShadowEpsilon, any, ts, 0);
+  return trace_hit(ts);
+}
+
+// Calls f(i, has) for the items i of [first, end), 64 consecutive ones per
+// wave at a time, taken from the launch's tile counters as waves need them
+// (without counters dealt round-robin), with all lanes of the wave: has is
+// false for those behind the last item.
 template <class F>
-__device__ inline void for_each_item(uint64_t first, uint64_t end, const LaunchCfg& L, F&& f) {
+__device__ inline void for_each_group(uint64_t first, uint64_t end, const LaunchCfg& L, F&& f) {
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
   const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
   const uint32_t lane = threadIdx.x & 63u;
   TileSupply sup = TileSupply::make(wave, nwaves, 0, end - first, 64, L.tiles);
   while (sup.next < sup.end) {
-    if (sup.next + lane < sup.end) f(first + sup.next + lane);
+    f(first + sup.next + lane, sup.next + lane < sup.end);
     sup.more();
   }
+}
+
+// The same for the items alone: f returns to skip the rest of an item.
+template <class F>
+__device__ inline void for_each_item(uint64_t first, uint64_t end, const LaunchCfg& L, F&& f) {
+  for_each_group(first, end, L, [&](uint64_t i, bool has) {
+    if (has) f(i);
+  });
 }
 
 // Edge sampling with the length distribution; returns the edge index and
@@ -85,20 +111,6 @@ __device__ inline EdgeGeo edge_geo(const SceneDev& S, const EdgeDev& e) {
 }
 
 __device__ inline F3 nan0(F3 v) { return finite3(v) ? v : F3{0.0f, 0.0f, 0.0f}; }
-
-// Radiance along a camera boundary ray: EvalRadianceEmitted + bounces with
-// throughput = sensor importance (GenerateBoundaryRays), all detached.
-__device__ F3 boundary_radiance(const SceneDev& S, TraceCtx& tc, const Its& its, F3 raydir, float sensor_val,
-                                uint32_t seed, uint32_t domain, uint64_t index, int B) {
-  F3 beta{sensor_val, sensor_val, sensor_val};
-  F3 rad{0.0f, 0.0f, 0.0f};
-  if (its.emitter >= 0) {
-    F3 e = beta * emitted(S, its.emitter, its.ng, -raydir);
-    if (finite3(e)) rad = rad + e;
-  }
-  path_bounces<false, false>(S, tc, its, beta, raydir, seed, domain, index, 1u, B, rad, nullptr, nullptr);
-  return rad;
-}
 
 // BSDF::Eval with the shading-normal correction (BSDF.cpp:172-195).
 __device__ inline F3 bsdf_eval_corrected(const SceneDev& S, const Its& s, F3 wo, F3 wi) {
@@ -303,7 +315,8 @@ struct BoundaryParams {
 // per wave and consecutive slots for the surviving lanes.  Chunks are large
 // (4M samples, one chunk for a 512^2 x 16 request): every chunk ends in two
 // kernel tails, and at 1M samples per chunk those cost more than the
-// compaction saved.  Survivors of the 512^2 metric scene: 10 % of the
+// compaction saved (kBndChunk; less where that much scratch is not to be had).
+// Survivors of the 512^2 metric scene: 10 % of the
 // primary, 0.8 % of the direct and 13 % of the indirect samples.
 // ---------------------------------------------------------------------------
 struct BndQueue {
@@ -312,7 +325,6 @@ struct BndQueue {
   uint32_t cap;
 };
 constexpr int kBndWords = 20;
-constexpr uint64_t kBndChunk = 1ull << 22;  // 335 MB of queue at most
 
 // Slot of the calling lane in the queue when `keep`, else -1.  Every active
 // lane of the wave calls it at the same point.
@@ -351,116 +363,245 @@ struct QReader {
 };
 
 // ---------------------------------------------------------------------------
-// Primary edges (BoundaryPrimary.cpp:36-181)
+// The camera-side terms: primary edges and the pixel boundary.
+//
+// A select kernel per term finds the samples that count and their first hits;
+// one bounce kernel runs the radiance paths of both (render_bounces: a lane
+// whose path has ended takes the next survivor); one scatter kernel weighs and
+// scatters.  A path per lane in one loop over the samples, as before, waits for
+// the longest of 64 paths and carries the samples that hit nothing.
 // ---------------------------------------------------------------------------
-// select: edge point, the ray away from the camera, its projection onto the
-// sensor, the edge point's visibility from the camera and baseVal.
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBndWaves))) k_bnd_primary_select(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L,
-                                                               EdgeSet E, uint64_t first, uint64_t end, BndQueue Q) {
-  __shared__ uint32_t lds_stack[kTraceLdsWords * kBlock];
-  TraceCtx tc = make_trace_ctx_b(lds_stack, L);
-  const F3 eye = cam_eye(C);
-  // no silhouette or boundary edge seen from this camera: no samples
-  if ((E.dyn ? E.dyn->n : E.n) <= 0) return;
-  for_each_item(first, end, L, [&](uint64_t i) {
-    bool keep = false;
-    Hit h;
-    SensorSample sd;
-    F3 p, rd, n;
-    float pdf, bv, rb;
-    int32_t ei;
-    do {
-      Rnd4 rnd = rng4(P.seed, kRngPrimaryEdge, i, 0u);
-      ei = sample_edge(E, rnd.a, &pdf);
-      const EdgeDev ed = E.e[ei];
-      EdgeGeo g = edge_geo(S, ed);
-      rb = rnd.b;
-      p = g.p0 + rnd.b * g.e1;
-      F3 edge = normalize(g.e1);
-      F3 edge2 = normalize(g.p2 - g.p0);
-      F3 dir = normalize(p - eye);
-      h = trace_ray<false>(S, tc, p, dir, kShadowEpsilon, 1e32f);
-      if (h.tri < 0) break;
-      F3 hitP = p + h.t * dir;
-      sd = sensor_sample(C, hitP);
-      if (!sd.valid) break;
-      rd = camera_dir(C, sd.qx * (float)C.width, sd.qy * (float)C.height);
-      float tmax = length(p - eye) - kShadowEpsilon;
-      if (trace_ray<true>(S, tc, eye, rd, kShadowEpsilon, tmax).tri >= 0) break;
-      Its its = post_intersect(S, h.tri, h.u, h.v);
-      bv = base_val_camera(its.p, its.ng, rd, p, eye, edge, edge2, &n, false);
-      // K = rad * bv / pdf vanishes or is not finite for every radiance
-      keep = bv != 0.0f && isfinite(bv);
-    } while (false);
-    const int64_t s = wave_append(keep, Q.count);
-    if (s >= 0) {
-      QWriter w{Q, (uint32_t)s};
-      w.u64(i); w.i(h.tri); w.f(h.u); w.f(h.v); w.f3(rd); w.f(sd.value); w.i(sd.pixel);
-      w.f(bv); w.f(pdf); w.f3(n); w.i(ei); w.f(rb); w.f3(p);
-    }
-  });
+// Words of a survivor: random index 0-1, hit 2-4, camera ray 5-7 (replaced by
+// the radiance along it), sensor value 8, pixel 9, baseVal 10, pdf 11, edge
+// normal 12-14, point 15-17, and for an edge its index 18 and the position on
+// it 19.
+constexpr int kQHit = 2, kQRad = 5, kQValue = 8, kQPixel = 9;
+
+// Survivors as a source of the bounce pass; paths are queue slots.
+template <uint32_t kRng>
+struct QueuePaths {
+  BndQueue q;
+  uint64_t base;
+  static constexpr uint32_t kDomain = kRng;
+  __device__ float word(int k, uint64_t s) const { return __uint_as_float(q.w[(size_t)k * q.cap + s]); }
+  __device__ bool open(uint64_t i, uint64_t end, uint32_t lane) {
+    base = i;
+    return i + lane < end;
+  }
+  __device__ uint64_t path(uint32_t off) const { return base + off; }
+  __device__ uint64_t rng_index(uint64_t s) const {
+    return (uint64_t)q.w[s] | ((uint64_t)q.w[(size_t)q.cap + s] << 32);
+  }
+  __device__ void first_hit(PathLane& L) const {
+    L.tri = (int32_t)q.w[(size_t)kQHit * q.cap + L.path];
+    L.u = word(kQHit + 1, L.path);
+    L.v = word(kQHit + 2, L.path);
+  }
+  // throughput = sensor importance (GenerateBoundaryRays)
+  __device__ void first_vertex(const SceneDev&, const Its&, PathLane& L) const {
+    L.raydir = F3{word(kQRad, L.path), word(kQRad + 1, L.path), word(kQRad + 2, L.path)};
+    const float value = word(kQValue, L.path);
+    L.beta = F3{value, value, value};
+  }
+};
+
+// bounces: the radiance along each survivor's camera ray, all detached.
+template <uint32_t kRng>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBounceWaves)))
+k_bnd_bounces(SceneDev S, BoundaryParams P, LaunchCfg L, BndQueue Q) {
+  __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
+  TraceCtx tc = make_trace_ctx_bw(lds_stack, L);
+  const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
+  const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+  TileSupply sup = TileSupply::make(wave, nwaves, 0, *Q.count, 64, L.tiles ? L.tiles + kTileSet : nullptr);
+  render_bounces<false>(S, QueuePaths<kRng>{Q, 0}, P.seed, P.max_bounces, tc, sup, CkptDev{},
+                        [&](uint64_t s, F3 c) {
+                          uint32_t* w = Q.w + (size_t)kQRad * Q.cap + s;
+                          w[0] = __float_as_uint(c.x);
+                          w[(size_t)Q.cap] = __float_as_uint(c.y);
+                          w[2 * (size_t)Q.cap] = __float_as_uint(c.z);
+                        });
 }
 
-// eval: the radiance seen through the sensor point and the scatter.
-// kTangent: the derivative image along tpos goes to dimg instead.
-template <bool kTangent>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBndWaves))) k_bnd_primary_eval(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L,
-                                                             EdgeSet E, BndQueue Q, const float* dLdI, float* dpos,
-                                                             const float* tpos, float* dimg) {
-  __shared__ uint32_t lds_stack[kTraceLdsWords * kBlock];
-  TraceCtx tc = make_trace_ctx_b(lds_stack, L);
+// Vertex gradients of a wave on their way to memory: every lane puts up to kN
+// of them down in LDS, and the wave then adds them with four lanes to a vertex
+// (three components and one idle), so that the components of a vertex go out
+// as one request to one line instead of one each.
+template <int kN>
+struct WaveGrads {
+  float4* e;  // [kN][64]: the gradient, and the vertex's bits (~0: none)
+  int k;
+  __device__ bool has_vn() const { return false; }
+  __device__ void open() {
+    const uint32_t lane = threadIdx.x & 63u;
+    k = 0;
+#pragma unroll
+    for (int j = 0; j < kN; ++j) e[j * 64 + lane].w = __uint_as_float(~0u);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+  __device__ void pos(uint32_t v, F3 g) {
+    e[(k++) * 64 + (threadIdx.x & 63u)] = make_float4(g.x, g.y, g.z, __uint_as_float(v));
+  }
+  // Sums the entries of the lanes whose hit is the same triangle into those of
+  // the first of them; all lanes of the wave.
+  __device__ void merge(int32_t tri, bool live) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t first = lane;
+    for (uint64_t todo = __builtin_amdgcn_ballot_w64(live); todo != 0ull;) {
+      const int l = __ffsll((unsigned long long)todo) - 1;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(live && tri == __builtin_amdgcn_readlane(tri, l));
+      if ((m >> lane) & 1ull) first = (uint32_t)l;
+      todo &= ~m;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (live && first != lane) {
+      for (int j = 0; j < k; ++j) {
+        const float4 g = e[j * 64 + lane];
+        float* d = reinterpret_cast<float*>(e + j * 64 + first);
+        if (__float_as_uint(d[3]) != __float_as_uint(g.w)) continue;
+        atomicAdd(&d[0], g.x);
+        atomicAdd(&d[1], g.y);
+        atomicAdd(&d[2], g.z);
+        e[j * 64 + lane].w = __uint_as_float(~0u);
+      }
+    }
+  }
+  // all lanes of the wave
+  __device__ void flush(float* dpos) {
+    const uint32_t lane = threadIdx.x & 63u, c = lane & 3u;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+    for (int j = 0; j < kN * 64; j += 16) {
+      const float* p = reinterpret_cast<const float*>(e + j + (lane >> 2));
+      const uint32_t v = __float_as_uint(p[3]);
+      const float g = p[c];
+      if (v != ~0u && c < 3u && g != 0.0f) atomicAdd(&dpos[3 * (size_t)v + c], g);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+};
+
+// scatter: weight and vertex gradients of each survivor; kTangent: the
+// derivative image along tpos goes to dimg instead.  kEdge: a primary edge,
+// whose end points move too.
+template <bool kEdge, bool kTangent>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBndWaves)))
+k_bnd_scatter(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L, EdgeSet E, BndQueue Q, const float* dLdI,
+              float* dpos, const float* tpos, float* dimg) {
   const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
   const F3 eye = cam_eye(C);
   const uint32_t n_q = *Q.count;
-  const uint32_t stride = (uint32_t)L.grid * kBlock;
-  for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < n_q; s += stride) {
-    QReader r{Q, s};
-    const uint64_t i = r.u64();
-    const int32_t tri = r.i();
-    const float u = r.f(), v = r.f();
-    const F3 rd = r.f3();
-    const float value = r.f();
-    const int32_t pixel = r.i();
-    const float bv = r.f(), pdf = r.f();
-    const F3 n = r.f3();
-    const int32_t ei = r.i();
-    const float rb = r.f();
-    const F3 p = r.f3();
-    Its its = post_intersect(S, tri, u, v);
-    F3 rad = boundary_radiance(S, tc, its, rd, value, P.seed, kRngPrimaryEdge, i, P.max_bounces);
-    F3 K = rad * bv / pdf;
-    if (!(length(K) > 0.0f) || !finite3(K)) continue;
-    const EdgeDev ed = E.e[ei];
-    if constexpr (kTangent) {
-      TangentSink sk{tpos, nullptr, nullptr, 0.0f};
-      scatter_xdn(S, tri, eye, p, n, 1.0f, &ed, rb, ed.f0, -1, 0.0f, 0.0f, sk);
-      add_deriv(dimg, WH, pixel, K * (sk.acc / (float)P.spp));
-    } else {
-      float w = dot(dLdI_at(dLdI, WH, pixel), K) / (float)P.spp;
-      if (w == 0.0f) continue;
-      GradSink sk{dpos, nullptr, nullptr, nullptr};
-      scatter_xdn(S, tri, eye, p, n, w, &ed, rb, ed.f0, -1, 0.0f, 0.0f, sk);
+  const uint32_t stride = (uint32_t)L.grid * kBlock, lane = threadIdx.x & 63u;
+  constexpr int kN = kEdge ? 5 : 3;
+  __shared__ float4 lds[kTangent ? 1 : kN * kBlock];
+  WaveGrads<kN> sk{lds + (kTangent ? 0 : kN * 64 * (threadIdx.x >> 6)), 0};
+  for (uint32_t s0 = blockIdx.x * kBlock + (threadIdx.x & ~63u); s0 < n_q; s0 += stride) {
+    const uint32_t s = s0 + lane;
+    bool live = s < n_q;
+    int32_t pixel = 0;
+    F3 K{0.0f, 0.0f, 0.0f}, n = K, p = K;
+    float w = 1.0f;
+    QReader r{Q, s, kQRad};
+    if (live) {
+      const F3 rad = r.f3();
+      r.k = kQPixel;
+      pixel = r.i();
+      const float bv = r.f(), pdf = r.f();
+      K = rad * bv / pdf;
+      live = finite3(K) && (!kEdge || length(K) > 0.0f);
+      if (!kTangent && live) {
+        w = dot(dLdI_at(dLdI, WH, pixel), K) / (float)P.spp;
+        live = w != 0.0f;
+      }
+    }
+    if (!kTangent) sk.open();
+    int32_t tri = -1;
+    if (live) {
+      n = r.f3();
+      p = r.f3();
+      tri = (int32_t)Q.w[(size_t)kQHit * Q.cap + s];
+      EdgeDev ed{};
+      float rb = 0.0f;
+      int32_t f0 = -1;
+      if (kEdge) {
+        ed = E.e[r.i()];
+        rb = r.f();
+        f0 = ed.f0;
+      }
+      if constexpr (kTangent) {
+        TangentSink tk{tpos, nullptr, nullptr, 0.0f};
+        scatter_xdn(S, tri, eye, p, n, 1.0f, kEdge ? &ed : nullptr, rb, f0, -1, 0.0f, 0.0f, tk);
+        add_deriv(dimg, WH, pixel, K * (tk.acc / (float)P.spp));
+      } else {
+        scatter_xdn(S, tri, eye, p, n, w, kEdge ? &ed : nullptr, rb, f0, -1, 0.0f, 0.0f, sk);
+      }
+    }
+    if (!kTangent) {
+      if (!kEdge) sk.merge(tri, live);
+      sk.flush(dpos);
     }
   }
 }
 
-// ---------------------------------------------------------------------------
+// Primary edges (BoundaryPrimary.cpp:36-181): edge point, the ray away from
+// the camera, its projection onto the sensor, the edge point's visibility from
+// the camera and baseVal.
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBndWaves)))
+k_bnd_primary_select(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L, EdgeSet E, uint64_t first, uint64_t end,
+                     BndQueue Q) {
+  __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
+  TraceCtx tc = make_trace_ctx_bw(lds_stack, L);
+  const F3 eye = cam_eye(C);
+  // no silhouette or boundary edge seen from this camera: no samples
+  if ((E.dyn ? E.dyn->n : E.n) <= 0) return;
+  for_each_group(first, end, L, [&](uint64_t i, bool has) {
+    const Rnd4 rnd = rng4(P.seed, kRngPrimaryEdge, i, 0u);
+    float pdf;
+    const int32_t ei = sample_edge(E, rnd.a, &pdf);
+    const EdgeGeo g = edge_geo(S, E.e[ei]);
+    const F3 p = g.p0 + rnd.b * g.e1;
+    const F3 dir = normalize(p - eye);
+    const Hit h = trace_wave(S, tc, has, p, dir, 1e32f, false);
+    const SensorSample sd = sensor_sample(C, p + h.t * dir);
+    const bool seen = h.tri >= 0 && sd.valid;
+    const F3 rd = camera_dir(C, sd.qx * (float)C.width, sd.qy * (float)C.height);
+    const float tmax = length(p - eye) - kShadowEpsilon;
+    const bool hidden = trace_wave(S, tc, seen, eye, rd, tmax, true).tri >= 0;
+    bool keep = false;
+    float bv = 0.0f;
+    F3 n{0.0f, 0.0f, 0.0f};
+    if (seen && !hidden) {
+      const Its its = post_intersect(S, h.tri, h.u, h.v);
+      bv = base_val_camera(its.p, its.ng, rd, p, eye, normalize(g.e1), normalize(g.p2 - g.p0), &n, false);
+      // K = rad * bv / pdf vanishes or is not finite for every radiance
+      keep = bv != 0.0f && isfinite(bv);
+    }
+    const int64_t s = wave_append(keep, Q.count);
+    if (s >= 0) {
+      QWriter w{Q, (uint32_t)s};
+      w.u64(i); w.i(h.tri); w.f(h.u); w.f(h.v); w.f3(rd); w.f(sd.value); w.i(sd.pixel);
+      w.f(bv); w.f(pdf); w.f3(n); w.f3(p); w.i(ei); w.f(rnd.b);
+    }
+  });
+}
+
 // Pixel boundary of the box filter (BoundaryPixel.cpp:36-159, Edge.cpp:377-409,
 // Camera.cpp:433-467).  4 antithetic positions per random number.
-// ---------------------------------------------------------------------------
-template <bool kTangent>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBndWaves))) k_boundary_pixel(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L,
-                                                           uint64_t N, const float* dLdI, float* dpos,
-                                                           const float* tpos, float* dimg) {
-  __shared__ uint32_t lds_stack[kTraceLdsWords * kBlock];
-  TraceCtx tc = make_trace_ctx_b(lds_stack, L);
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBndWaves)))
+k_bnd_pixel_select(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L, uint64_t N, PathRange range, BndQueue Q) {
+  __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
+  TraceCtx tc = make_trace_ctx_bw(lds_stack, L);
   const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
   const F3 eye = cam_eye(C);
   const F3 R{C.right[0], C.right[1], C.right[2]}, U{C.up[0], C.up[1], C.up[2]}, D{C.dir[0], C.dir[1], C.dir[2]};
   const float plx = 2.0f * C.ratio * C.tan_half, ply = 2.0f * C.tan_half;
   const F3 vdir = normalize(C.ay * U), hdir = normalize(C.ax * R);
   const uint64_t per_anti = N / 4;
-  for_each_item(0, N, L, [&](uint64_t i) {
+  const uint32_t lane = threadIdx.x & 63u;
+  for_each_group(0, range.slots, L, [&](uint64_t slot, bool) {
+    const PathGroup g = PathGroup::at(C, range, slot - lane);
+    const bool has = g.has(lane);
+    const uint64_t i = has ? g.path(lane) : g.base;
     const uint64_t j = i % per_anti, anti = i / per_anti;
     float rr = rng4(P.seed, kRngPixelEdge, j, 0u).a;
     float rv;
@@ -478,30 +619,28 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
     const uint32_t pix = (uint32_t)(i % WH);
     float rx = (float)(pix % (uint32_t)C.width) + ox, ry = (float)(pix / (uint32_t)C.width) + oy;
     F3 p0 = ((eye + (C.ax * rx + C.bx) * R) + (C.ay * ry + C.by) * U) + D;
-    F3 edge = (side == 0 || side == 2) ? vdir : hdir;
-    F3 edge2 = side == 0 ? hdir : (side == 1 ? -vdir : (side == 2 ? -hdir : vdir));
-    float pdf = (side == 0 || side == 2) ? 0.25f / (ply * (float)C.width) : 0.25f / (plx * (float)C.height);
     F3 dir = normalize(p0 - eye);
-    Hit h = trace_ray<false>(S, tc, p0, dir, kShadowEpsilon, 1e32f);
-    if (h.tri < 0) return;
-    F3 hitP = p0 + h.t * dir;
-    SensorSample sd = sensor_sample(C, hitP);
-    F3 rd = camera_dir(C, sd.qx * (float)C.width, sd.qy * (float)C.height);
-    Its its = post_intersect(S, h.tri, h.u, h.v);
-    F3 n;
-    float bv = base_val_camera(its.p, its.ng, rd, p0, eye, edge, edge2, &n, true);
-    F3 rad = boundary_radiance(S, tc, its, rd, sd.value, P.seed, kRngPixelEdge, j, P.max_bounces);
-    F3 K = rad * bv / pdf;
-    if (!finite3(K)) return;
-    if constexpr (kTangent) {
-      TangentSink sk{tpos, nullptr, nullptr, 0.0f};
-      scatter_xdn(S, h.tri, eye, p0, n, 1.0f, nullptr, 0.0f, -1, -1, 0.0f, 0.0f, sk);
-      add_deriv(dimg, WH, (int32_t)pix, K * (sk.acc / (float)P.spp));
-    } else {
-      float w = dot(dLdI_at(dLdI, WH, (int32_t)pix), K) / (float)P.spp;
-      if (w == 0.0f) return;
-      GradSink sk{dpos, nullptr, nullptr, nullptr};
-      scatter_xdn(S, h.tri, eye, p0, n, w, nullptr, 0.0f, -1, -1, 0.0f, 0.0f, sk);
+    const Hit h = trace_wave(S, tc, has, p0, dir, 1e32f, false);
+    bool keep = false;
+    float bv = 0.0f, pdf = 0.0f, value = 0.0f;
+    F3 n{0.0f, 0.0f, 0.0f}, rd = n;
+    if (h.tri >= 0) {
+      F3 edge = (side == 0 || side == 2) ? vdir : hdir;
+      F3 edge2 = side == 0 ? hdir : (side == 1 ? -vdir : (side == 2 ? -hdir : vdir));
+      pdf = (side == 0 || side == 2) ? 0.25f / (ply * (float)C.width) : 0.25f / (plx * (float)C.height);
+      const SensorSample sd = sensor_sample(C, p0 + h.t * dir);
+      value = sd.value;
+      rd = camera_dir(C, sd.qx * (float)C.width, sd.qy * (float)C.height);
+      const Its its = post_intersect(S, h.tri, h.u, h.v);
+      bv = base_val_camera(its.p, its.ng, rd, p0, eye, edge, edge2, &n, true);
+      // K = rad * bv / pdf vanishes or is not finite for every radiance
+      keep = bv != 0.0f && isfinite(bv);
+    }
+    const int64_t s = wave_append(keep, Q.count);
+    if (s >= 0) {
+      QWriter w{Q, (uint32_t)s};
+      w.u64(j); w.i(h.tri); w.f(h.u); w.f(h.v); w.f3(rd); w.f(value); w.i((int32_t)pix);
+      w.f(bv); w.f(pdf); w.f3(n); w.f3(p0);
     }
   });
 }
@@ -962,10 +1101,10 @@ hipError_t launch_guide_build(const SceneDev& S, const LaunchCfg& L, uint32_t se
   return hipGetLastError();
 }
 
-uint64_t boundary_queue_bytes(int kind, uint64_t n_samples) {
-  if (kind == 1 || n_samples == 0) return 0;
-  const uint64_t nchunk = (n_samples + kBndChunk - 1) / kBndChunk;
-  const uint64_t cap = n_samples < kBndChunk ? n_samples : kBndChunk;
+uint64_t boundary_queue_bytes(uint64_t n_samples, uint64_t chunk) {
+  if (n_samples == 0) return 0;
+  const uint64_t nchunk = (n_samples + chunk - 1) / chunk;
+  const uint64_t cap = n_samples < chunk ? n_samples : chunk;
   return ((uint64_t)kBndWords * cap + nchunk) * sizeof(uint32_t);
 }
 
@@ -973,43 +1112,39 @@ template <bool kTangent>
 static hipError_t launch_boundary_t(int kind, const SceneDev& S, const CameraDev& C, const BoundaryParams& P,
                                     uint64_t N, const LaunchCfg& L, const EdgeSet& prim, const GuideDev& guide,
                                     const float* dLdI, float* dpos, const float* tpos, float* dimg, void* queue,
-                                    hipStream_t st) {
-  if (kind == 1) {
-    const LaunchCfg Lk = fit_grid(k_boundary_pixel<kTangent>, L);
-    if (Lk.tiles) {
-      const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(Lk.tiles), kTileSet, st);
-      if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(k_boundary_pixel<kTangent>, dim3(Lk.grid), dim3(kBlock), 0, st, S, C, P, Lk, N, dLdI, dpos,
-                       tpos, dimg);
-    return hipGetLastError();
-  }
-  // select / eval per chunk of kBndChunk samples over one survivor queue;
+                                    uint64_t chunk, hipStream_t st) {
+  // select / eval per chunk of samples over one survivor queue;
   // the chunks' counters are cleared by a kernel (no memset node when captured)
   if (!queue) return hipErrorInvalidValue;
-  const uint64_t nchunk = (N + kBndChunk - 1) / kBndChunk;
-  const uint32_t cap = (uint32_t)(N < kBndChunk ? N : kBndChunk);
+  const uint64_t nchunk = (N + chunk - 1) / chunk;
+  const uint32_t cap = (uint32_t)(N < chunk ? N : chunk);
   uint32_t* buf = (uint32_t*)queue;
   uint32_t* counts = buf + (size_t)kBndWords * cap;
   hipError_t e = launch_fill_zero((float*)counts, nchunk, st);
   for (uint64_t c = 0; c < nchunk && e == hipSuccess; ++c) {
-    const uint64_t first = c * kBndChunk, end = first + kBndChunk < N ? first + kBndChunk : N;
+    const uint64_t first = c * chunk, end = first + chunk < N ? first + chunk : N;
     const BndQueue Q{counts + c, buf, cap};
+    if (L.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2 * kTileSet, st)) != hipSuccess) break;
     if (kind == 0) {
-      const LaunchCfg Ls = fit_grid(k_bnd_primary_select, L), Le = fit_grid(k_bnd_primary_eval<kTangent>, L);
-      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), kTileSet, st)) != hipSuccess) break;
+      const LaunchCfg Ls = fit_grid(k_bnd_primary_select, L), Lb = fit_grid(k_bnd_bounces<kRngPrimaryEdge>, L);
       hipLaunchKernelGGL(k_bnd_primary_select, dim3(Ls.grid), dim3(kBlock), 0, st, S, C, P, Ls, prim, first, end, Q);
-      hipLaunchKernelGGL(k_bnd_primary_eval<kTangent>, dim3(Le.grid), dim3(kBlock), 0, st, S, C, P, Le, prim, Q,
-                         dLdI, dpos, tpos, dimg);
+      hipLaunchKernelGGL(k_bnd_bounces<kRngPrimaryEdge>, dim3(Lb.grid), dim3(kBlock), 0, st, S, P, Lb, Q);
+      hipLaunchKernelGGL((k_bnd_scatter<true, kTangent>), dim3(L.grid), dim3(kBlock), 0, st, S, C, P, L, prim, Q, dLdI,
+                         dpos, tpos, dimg);
+    } else if (kind == 1) {
+      const LaunchCfg Ls = fit_grid(k_bnd_pixel_select, L), Lb = fit_grid(k_bnd_bounces<kRngPixelEdge>, L);
+      hipLaunchKernelGGL(k_bnd_pixel_select, dim3(Ls.grid), dim3(kBlock), 0, st, S, C, P, Ls, N,
+                         path_range(C, first, end - first), Q);
+      hipLaunchKernelGGL(k_bnd_bounces<kRngPixelEdge>, dim3(Lb.grid), dim3(kBlock), 0, st, S, P, Lb, Q);
+      hipLaunchKernelGGL((k_bnd_scatter<false, kTangent>), dim3(L.grid), dim3(kBlock), 0, st, S, C, P, L, prim, Q, dLdI,
+                         dpos, tpos, dimg);
     } else if (kind == 2) {
       const LaunchCfg Ls = fit_grid(k_bnd_direct_select, L), Le = fit_grid(k_bnd_direct_eval<kTangent>, L);
-      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), kTileSet, st)) != hipSuccess) break;
       hipLaunchKernelGGL(k_bnd_direct_select, dim3(Ls.grid), dim3(kBlock), 0, st, S, C, P, Ls, guide, first, end, Q);
       hipLaunchKernelGGL(k_bnd_direct_eval<kTangent>, dim3(Le.grid), dim3(kBlock), 0, st, S, C, P, Le, Q, dLdI, dpos,
                          tpos, dimg);
     } else {
       const LaunchCfg Ls = fit_grid(k_bnd_indirect_select, L), Le = fit_grid(k_bnd_indirect_eval<kTangent>, L);
-      if (Ls.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(Ls.tiles), kTileSet, st)) != hipSuccess) break;
       hipLaunchKernelGGL(k_bnd_indirect_select, dim3(Ls.grid), dim3(kBlock), 0, st, S, C, P, Ls, first, end, Q);
       hipLaunchKernelGGL(k_bnd_indirect_eval<kTangent>, dim3(Le.grid), dim3(kBlock), 0, st, S, C, P, Le, Q, dLdI,
                          dpos, tpos, dimg);
@@ -1021,13 +1156,14 @@ static hipError_t launch_boundary_t(int kind, const SceneDev& S, const CameraDev
 
 hipError_t launch_boundary(int kind, const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
                            const LaunchCfg& L, const EdgeSet& prim, const GuideDev& guide, const float* dLdI,
-                           float* dpos, const float* tpos, float* dimg, void* queue, hipStream_t st) {
+                           float* dpos, const float* tpos, float* dimg, void* queue,
+                           uint64_t chunk, hipStream_t st) {
   const BoundaryParams P{seed, max_bounces, spp, 0u};
   const uint64_t N = (uint64_t)spp * (uint64_t)C.width * (uint64_t)C.height;
   if (N == 0) return hipSuccess;
   if (dimg)
-    return launch_boundary_t<true>(kind, S, C, P, N, L, prim, guide, nullptr, nullptr, tpos, dimg, queue, st);
-  return launch_boundary_t<false>(kind, S, C, P, N, L, prim, guide, dLdI, dpos, nullptr, nullptr, queue, st);
+    return launch_boundary_t<true>(kind, S, C, P, N, L, prim, guide, nullptr, nullptr, tpos, dimg, queue, chunk, st);
+  return launch_boundary_t<false>(kind, S, C, P, N, L, prim, guide, dLdI, dpos, nullptr, nullptr, queue, chunk, st);
 }
 
 }  // namespace trc

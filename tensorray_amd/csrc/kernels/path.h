@@ -485,7 +485,7 @@ __device__ inline void trace_primary(const SceneDev& S, const CameraDev& C, cons
 // contribution.  Returns true when the path continues from the new vertex
 // x_{b+1} (L.tri, L.u, L.v).
 template <bool kCkpt, class Finish>
-__device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const CkptDev& ck, const Its& its, F3 wo,
+__device__ inline bool bsdf_hit(const SceneDev& S, int max_bounces, const CkptDev& ck, const Its& its, F3 wo,
                                 const Hit& h, F3 ret, PathLane& L, uint32_t& meta, Finish& finish) {
   const F3 zero{0.0f, 0.0f, 0.0f};
   bool ok = h.tri >= 0 && L.pdfb > 0.0f && bsdf_dir_valid(S, its, L.d2);
@@ -524,7 +524,7 @@ __device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const Ck
     ckpt_put_vertex(ck, L.path, (int)L.b(), h.tri, h.u, h.v);
     meta += 1u;
   }
-  if ((int)L.b() >= P.max_bounces) {
+  if ((int)L.b() >= max_bounces) {
     if (kCkpt) ck.meta[L.path] = meta;
     finish(L.path, L.contrib);
     L.set_stage(kStageIdle);
@@ -533,17 +533,54 @@ __device__ inline bool bsdf_hit(const SceneDev& S, const PathParams& P, const Ck
   return true;
 }
 
+// The camera paths of the interior integrator as a source of the bounce pass:
+// slots count the launch's order of paths R, first hits lie in `paths`.
+struct CameraPaths {
+  const CameraDev& C;
+  const PathRange& R;
+  const float* paths;
+  uint64_t paths_first;
+  PathGroup group;
+  static constexpr uint32_t kDomain = kRngInterior;
+  // takes the group of slots i .. i + 63: whether the calling lane's survives
+  __device__ bool open(uint64_t i, uint64_t, uint32_t lane) {
+    group = PathGroup::at(C, R, i);
+    return group.has(lane) && __float_as_uint(paths[3 * (group.path(lane) - paths_first)]) != 0u;
+  }
+  // path of the group's offset
+  __device__ uint64_t path(uint32_t off) const { return group.path(off); }
+  __device__ uint64_t rng_index(uint64_t path) const { return path; }
+  __device__ void first_hit(PathLane& L) const {
+    const float* w = paths + 3 * (L.path - paths_first);
+    L.tri = (int32_t)(__float_as_uint(w[0]) - 1u);
+    L.u = w[1];
+    L.v = w[2];
+  }
+  // direction to and throughput at the first vertex (Integrator.cpp:55-73)
+  __device__ void first_vertex(const SceneDev& S, const Its& its, PathLane& L) const {
+    const F3 eye{C.eye[0], C.eye[1], C.eye[2]};
+    const F3 cdir{C.dir[0], C.dir[1], C.dir[2]};
+    F3 cd = its.p - eye;
+    float dist;
+    cd = over_sqrt(cd, len2(cd), &dist);
+    L.raydir = cd;
+    float cosy = dot(cd, cdir);
+    float cosx = dot(-cd, its.ng);
+    float G = fabsf(cosx) / (cosy * cosy * cosy * (dist * dist));
+    const float beta0 = ratio_self(G) * ratio_self(S.shade[its.tri].area);
+    L.beta = F3{beta0, beta0, beta0};
+  }
+};
+
 // The bounce pass: the wave renders the surviving paths of its tile supply,
-// which counts slots of the launch's order of paths R.  A bounce is
-// two ray queries, the shadow ray of next-event estimation and the
-// BSDF-sampled ray, traced as one chained query and shaded together.
-template <bool kCkpt, class Finish>
-__device__ void render_bounces(const SceneDev& S, const CameraDev& C, const PathParams& P, TraceCtx& tc,
-                               TileSupply& sup, const PathRange& R, const CkptDev& ck, const float* paths,
-                               uint64_t paths_first, Finish finish) {
+// which counts slots of the source (camera paths, or the survivors of a
+// boundary term's selection).  A bounce is two ray queries, the shadow ray of
+// next-event estimation and the BSDF-sampled ray, traced as one chained query
+// and shaded together.
+template <bool kCkpt, class Source, class Finish>
+__device__ void render_bounces(const SceneDev& S, Source src, uint32_t seed, int max_bounces, TraceCtx& tc,
+                               TileSupply& sup, const CkptDev& ck, Finish finish) {
   const F3 zero{0.0f, 0.0f, 0.0f};
-  const F3 eye{C.eye[0], C.eye[1], C.eye[2]};
-  const F3 cdir{C.dir[0], C.dir[1], C.dir[2]};
   const uint32_t lane = threadIdx.x & 63u;
   PathLane L;
   L.sb = kStageIdle;
@@ -551,7 +588,6 @@ __device__ void render_bounces(const SceneDev& S, const CameraDev& C, const Path
   uint32_t meta = 0u;  // checkpoint meta word of the current path
   // the current group's surviving paths, not yet handed out from `pool_next`
   // on: lane r holds the offset of the r-th
-  PathGroup group{};
   uint32_t pool = 0u, pool_next = 0u, pool_n = 0u;
   for (;;) {
     // ---- one chained query per lane ----
@@ -586,16 +622,15 @@ __device__ void render_bounces(const SceneDev& S, const CameraDev& C, const Path
       val = val * mis;
       F3 ret = zero;
       ret = ret + val;
-      setup = bsdf_hit<kCkpt>(S, P, ck, its, wo, h, ret, L, meta, finish);
+      setup = bsdf_hit<kCkpt>(S, max_bounces, ck, its, wo, h, ret, L, meta, finish);
     }
     // ---- regenerate: idle lanes take the next surviving paths ----
     const uint64_t idle_mask = __builtin_amdgcn_ballot_w64(L.stage() == kStageIdle);
     if (idle_mask != 0ull) {
       while (pool_next == pool_n) {
         if (sup.next >= sup.end && !sup.more()) break;
-        group = PathGroup::at(C, R, sup.next);
+        const bool live = src.open(sup.next, sup.end, lane);
         sup.next += 64u;
-        const bool live = group.has(lane) && __float_as_uint(paths[3 * (group.path(lane) - paths_first)]) != 0u;
         const uint64_t m = __builtin_amdgcn_ballot_w64(live);
         // lane r of the list: the r-th live lane (dead lanes write behind it)
         const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -610,11 +645,8 @@ __device__ void render_bounces(const SceneDev& S, const CameraDev& C, const Path
       const uint32_t n_idle = (uint32_t)__popcll(idle_mask);
       pool_next = pool_next + n_idle < pool_n ? pool_next + n_idle : pool_n;
       if (take) {
-        L.path = group.path(off);
-        const float* w = paths + 3 * (L.path - paths_first);
-        L.tri = (int32_t)(__float_as_uint(w[0]) - 1u);
-        L.u = w[1];
-        L.v = w[2];
+        L.path = src.path(off);
+        src.first_hit(L);
         L.sb = kStageBounce;  // b = 0
         meta = 1u;
         setup = true;
@@ -627,19 +659,7 @@ __device__ void render_bounces(const SceneDev& S, const CameraDev& C, const Path
       // frame would be live through the hand-out.
       const Its its = post_intersect(S, L.tri, L.u, L.v);
       if (L.b() == 0u) {
-        // the first vertex (Integrator.cpp:55-73)
-        float beta0;
-        {
-          F3 cd = its.p - eye;
-          float dist;
-          cd = over_sqrt(cd, len2(cd), &dist);
-          L.raydir = cd;
-          float cosy = dot(cd, cdir);
-          float cosx = dot(-cd, its.ng);
-          float G = fabsf(cosx) / (cosy * cosy * cosy * (dist * dist));
-          beta0 = ratio_self(G) * ratio_self(S.shade[its.tri].area);
-        }
-        L.beta = F3{beta0, beta0, beta0};
+        src.first_vertex(S, its, L);
         L.contrib = zero;
         if (its.emitter >= 0) {
           F3 Le = emitted(S, its.emitter, its.ng, -L.raydir);
@@ -647,7 +667,7 @@ __device__ void render_bounces(const SceneDev& S, const CameraDev& C, const Path
           if (finite3(e0)) L.contrib = L.contrib + e0;
         }
       }
-      if (P.max_bounces <= 0) {
+      if (max_bounces <= 0) {
         // no bounce: the path ends at its first vertex, and the lane takes
         // another one in the next iteration
         if (kCkpt) ck.meta[L.path] = meta;
@@ -659,11 +679,12 @@ __device__ void render_bounces(const SceneDev& S, const CameraDev& C, const Path
       // ---- bounce b at `its`: light sample, shadow ray and BSDF direction ----
       // (Integrator.cpp:196-213 and 232-245; the draws of the reference's
       // loop in its order: light sample 1 + 2b, BSDF sample 2 + 2b)
-      const Rnd4 rl = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b());
+      const uint64_t index = src.rng_index(L.path);
+      const Rnd4 rl = rng4(seed, Source::kDomain, index, 1u + 2u * L.b());
       const NeeGeo g2 = nee_geo(S, its, rl.a, rl.b);
       L.li = g2.ls.index;
       L.ld2 = g2.d2;
-      const Rnd4 rb = rng4(P.seed, kRngInterior, L.path, 1u + 2u * L.b() + 1u);
+      const Rnd4 rb = rng4(seed, Source::kDomain, index, 1u + 2u * L.b() + 1u);
       L.d2 = bsdf_sample(S, its, -L.raydir, rb.a, rb.b, &L.pdfb);
       L.sb = (L.sb & ~15u) | kStageBounce | (L.pdfb > 0.0f ? 4u : 0u) | (g2.ray ? 8u : 0u);
       L.o = its.p;

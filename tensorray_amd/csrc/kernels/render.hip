@@ -84,7 +84,7 @@ k_bounces(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, uint3
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
   const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
   TileSupply sup = TileSupply::make(wave, nwaves, 0, R.slots, tile, L.tiles ? L.tiles + kTileSet : nullptr);
-  render_bounces<kCkpt>(S, C, P, tc, sup, R, ck, paths, paths_first,
+  render_bounces<kCkpt>(S, CameraPaths{C, R, paths, paths_first}, P.seed, P.max_bounces, tc, sup, ck,
                         [&](uint64_t p, F3 c) {
                           const uint64_t q = p - paths_first;
                           paths[3 * q] = c.x;
@@ -391,7 +391,7 @@ k_batch_bounces(const JobDev* __restrict__ jobs, int njobs, uint64_t ntiles, uin
     float* paths = jobs[j].paths;
     // the wave's tiles of this job, rendered without draining between them
     TileSupply sup = TileSupply::make(t, nwaves, t0, slots, tile, L.tiles ? L.tiles + kTileSet : nullptr);
-    render_bounces<true>(S, C, P, tc, sup, R, ck, paths, 0, [&](uint64_t p, F3 c) {
+    render_bounces<true>(S, CameraPaths{C, R, paths, 0}, P.seed, P.max_bounces, tc, sup, ck, [&](uint64_t p, F3 c) {
       paths[3 * p] = c.x;
       paths[3 * p + 1] = c.y;
       paths[3 * p + 2] = c.z;

@@ -102,7 +102,8 @@ struct trc_scene {
     int32_t spp = 0, n = 0;
     float eps = 0.0f;
   } guide_key;
-  // survivor queue of the primary / direct / indirect boundary kernels
+  // survivor queue of the primary / direct / indirect boundary kernels (the
+  // pixel boundary's is allocated on its stream)
   DevBuf bq_buf;
   // adjoint of the vertex normals [V][3] (kept zero between calls), present
   // when a differentiable mesh is smooth-shaded
@@ -301,16 +302,18 @@ constexpr int kSumChunk = 1024;
 // Builds the guide on `st`; g.enabled is ignored.
 hipError_t launch_guide_build(const SceneDev& S, const LaunchCfg& L, uint32_t seed, const GuideDev& g,
                               hipStream_t st);
-// Bytes of the survivor queue launch_boundary needs for `n_samples` samples
-// of `kind` (0 for the pixel boundary, which runs in one pass).
-uint64_t boundary_queue_bytes(int kind, uint64_t n_samples);
+// Bytes of the survivor queue launch_boundary needs for `n_samples` samples in
+// chunks of `chunk`.
+constexpr uint64_t kBndChunk = 1ull << 22;  // 335 MB of queue at most
+uint64_t boundary_queue_bytes(uint64_t n_samples, uint64_t chunk);
 // kind: 0 primary edges, 1 pixel boundary, 2 secondary direct, 3 secondary
-// indirect; queue: boundary_queue_bytes(kind, spp * W * H) bytes of scratch.
+// indirect; queue: boundary_queue_bytes(spp * W * H, chunk) bytes of scratch.
 // Gradient mode (dimg null): dpos += d/dV of <dLdI, boundary term>.
 // Tangent mode: dimg [3][W*H] += derivative image along tpos [V][3].
 hipError_t launch_boundary(int kind, const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
                            const LaunchCfg& L, const EdgeSet& prim, const GuideDev& guide, const float* dLdI,
-                           float* dpos, const float* tpos, float* dimg, void* queue, hipStream_t st);
+                           float* dpos, const float* tpos, float* dimg, void* queue, uint64_t chunk,
+                           hipStream_t st);
 // Interior derivative image: dimg [3][W*H] += d film / d theta along tpos
 // [V][3] and tmat [M][8] (or null); tvn [V][3] scratch for the vertex-normal
 // tangents when a differentiable mesh is smooth-shaded, else null.
