@@ -919,7 +919,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
     if constexpr (!kTangent) {
       w = w / (float)P.spp;
       if (w == 0.0f || !isfinite(w)) continue;
-      GradSink sk{dpos, nullptr, nullptr, nullptr};
+      GradSink sk{dpos, nullptr, nullptr, nullptr, nullptr};
       scatter_xdn(S, tri0, its.p, p, n, w, &ed, t, ed.f0, tri, hu, hv, sk);
     }
   }
@@ -1070,7 +1070,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
     if constexpr (!kTangent) {
       w = w / (float)P.spp;
       if (w == 0.0f || !isfinite(w)) continue;
-      GradSink sk{dpos, nullptr, nullptr, nullptr};
+      GradSink sk{dpos, nullptr, nullptr, nullptr, nullptr};
       scatter_xdn(S, tri_e, its.p, p, n, w, &ed, t, ed.f0, tri_s, us, vs, sk);
     }
   }

@@ -211,6 +211,7 @@ k_render_adj_ckpt(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, uint64_t f
                   const float* dLdI, float* dpos, float* dmat, float* adj_vn, float* dtex, GradCopies gc,
                   uint32_t* chunk_ctr) {
   if (gc.base) dpos = gc.base + (size_t)(blockIdx.x % gc.copies) * gc.n3;
+  __shared__ __align__(16) float stage[(kBlock / 64) * kSinkStage];
   __shared__ float mat_grad[kMaxMatGrad * kMatGradStride];
   for (int i = threadIdx.x; i < kMaxMatGrad * kMatGradStride; i += kBlock) mat_grad[i] = 0.0f;
   const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
@@ -224,7 +225,7 @@ k_render_adj_ckpt(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, uint64_t f
         CkptSrc src{&ck, p, ck.meta[p]};
         PathRec R;
         path_forward<true>(S, C, P, p, src, &R);
-        GradSink sk{dpos, mat_grad, adj_vn, dtex};
+        GradSink sk{dpos, mat_grad, adj_vn, dtex, &stage[(threadIdx.x >> 6) * kSinkStage]};
         path_backward(S, C, P, R, g, sk);
       });
   if (dmat) {
@@ -413,6 +414,7 @@ __device__ inline uint32_t adj_bucket(const CkptDev& ck, const float* dLdI, uint
 
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) k_render_batch_adj(const JobDev* __restrict__ jobs, int njobs, uint64_t ntiles,
                                                              uint32_t tile, LaunchCfg L) {
+  __shared__ __align__(16) float stage[(kBlock / 64) * kSinkStage];
   __shared__ float mat_lds[(kBlock / 64) * kMaxMatGrad * kMatGradStride];
   __shared__ uint16_t ord_lds[(kBlock / 64) * kAdjChunk];
   __shared__ uint32_t cnt_lds[(kBlock / 64) * 2 * kLenBuckets];
@@ -483,7 +485,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAd
         CkptSrc src{&ck, p, ck.meta[p]};
         PathRec R;
         path_forward<true>(S, C, P, p, src, &R);
-        GradSink sk{dpos, mat_grad, vn, dtex};
+        GradSink sk{dpos, mat_grad, vn, dtex, &stage[(threadIdx.x >> 6) * kSinkStage]};
         path_backward(S, C, P, R, g, sk);
       }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
