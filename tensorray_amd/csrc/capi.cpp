@@ -1418,14 +1418,14 @@ static void boundary_call(trc_scene* s, const trc_camera* cam, const trc_options
   LaunchCfg L = make_cfg(s->ctx, s, st, N);
   if (kind == 1) {
     // of the call alone: pixel terms of one scene may run on several streams
-    WindowScratch q(kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes((uint64_t)N, chunk) + 4; });
+    WindowScratch q(kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes(kind, (uint64_t)N, chunk) + 4; });
     hip_check(!q.ptr ? hipErrorOutOfMemory
                      : launch_boundary(kind, s->dev, C, opt->seed, opt->max_bounces, spp, L, prim, guide, dLdI, dpos,
                                        tpos, dimg, q.ptr, q.window, st),
               "k_boundary");
     return;
   }
-  const size_t qb = (size_t)boundary_queue_bytes((uint64_t)N, kBndChunk);
+  const size_t qb = (size_t)boundary_queue_bytes(kind, (uint64_t)N, kBndChunk);
   if (s->bq_buf.bytes < qb) {
     hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
     if (s->bq_buf.ptr) hipFree(s->bq_buf.ptr);

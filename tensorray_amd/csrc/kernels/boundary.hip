@@ -319,26 +319,69 @@ struct BoundaryParams {
 // Survivors of the 512^2 metric scene: 10 % of the
 // primary, 0.8 % of the direct and 13 % of the indirect samples.
 // ---------------------------------------------------------------------------
+// One counter word serves an append every 11.5 ns (16,384 groups of 64 samples:
+// 0.19 ms), so the queue has kTileCtrs segments, each with a counter in a cache
+// line of its own: samples of group g go to segment g % kTileCtrs, which has
+// room for all of its groups.  Readers take the survivors of a segment 64 at a
+// time, as one list of groups over the segments.  (512 x 512 x 4 pixel select
+// 197 us with one counter, 146 us with eight.)
 struct BndQueue {
-  uint32_t* count;  // survivors of this chunk
+  uint32_t* count;  // survivors of this chunk: kTileSet words
   uint32_t* w;      // kBndWords x cap words
-  uint32_t cap;
+  uint32_t cap;     // kTileCtrs segments of cap / kTileCtrs slots
+  __device__ uint32_t groups() const {
+    uint32_t n = 0u;
+#pragma unroll
+    for (int k = 0; k < kTileCtrs; ++k) n += (count[k * kTileCtrStride] + 63u) >> 6;
+    return n;
+  }
+  // first slot of group g, which is less than groups(), and its survivors
+  __device__ uint32_t group(uint32_t g, uint32_t* n) const {
+    uint32_t base = 0u;
+    *n = 0u;
+#pragma unroll
+    for (int k = 0; k < kTileCtrs; ++k) {
+      const uint32_t c = count[k * kTileCtrStride], m = (c + 63u) >> 6;
+      if (g < m) {
+        base = (uint32_t)k * (cap / (uint32_t)kTileCtrs) + g * 64u;
+        *n = c - g * 64u < 64u ? c - g * 64u : 64u;
+        break;
+      }
+      g -= m;
+    }
+    return base;
+  }
 };
 constexpr int kBndWords = 20;
 
-// Slot of the calling lane in the queue when `keep`, else -1.  Every active
-// lane of the wave calls it at the same point.
-__device__ inline int64_t wave_append(bool keep, uint32_t* count) {
+// Slot of the calling lane in the queue when `keep`, else -1; group: the
+// wave's, of 64 samples of the chunk.  Every active lane of the wave calls it
+// at the same point.
+__device__ inline int64_t wave_append(bool keep, const BndQueue& Q, uint64_t group) {
   const uint64_t act = __ballot(1);
   const uint64_t m = __ballot(keep);
   if (m == 0ull) return -1;
   const int lane = (int)(threadIdx.x & 63u);
   const int leader = __ffsll((unsigned long long)act) - 1;
   uint32_t base = 0u;
-  if (lane == leader) base = atomicAdd(count, (uint32_t)__popcll(m));
+  const uint32_t seg = (uint32_t)(group % (uint64_t)kTileCtrs);
+  if (lane == leader) base = atomicAdd(Q.count + seg * (uint32_t)kTileCtrStride, (uint32_t)__popcll(m));
   base = (uint32_t)__shfl((int)base, leader);
   if (!keep) return -1;
-  return (int64_t)base + (int64_t)__popcll(m & ((1ull << lane) - 1ull));
+  return (int64_t)(seg * (Q.cap / (uint32_t)kTileCtrs) + base) + (int64_t)__popcll(m & ((1ull << lane) - 1ull));
+}
+
+// Calls f(s) for the survivors' slots s, a group per wave at a time from the
+// launch's second set of tile counters.
+template <class F>
+__device__ inline void for_each_survivor(const BndQueue& Q, LaunchCfg L, F&& f) {
+  if (L.tiles) L.tiles += kTileSet;
+  const uint32_t lane = threadIdx.x & 63u;
+  for_each_group(0, (uint64_t)Q.groups() * 64u, L, [&](uint64_t i, bool) {
+    uint32_t n;
+    const uint32_t s = Q.group((uint32_t)(i >> 6), &n) + lane;
+    if (lane < n) f(s);
+  });
 }
 
 struct QWriter {
@@ -381,12 +424,13 @@ constexpr int kQHit = 2, kQRad = 5, kQValue = 8, kQPixel = 9;
 template <uint32_t kRng>
 struct QueuePaths {
   BndQueue q;
-  uint64_t base;
+  uint32_t base;
   static constexpr uint32_t kDomain = kRng;
   __device__ float word(int k, uint64_t s) const { return __uint_as_float(q.w[(size_t)k * q.cap + s]); }
-  __device__ bool open(uint64_t i, uint64_t end, uint32_t lane) {
-    base = i;
-    return i + lane < end;
+  __device__ bool open(uint64_t i, uint32_t lane) {
+    uint32_t n;
+    base = q.group((uint32_t)(i >> 6), &n);
+    return lane < n;
   }
   __device__ uint64_t path(uint32_t off) const { return base + off; }
   __device__ uint64_t rng_index(uint64_t s) const {
@@ -413,7 +457,7 @@ k_bnd_bounces(SceneDev S, BoundaryParams P, LaunchCfg L, BndQueue Q) {
   TraceCtx tc = make_trace_ctx_bw(lds_stack, L);
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
   const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-  TileSupply sup = TileSupply::make(wave, nwaves, 0, *Q.count, 64, L.tiles ? L.tiles + kTileSet : nullptr);
+  TileSupply sup = TileSupply::make(wave, nwaves, 0, (uint64_t)Q.groups() * 64u, 64, L.tiles ? L.tiles + kTileSet : nullptr);
   render_bounces<false>(S, QueuePaths<kRng>{Q, 0}, P.seed, P.max_bounces, tc, sup, CkptDev{},
                         [&](uint64_t s, F3 c) {
                           uint32_t* w = Q.w + (size_t)kQRad * Q.cap + s;
@@ -490,14 +534,14 @@ k_bnd_scatter(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L, EdgeSet E,
               float* dpos, const float* tpos, float* dimg) {
   const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
   const F3 eye = cam_eye(C);
-  const uint32_t n_q = *Q.count;
-  const uint32_t stride = (uint32_t)L.grid * kBlock, lane = threadIdx.x & 63u;
+  const uint32_t n_g = Q.groups(), nwaves = (uint32_t)L.grid * (kBlock / 64), lane = threadIdx.x & 63u;
   constexpr int kN = kEdge ? 5 : 3;
   __shared__ float4 lds[kTangent ? 1 : kN * kBlock];
   WaveGrads<kN> sk{lds + (kTangent ? 0 : kN * 64 * (threadIdx.x >> 6)), 0};
-  for (uint32_t s0 = blockIdx.x * kBlock + (threadIdx.x & ~63u); s0 < n_q; s0 += stride) {
-    const uint32_t s = s0 + lane;
-    bool live = s < n_q;
+  for (uint32_t g = (blockIdx.x * kBlock + threadIdx.x) >> 6; g < n_g; g += nwaves) {
+    uint32_t n_live;
+    const uint32_t s = Q.group(g, &n_live) + lane;
+    bool live = lane < n_live;
     int32_t pixel = 0;
     F3 K{0.0f, 0.0f, 0.0f}, n = K, p = K;
     float w = 1.0f;
@@ -576,7 +620,7 @@ k_bnd_primary_select(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L, Edg
       // K = rad * bv / pdf vanishes or is not finite for every radiance
       keep = bv != 0.0f && isfinite(bv);
     }
-    const int64_t s = wave_append(keep, Q.count);
+    const int64_t s = wave_append(keep, Q, (i - first) >> 6);
     if (s >= 0) {
       QWriter w{Q, (uint32_t)s};
       w.u64(i); w.i(h.tri); w.f(h.u); w.f(h.v); w.f3(rd); w.f(sd.value); w.i(sd.pixel);
@@ -636,7 +680,7 @@ k_bnd_pixel_select(SceneDev S, CameraDev C, BoundaryParams P, LaunchCfg L, uint6
       // K = rad * bv / pdf vanishes or is not finite for every radiance
       keep = bv != 0.0f && isfinite(bv);
     }
-    const int64_t s = wave_append(keep, Q.count);
+    const int64_t s = wave_append(keep, Q, slot >> 6);
     if (s >= 0) {
       QWriter w{Q, (uint32_t)s};
       w.u64(j); w.i(h.tri); w.f(h.u); w.f(h.v); w.f3(rd); w.f(value); w.i((int32_t)pix);
@@ -859,7 +903,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
       // every contribution K0 * importance then vanishes or is not finite
       keep = finite3(K0) && (K0.x != 0.0f || K0.y != 0.0f || K0.z != 0.0f);
     } while (false);
-    const int64_t s = wave_append(keep, Q.count);
+    const int64_t s = wave_append(keep, Q, (i - first) >> 6);
     if (s >= 0) {
       QWriter w{Q, (uint32_t)s};
       w.u64(i); w.f3(K0); w.i(h.tri); w.f(h.u); w.f(h.v); w.f3(rdir); w.i(h0.tri); w.f3(p); w.f3(n); w.i(ei);
@@ -878,9 +922,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
   TraceCtx tc = make_trace_ctx_b(lds_stack, L);
   const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
   const EdgeSet& E = S.sec;
-  const uint32_t n_q = *Q.count;
-  const uint32_t stride = (uint32_t)L.grid * kBlock;
-  for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < n_q; s += stride) {
+  for_each_survivor(Q, L, [&](uint32_t s) {
     QReader r{Q, s};
     const uint64_t i = r.u64();
     const F3 K0 = r.f3();
@@ -899,7 +941,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
       TangentSink sk{tpos, nullptr, nullptr, 0.0f};
       scatter_xdn(S, tri0, its.p, p, n, 1.0f, &ed, t, ed.f0, tri, hu, hv, sk);
       ds = sk.acc / (float)P.spp;
-      if (ds == 0.0f || !isfinite(ds)) continue;
+      if (ds == 0.0f || !isfinite(ds)) return;
     }
     // sensor side: EvalImportance for B bounces, throughput 1
     float w = 0.0f;
@@ -918,11 +960,11 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
     }
     if constexpr (!kTangent) {
       w = w / (float)P.spp;
-      if (w == 0.0f || !isfinite(w)) continue;
+      if (w == 0.0f || !isfinite(w)) return;
       GradSink sk{dpos, nullptr, nullptr, nullptr, nullptr};
       scatter_xdn(S, tri0, its.p, p, n, w, &ed, t, ed.f0, tri, hu, hv, sk);
     }
-  }
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -992,7 +1034,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
       // makes every contribution vanish or not finite
       keep = P.max_bounces > 1 && v0 != 0.0f && isfinite(v0);
     } while (false);
-    const int64_t s = wave_append(keep, Q.count);
+    const int64_t s = wave_append(keep, Q, (i - first) >> 6);
     if (s >= 0) {
       QWriter w{Q, (uint32_t)s};
       w.u64(i); w.i(he.tri); w.f(he.u); w.f(he.v); w.i(hs.tri); w.f(hs.u); w.f(hs.v); w.f3(dir); w.f(v0);
@@ -1013,9 +1055,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
   const uint32_t WH = (uint32_t)C.width * (uint32_t)C.height;
   const EdgeSet& E = S.sec;
   const int B = P.max_bounces;
-  const uint32_t n_q = *Q.count;
-  const uint32_t stride = (uint32_t)L.grid * kBlock;
-  for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < n_q; s += stride) {
+  for_each_survivor(Q, L, [&](uint32_t s) {
     QReader r{Q, s};
     const uint64_t i = r.u64();
     const int32_t tri_e = r.i();
@@ -1036,7 +1076,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
       TangentSink sk{tpos, nullptr, nullptr, 0.0f};
       scatter_xdn(S, tri_e, its.p, p, n, 1.0f, &ed, t, ed.f0, tri_s, us, vs, sk);
       ds = sk.acc / (float)P.spp;
-      if (ds == 0.0f || !isfinite(ds)) continue;
+      if (ds == 0.0f || !isfinite(ds)) return;
     }
     // emitter side: cumulative radiance after 1..B-1 bounces
     F3 cum[kMaxBounces];
@@ -1069,11 +1109,11 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kBn
     }
     if constexpr (!kTangent) {
       w = w / (float)P.spp;
-      if (w == 0.0f || !isfinite(w)) continue;
+      if (w == 0.0f || !isfinite(w)) return;
       GradSink sk{dpos, nullptr, nullptr, nullptr, nullptr};
       scatter_xdn(S, tri_e, its.p, p, n, w, &ed, t, ed.f0, tri_s, us, vs, sk);
     }
-  }
+  });
 }
 
 hipError_t launch_guide_build(const SceneDev& S, const LaunchCfg& L, uint32_t seed, const GuideDev& g,
@@ -1101,11 +1141,19 @@ hipError_t launch_guide_build(const SceneDev& S, const LaunchCfg& L, uint32_t se
   return hipGetLastError();
 }
 
-uint64_t boundary_queue_bytes(uint64_t n_samples, uint64_t chunk) {
+// Slots for the survivors of `count` samples: whole groups of 64 in each
+// segment; the pixel boundary's blocks of pixels may leave an eighth empty.
+static uint64_t queue_slots(int kind, uint64_t count) {
+  const uint64_t slots = kind == 1 ? count + count / 8 : count;
+  const uint64_t groups = (slots + 63) / 64;
+  return (groups + kTileCtrs - 1) / kTileCtrs * kTileCtrs * 64;
+}
+
+uint64_t boundary_queue_bytes(int kind, uint64_t n_samples, uint64_t chunk) {
   if (n_samples == 0) return 0;
   const uint64_t nchunk = (n_samples + chunk - 1) / chunk;
-  const uint64_t cap = n_samples < chunk ? n_samples : chunk;
-  return ((uint64_t)kBndWords * cap + nchunk) * sizeof(uint32_t);
+  const uint64_t cap = queue_slots(kind, n_samples < chunk ? n_samples : chunk);
+  return ((uint64_t)kBndWords * cap + nchunk * kTileSet) * sizeof(uint32_t);
 }
 
 template <bool kTangent>
@@ -1117,13 +1165,13 @@ static hipError_t launch_boundary_t(int kind, const SceneDev& S, const CameraDev
   // the chunks' counters are cleared by a kernel (no memset node when captured)
   if (!queue) return hipErrorInvalidValue;
   const uint64_t nchunk = (N + chunk - 1) / chunk;
-  const uint32_t cap = (uint32_t)(N < chunk ? N : chunk);
+  const uint32_t cap = (uint32_t)queue_slots(kind, N < chunk ? N : chunk);
   uint32_t* buf = (uint32_t*)queue;
   uint32_t* counts = buf + (size_t)kBndWords * cap;
-  hipError_t e = launch_fill_zero((float*)counts, nchunk, st);
+  hipError_t e = launch_fill_zero((float*)counts, nchunk * kTileSet, st);
   for (uint64_t c = 0; c < nchunk && e == hipSuccess; ++c) {
     const uint64_t first = c * chunk, end = first + chunk < N ? first + chunk : N;
-    const BndQueue Q{counts + c, buf, cap};
+    const BndQueue Q{counts + c * kTileSet, buf, cap};
     if (L.tiles && (e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2 * kTileSet, st)) != hipSuccess) break;
     if (kind == 0) {
       const LaunchCfg Ls = fit_grid(k_bnd_primary_select, L), Lb = fit_grid(k_bnd_bounces<kRngPrimaryEdge>, L);

@@ -543,7 +543,7 @@ struct CameraPaths {
   PathGroup group;
   static constexpr uint32_t kDomain = kRngInterior;
   // takes the group of slots i .. i + 63: whether the calling lane's survives
-  __device__ bool open(uint64_t i, uint64_t, uint32_t lane) {
+  __device__ bool open(uint64_t i, uint32_t lane) {
     group = PathGroup::at(C, R, i);
     return group.has(lane) && __float_as_uint(paths[3 * (group.path(lane) - paths_first)]) != 0u;
   }
@@ -629,7 +629,7 @@ __device__ void render_bounces(const SceneDev& S, Source src, uint32_t seed, int
     if (idle_mask != 0ull) {
       while (pool_next == pool_n) {
         if (sup.next >= sup.end && !sup.more()) break;
-        const bool live = src.open(sup.next, sup.end, lane);
+        const bool live = src.open(sup.next, lane);
         sup.next += 64u;
         const uint64_t m = __builtin_amdgcn_ballot_w64(live);
         // lane r of the list: the r-th live lane (dead lanes write behind it)

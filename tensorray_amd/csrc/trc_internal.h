@@ -302,12 +302,12 @@ constexpr int kSumChunk = 1024;
 // Builds the guide on `st`; g.enabled is ignored.
 hipError_t launch_guide_build(const SceneDev& S, const LaunchCfg& L, uint32_t seed, const GuideDev& g,
                               hipStream_t st);
-// Bytes of the survivor queue launch_boundary needs for `n_samples` samples in
-// chunks of `chunk`.
-constexpr uint64_t kBndChunk = 1ull << 22;  // 335 MB of queue at most
-uint64_t boundary_queue_bytes(uint64_t n_samples, uint64_t chunk);
+// Bytes of the survivor queue launch_boundary needs for `n_samples` samples of
+// `kind` in chunks of `chunk`.
+constexpr uint64_t kBndChunk = 1ull << 22;  // 335 MB of queue at most (pixel boundary: 377)
+uint64_t boundary_queue_bytes(int kind, uint64_t n_samples, uint64_t chunk);
 // kind: 0 primary edges, 1 pixel boundary, 2 secondary direct, 3 secondary
-// indirect; queue: boundary_queue_bytes(spp * W * H, chunk) bytes of scratch.
+// indirect; queue: boundary_queue_bytes(kind, spp * W * H, chunk) bytes of scratch.
 // Gradient mode (dimg null): dpos += d/dV of <dLdI, boundary term>.
 // Tangent mode: dimg [3][W*H] += derivative image along tpos [V][3].
 hipError_t launch_boundary(int kind, const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
