@@ -69,7 +69,7 @@ def parse():
 def algorithmic_bytes(stats, spp_paths, B, n_light_tris):
     """Algorithmic HBM bytes per path of the forward and adjoint passes.
 
-    Per ray query: 32 B ray + 16 B hit + 128 B per BVH node visited + 48 B
+    Per ray query: 32 B ray + 16 B hit + 64 B per BVH node visited + 48 B
     per triangle tested (averages measured on the same rays and BVH by the
     statistics kernel).  Per bounce: 56 B shading data + NEE light-table
     search 4*ceil(log2 T_L) + 48 B light triangle; film read-modify-write 24 B.
@@ -81,7 +81,7 @@ def algorithmic_bytes(stats, spp_paths, B, n_light_tris):
     """
     paths, queries, nodes, tris = stats
     q_per_path = queries / paths
-    b_query = 32 + 16 + 128 * (nodes / queries) + 48 * (tris / queries)
+    b_query = 32 + 16 + 64 * (nodes / queries) + 48 * (tris / queries)
     bounces = max(0.0, (q_per_path - 1.0) / 2.0)  # 1 primary + (shadow + bsdf) per bounce
     b_shade = 56 * (1 + bounces)
     b_nee = bounces * (4 * math.ceil(math.log2(max(2, n_light_tris))) + 48)
@@ -484,11 +484,12 @@ def main():
     adj_avg = sum(adj_ms) / len(adj_ms)
     ck = a.adjoint == "checkpoint"
     if adj_avg >= fwd_avg:
-        kname, kms = ("k_render_adj_ckpt", adj_avg) if ck else ("k_render_adj", adj_avg)
+        kname, kms = ("k_render_adj_ckpt", adj_avg) if ck else ("k_primary<true> + k_bounces<true> + k_render_adj_ckpt", adj_avg)
         kbytes = (bb["adj_ckpt"] if ck else bb["adj"]) * P
     else:
-        # the forward kernel with (true) or without (false) checkpoint writes
-        kname, kms = f"k_render_paths<{'true' if ck else 'false'}>", fwd_avg
+        # the forward's two kernels with (true) or without (false) checkpoint writes
+        t = "true" if ck else "false"
+        kname, kms = f"k_primary<{t}> + k_bounces<{t}>", fwd_avg
         kbytes = (bb["fwd_ckpt"] if ck else bb["fwd"]) * P
     achieved = kbytes / (kms * 1e-3)
     traffic = None

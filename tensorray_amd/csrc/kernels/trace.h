@@ -317,8 +317,8 @@ __device__ inline void flush_wave(const SceneDev& S, TraceCtx& ctx, const RayPre
 //
 // Per node visit: slab tests of the four children; hit inner children are
 // sorted near to far and pushed, hit leaves are appended to a per-lane queue
-// in LDS.  Leaves are tested later, in one flat loop over (leaf, triangle)
-// pairs, when the wave decides to: at least three quarters of its live lanes
+// in LDS.  Leaves (one triangle each) are tested later, when the wave decides
+// to: at least three quarters of its live lanes
 // have queued leaves, or some lane has no inner node left or a nearly full
 // queue (the threshold was picked by timing 1/4, 1/2 and 3/4).
 // Testing a leaf late only loosens culling (best_t shrinks later); it never
