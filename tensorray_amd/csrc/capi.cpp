@@ -96,15 +96,23 @@ GradCopies make_grad_copies(int n_verts, hipStream_t st) {
   return g;
 }
 
-// Stream-ordered scratch of a pass that runs in windows of paths or samples:
-// bytes(window), for the largest window (halved down to 32k) that can be
-// allocated; null when none can.
+// Scratch of a pass that runs in windows of paths or samples: bytes(window),
+// the stream's own where that is enough for the first window, else allocated on
+// the stream, for the largest window (halved down to 32k) that can be; null
+// when none can.
 struct WindowScratch {
   void* ptr = nullptr;
+  bool kept = false;
   uint64_t window = 0;
   hipStream_t st;
   template <class Bytes>
-  WindowScratch(uint64_t first_window, hipStream_t stream, Bytes&& bytes) : window(first_window), st(stream) {
+  WindowScratch(const LaunchCfg& L, uint64_t first_window, hipStream_t stream, Bytes&& bytes)
+      : window(first_window), st(stream) {
+    kept = L.scratch && bytes(window) <= kStreamScratch;
+    if (kept) {
+      ptr = L.scratch;
+      return;
+    }
     while (hipMallocAsync(&ptr, (size_t)bytes(window), st) != hipSuccess) {
       (void)hipGetLastError();
       ptr = nullptr;
@@ -113,21 +121,21 @@ struct WindowScratch {
     }
   }
   ~WindowScratch() {
-    if (ptr) hipFreeAsync(ptr, st);
+    if (ptr && !kept) hipFreeAsync(ptr, st);
   }
   WindowScratch(const WindowScratch&) = delete;
   WindowScratch& operator=(const WindowScratch&) = delete;
 };
 // that of a pass which traces its own checkpoint
 struct ReplayScratch : WindowScratch {
-  ReplayScratch(uint64_t npaths, int max_bounces, hipStream_t stream)
-      : WindowScratch(replay_window(npaths), stream,
+  ReplayScratch(const LaunchCfg& L, uint64_t npaths, int max_bounces, hipStream_t stream)
+      : WindowScratch(L, replay_window(npaths), stream,
                       [=](uint64_t window) { return replay_bytes(window, max_bounces); }) {}
 };
 
 // Words of a stream's spill buffer: the traversal stacks' spill area, then
 // the launches' tile counters (one set for the forward's camera rays and for
-// the other kernels, one for its bounces).
+// the other kernels, one for its bounces), and for a stream's the scratch.
 constexpr size_t kTileCtrWords = 2 * kTileSet;
 static size_t spill_words(int max_grid) { return (size_t)kSpillDepth * (size_t)max_grid * kBlock; }
 
@@ -144,6 +152,7 @@ LaunchCfg make_cfg(trc_ctx* ctx, const trc_scene* s, hipStream_t st, long long w
   L.cap = kStackLds + kSpillDepth;
   L.cus = ctx->num_cus;
   L.spill = nullptr;
+  L.scratch = nullptr;
   L.tiles = nullptr;
   if (!with_spill) return L;
   // one spill buffer per (context, stream): launches on different streams
@@ -152,11 +161,12 @@ LaunchCfg make_cfg(trc_ctx* ctx, const trc_scene* s, hipStream_t st, long long w
   auto it = ctx->spill.find(st);
   if (it == ctx->spill.end()) {
     uint32_t* p = nullptr;
-    hip_check(hipMalloc(&p, (spill_words(max_grid) + kTileCtrWords) * 4), "hipMalloc(spill)");
+    hip_check(hipMalloc(&p, (spill_words(max_grid) + kTileCtrWords) * 4 + kStreamScratch), "hipMalloc(spill)");
     it = ctx->spill.emplace(st, p).first;
   }
   L.spill = it->second;
   L.tiles = it->second + spill_words(max_grid);
+  L.scratch = L.tiles + kTileCtrWords;
   return L;
 }
 
@@ -1418,7 +1428,7 @@ static void boundary_call(trc_scene* s, const trc_camera* cam, const trc_options
   LaunchCfg L = make_cfg(s->ctx, s, st, N);
   if (kind == 1) {
     // of the call alone: pixel terms of one scene may run on several streams
-    WindowScratch q(kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes(kind, (uint64_t)N, chunk) + 4; });
+    WindowScratch q(L, kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes(kind, (uint64_t)N, chunk) + 4; });
     hip_check(!q.ptr ? hipErrorOutOfMemory
                      : launch_boundary(kind, s->dev, C, opt->seed, opt->max_bounces, spp, L, prim, guide, dLdI, dpos,
                                        tpos, dimg, q.ptr, q.window, st),
@@ -1467,7 +1477,7 @@ trc_status trc_render_deriv(trc_scene* s, const trc_camera* cam, const trc_optio
     float* tvn = nullptr;
     if (s->vn_adj)
       hip_check(hipMallocAsync((void**)&tvn, 3 * (size_t)s->dev.n_verts * sizeof(float), st), "hipMallocAsync(tvn)");
-    ReplayScratch rs((uint64_t)np, opt->max_bounces, st);
+    ReplayScratch rs(L, (uint64_t)np, opt->max_bounces, st);
     const hipError_t e = !rs.ptr ? hipErrorOutOfMemory : launch_render_deriv(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, tpos, tmat, tvn,
                                              dimg, rs.ptr, rs.window, st);
     if (tvn) hipFreeAsync(tvn, st);
@@ -1486,7 +1496,7 @@ trc_status trc_render_adj(trc_scene* s, const trc_camera* cam, const trc_options
     LaunchCfg L = make_cfg(s->ctx, s, (hipStream_t)stream, np);
     GradCopies gc = make_grad_copies(s->dev.n_verts, (hipStream_t)stream);
     hipError_t e = hipErrorOutOfMemory;
-    ReplayScratch rs((uint64_t)np, opt->max_bounces, (hipStream_t)stream);
+    ReplayScratch rs(L, (uint64_t)np, opt->max_bounces, (hipStream_t)stream);
     if (rs.ptr)
       e = launch_render_adj(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, dLdI, dpos, dmat, dtex, s->vn_adj, gc,
                             rs.ptr, rs.window, (hipStream_t)stream);
