@@ -219,7 +219,7 @@ struct Collapser {
   BvhBuildStats& st;
   std::vector<int> depth_of;  // depth of every 4-wide node (root 1)
 
-  // Emits one leaf's triangles, splitting ranges larger than kMaxLeafTris.
+  // Emits one leaf's triangles.
   uint32_t emit_leaf(const BinNode& n) {
     uint32_t first = (uint32_t)tris.size();
     for (uint32_t i = n.first; i < n.first + n.count; ++i) {
