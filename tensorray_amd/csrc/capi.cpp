@@ -139,9 +139,8 @@ struct ReplayScratch : WindowScratch {
 constexpr size_t kTileCtrWords = 2 * kTileSet;
 static size_t spill_words(int max_grid) { return (size_t)kSpillDepth * (size_t)max_grid * kBlock; }
 
-// Launch shape for `work_items` items over scene `s`, with the spill buffer of
-// stream `st` (none when with_spill is false; the caller supplies one).
-LaunchCfg make_cfg(trc_ctx* ctx, const trc_scene* s, hipStream_t st, long long work_items, bool with_spill = true) {
+// Launch shape for `work_items` items over scene `s`, without device memory.
+LaunchCfg make_cfg(const trc_ctx* ctx, const trc_scene* s, long long work_items) {
   LaunchCfg L;
   int max_grid = ctx->num_cus * kBlocksPerCU;
   long long need = (work_items + kBlock - 1) / kBlock;
@@ -154,21 +153,30 @@ LaunchCfg make_cfg(trc_ctx* ctx, const trc_scene* s, hipStream_t st, long long w
   L.spill = nullptr;
   L.scratch = nullptr;
   L.tiles = nullptr;
-  if (!with_spill) return L;
-  // one spill buffer per (context, stream): launches on different streams
-  // never share one (word 0 doubles as the chunk counter of the adjoint)
-  std::lock_guard<std::mutex> lk(ctx->mu);
-  auto it = ctx->spill.find(st);
-  if (it == ctx->spill.end()) {
-    uint32_t* p = nullptr;
-    hip_check(hipMalloc(&p, (spill_words(max_grid) + kTileCtrWords) * 4 + kStreamScratch), "hipMalloc(spill)");
-    it = ctx->spill.emplace(st, p).first;
-  }
-  L.spill = it->second;
-  L.tiles = it->second + spill_words(max_grid);
-  L.scratch = L.tiles + kTileCtrWords;
   return L;
 }
+
+// The launch shape with the memory of stream `st`, for as long as a call
+// queues its kernels there: launches on different streams never share it
+// (word 0 of the spill area doubles as the chunk counter of the adjoint).
+struct StreamCfg : LaunchCfg {
+  std::unique_lock<std::mutex> own;
+  StreamCfg(trc_ctx* ctx, const trc_scene* s, hipStream_t st, long long work_items)
+      : LaunchCfg(make_cfg(ctx, s, work_items)) {
+    const size_t words = spill_words(ctx->num_cus * kBlocksPerCU);
+    trc_ctx::StreamMem* m;
+    {
+      std::lock_guard<std::mutex> lk(ctx->mu);
+      m = &ctx->streams[st];
+    }
+    own = std::unique_lock<std::mutex>(m->queueing);
+    if (!m->spill)
+      hip_check(hipMalloc((void**)&m->spill, (words + kTileCtrWords) * 4 + kStreamScratch), "hipMalloc(spill)");
+    spill = m->spill;
+    tiles = m->spill + words;
+    scratch = tiles + kTileCtrWords;
+  }
+};
 
 template <class T>
 T* upload(trc_scene* s, const std::vector<T>& v, hipStream_t st) {
@@ -443,8 +451,9 @@ trc_status trc_context_destroy(trc_ctx* ctx) {
   if (!ctx) return TRC_ERR_INVALID;
   {
     std::lock_guard<std::mutex> lk(ctx->mu);
-    for (auto& kv : ctx->spill) hipFree(kv.second);
-    ctx->spill.clear();
+    for (auto& kv : ctx->streams)
+      if (kv.second.spill) hipFree(kv.second.spill);
+    ctx->streams.clear();
   }
   for (auto& b : ctx->batch) {
     if (b.done) {
@@ -702,7 +711,7 @@ trc_status trc_intersect(trc_scene* s, const float* rays, int32_t n, int32_t* tr
     if (!s->configured) throw Fail(TRC_ERR_STATE, "scene is not configured");
     if (n < 0 || (n > 0 && (!rays || !tri || !uvt))) throw Fail(TRC_ERR_INVALID, "bad ray buffers");
     if (n == 0) return;
-    LaunchCfg L = make_cfg(s->ctx, s, (hipStream_t)stream, n);
+    const StreamCfg L(s->ctx, s, (hipStream_t)stream, n);
     hip_check(launch_intersect(s->dev, L, rays, n, tri, uvt, any_hit, (hipStream_t)stream), "k_intersect");
   });
 }
@@ -715,7 +724,7 @@ trc_status trc_render_paths(trc_scene* s, const trc_camera* cam, const trc_optio
     CameraDev C = to_cam(cam);
     if (!paths) throw Fail(TRC_ERR_INVALID, "paths buffer is NULL");
     long long np = (long long)opt->spp * C.width * C.height;
-    LaunchCfg L = make_cfg(s->ctx, s, (hipStream_t)stream, np);
+    const StreamCfg L(s->ctx, s, (hipStream_t)stream, np);
     hip_check(launch_render_paths(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, paths, nullptr,
                                   (hipStream_t)stream),
               "k_render_paths");
@@ -733,7 +742,7 @@ static void render_fwd_impl(trc_scene* s, const trc_camera* cam, const trc_optio
     throw Fail(TRC_ERR_INVALID, "checkpoint buffer too small (trc_checkpoint_bytes)");
   float* paths = nullptr;
   hip_check(hipMallocAsync((void**)&paths, (size_t)np * 12, st), "hipMallocAsync(paths)");
-  LaunchCfg L = make_cfg(s->ctx, s, st, np);
+  const StreamCfg L(s->ctx, s, st, np);
   hipError_t e = launch_render_paths(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, paths, ckpt, st);
   if (e == hipSuccess) e = launch_film_reduce(paths, opt->spp, C.width * C.height, film, st);
   hipFreeAsync(paths, st);
@@ -761,7 +770,7 @@ trc_status trc_render_fwd_noalloc(trc_scene* s, const trc_camera* cam, const trc
     // launch shape as trc_render_fwd's, but the traversal stack gets only the
     // spill depth this scene's BVH needs, and the spill slice and the chunk
     // of per-path radiance live in the fixed scratch
-    LaunchCfg L = make_cfg(ctx, s, st, (long long)np, /*with_spill=*/false);
+    LaunchCfg L = make_cfg(ctx, s, (long long)np);
     const int cap = std::max(s->dev.stack_need, kStackLds);
     L.cap = cap;
     const uint64_t spill_bytes = ((uint64_t)(cap - kStackLds) * (uint64_t)L.grid * kBlock * 4 + 255) / 256 * 256;
@@ -938,7 +947,7 @@ trc_status trc_render_batch(trc_ctx* ctx, const trc_job* jobs, int32_t n, int32_
       hip_check(launch_fill_zero(gbase, gfloats, st), "k_fill_zero");
       assign_grad_copies(jd, gbase);
     }
-    LaunchCfg L = make_cfg(ctx, deepest, st, (long long)total);
+    const StreamCfg L(ctx, deepest, st, (long long)total);
     const uint64_t tiled = mark_solo(jd);
     const uint64_t tile = default_tile(tiled, adjoint);
     const uint64_t ntiles = assign_tiles(jd, tile);
@@ -1027,7 +1036,7 @@ trc_status trc_plan_create(trc_ctx* ctx, const trc_job* jobs, int32_t n, int32_t
       }
       // launch shape of the deepest scene, with a spill buffer owned by the plan
       // so that launches never allocate
-      p->L = make_cfg(ctx, deepest, nullptr, (long long)p->total, false);
+      p->L = make_cfg(ctx, deepest, (long long)p->total);
       const size_t words = spill_words(ctx->num_cus * kBlocksPerCU);
       hip_check(hipMalloc((void**)&p->spill, (words + kTileCtrWords) * 4), "hipMalloc(plan spill)");
       p->L.spill = p->spill;
@@ -1139,7 +1148,7 @@ trc_status trc_render_adj_ckpt(trc_scene* s, const trc_camera* cam, const trc_op
     long long np = (long long)opt->spp * C.width * C.height;
     if (ckpt_bytes < (int64_t)checkpoint_bytes((uint64_t)np, opt->max_bounces))
       throw Fail(TRC_ERR_INVALID, "checkpoint buffer too small (trc_checkpoint_bytes)");
-    LaunchCfg L = make_cfg(s->ctx, s, (hipStream_t)stream, np);
+    const StreamCfg L(s->ctx, s, (hipStream_t)stream, np);
     GradCopies gc = make_grad_copies(s->dev.n_verts, (hipStream_t)stream);
     hipError_t e = launch_render_adj_ckpt(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, ckpt, dLdI, dpos, dmat,
                                           dtex, s->vn_adj, gc, (hipStream_t)stream);
@@ -1347,7 +1356,7 @@ trc_status trc_render_stats(trc_scene* s, const trc_camera* cam, const trc_optio
     unsigned long long* d = nullptr;
     hip_check(hipMalloc((void**)&d, 4 * sizeof(unsigned long long)), "hipMalloc(counters)");
     hipError_t e = hipMemsetAsync(d, 0, 4 * sizeof(unsigned long long), st);
-    LaunchCfg L = make_cfg(s->ctx, s, st, np);
+    const StreamCfg L(s->ctx, s, st, np);
     if (e == hipSuccess) e = launch_render_stats(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, d, st);
     if (e == hipSuccess) e = hipMemcpyAsync(counters, d, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1420,12 +1429,12 @@ static void boundary_call(trc_scene* s, const trc_camera* cam, const trc_options
     guide.enabled = 1;
     if (!reuse) {
       s->guide_key.valid = false;
-      LaunchCfg Lg = make_cfg(s->ctx, s, st, (long long)nv);
+      const StreamCfg Lg(s->ctx, s, st, (long long)nv);
       hip_check(launch_guide_build(s->dev, Lg, gseed, guide, st), "k_guide");
       if (opt->g_keep) s->guide_key = key;
     }
   }
-  LaunchCfg L = make_cfg(s->ctx, s, st, N);
+  const StreamCfg L(s->ctx, s, st, N);
   if (kind == 1) {
     // of the call alone: pixel terms of one scene may run on several streams
     WindowScratch q(L, kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes(kind, (uint64_t)N, chunk) + 4; });
@@ -1472,7 +1481,7 @@ trc_status trc_render_deriv(trc_scene* s, const trc_camera* cam, const trc_optio
     CameraDev C = to_cam(cam);
     hipStream_t st = (hipStream_t)stream;
     const long long np = (long long)opt->spp * C.width * C.height;
-    LaunchCfg L = make_cfg(s->ctx, s, st, np);
+    const StreamCfg L(s->ctx, s, st, np);
     // vertex-normal tangents only where a differentiable mesh is smooth
     float* tvn = nullptr;
     if (s->vn_adj)
@@ -1493,7 +1502,7 @@ trc_status trc_render_adj(trc_scene* s, const trc_camera* cam, const trc_options
     CameraDev C = to_cam(cam);
     if (!dLdI || !dpos) throw Fail(TRC_ERR_INVALID, "dLdI / dpos is NULL");
     long long np = (long long)opt->spp * C.width * C.height;
-    LaunchCfg L = make_cfg(s->ctx, s, (hipStream_t)stream, np);
+    const StreamCfg L(s->ctx, s, (hipStream_t)stream, np);
     GradCopies gc = make_grad_copies(s->dev.n_verts, (hipStream_t)stream);
     hipError_t e = hipErrorOutOfMemory;
     ReplayScratch rs(L, (uint64_t)np, opt->max_bounces, (hipStream_t)stream);

@@ -15,9 +15,16 @@ struct trc_ctx {
   int device = 0;
   int num_cus = 0;
   std::string last_error;
-  // traversal stack spill per stream ([depth][threads] of the largest grid),
-  // allocated on a stream's first launch; guarded by mu
-  std::map<hipStream_t, uint32_t*> spill;
+  // Device memory of the launches on a stream: traversal stack spill
+  // ([depth][threads] of the largest grid), tile counters and scratch,
+  // allocated on the stream's first launch.  A call's kernels hand their
+  // results to one another in it, so a call holds `queueing` while it queues
+  // them: calls of several threads on one stream follow each other whole.
+  struct StreamMem {
+    uint32_t* spill = nullptr;
+    std::mutex queueing;
+  };
+  std::map<hipStream_t, StreamMem> streams;  // guarded by mu
   std::mutex mu;
   // this device's copy of the fixed scratch of trc_render_fwd_noalloc
   // (hipGetSymbolAddress, looked up once per device at context creation)
