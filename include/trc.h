@@ -12,6 +12,13 @@
  * owned by the library and stay resident in HBM until trc_scene_destroy.
  * Films, adjoint images and gradient buffers are caller-owned device memory.
  *
+ * Streams: the kernels of a call hand results over in memory that the context
+ * keeps per stream.  Threads may share a stream.  A call that is captured into
+ * a HIP graph uses that memory of the captured stream at every replay: a
+ * replay must not overlap calls on that stream, nor replays of other graphs
+ * captured on it.  The stream's first call has to be an eager one.  (Prepared
+ * batches, trc_plan, have memory of their own.)
+ *
  * Image layout (as the reference Tensorf image, Shape({W*H}, Vec3)): three
  * planes [3][H*W] of float, pixel index = y * W + x.
  * Vertex gradients: [V][3] float, V = total vertex count of the scene, in

@@ -96,10 +96,18 @@ GradCopies make_grad_copies(int n_verts, hipStream_t st) {
   return g;
 }
 
+bool is_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // the default stream, while another one is captured
+  return false;
+}
+
 // Scratch of a pass that runs in windows of paths or samples: bytes(window),
 // the stream's own where that is enough for the first window, else allocated on
 // the stream, for the largest window (halved down to 32k) that can be; null
-// when none can.
+// when none can.  A captured call runs in the largest window that the stream's
+// own holds: a graph then has no allocation node.
 struct WindowScratch {
   void* ptr = nullptr;
   bool kept = false;
@@ -108,6 +116,9 @@ struct WindowScratch {
   template <class Bytes>
   WindowScratch(const LaunchCfg& L, uint64_t first_window, hipStream_t stream, Bytes&& bytes)
       : window(first_window), st(stream) {
+    auto halve = [&] { window = (window / 2 + 63) / 64 * 64; };
+    if (L.scratch && is_capturing(st))
+      while (bytes(window) > kStreamScratch && window > (32u << 10)) halve();
     kept = L.scratch && bytes(window) <= kStreamScratch;
     if (kept) {
       ptr = L.scratch;
@@ -117,7 +128,7 @@ struct WindowScratch {
       (void)hipGetLastError();
       ptr = nullptr;
       if (window <= (32u << 10)) return;
-      window = (window / 2 + 63) / 64 * 64;
+      halve();
     }
   }
   ~WindowScratch() {
@@ -1304,11 +1315,7 @@ trc_status trc_lsolver_solve(trc_lsolver* s, const float* b, float* x, int32_t m
     const size_t nv3 = 3 * (size_t)s->n;
     float *r = s->work, *p0 = r + nv3, *p1 = p0 + nv3, *ap = p1 + nv3;
     // under capture every iteration is recorded: a replay may need them all
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const bool plain =
-        hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
-    if (!plain) (void)hipGetLastError();
-    uint32_t* done = plain ? s->done : nullptr;
+    uint32_t* done = is_capturing((hipStream_t)stream) ? nullptr : s->done;
     if (++s->seq == 0u) s->seq = 1u;
     hip_check(launch_cg(s->dev(), b, x, r, p0, p1, ap, s->scal, max_iter, tol, done, s->seq, (hipStream_t)stream),
               "k_cg");
@@ -1436,7 +1443,7 @@ static void boundary_call(trc_scene* s, const trc_camera* cam, const trc_options
   }
   const StreamCfg L(s->ctx, s, st, N);
   if (kind == 1) {
-    // of the call alone: pixel terms of one scene may run on several streams
+    // the call's or its stream's: pixel terms of one scene may run on several streams
     WindowScratch q(L, kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes(kind, (uint64_t)N, chunk) + 4; });
     hip_check(!q.ptr ? hipErrorOutOfMemory
                      : launch_boundary(kind, s->dev, C, opt->seed, opt->max_bounces, spp, L, prim, guide, dLdI, dpos,

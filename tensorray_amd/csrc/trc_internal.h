@@ -110,7 +110,7 @@ struct trc_scene {
     float eps = 0.0f;
   } guide_key;
   // survivor queue of the primary / direct / indirect boundary kernels (the
-  // pixel boundary's is allocated on its stream)
+  // pixel boundary's belongs to its call or stream)
   DevBuf bq_buf;
   // adjoint of the vertex normals [V][3] (kept zero between calls), present
   // when a differentiable mesh is smooth-shaded

@@ -58,7 +58,7 @@ def test_pixel_boundary(gpu_ctx, oracle_mod, W, H, spp):
 
 
 def test_pixel_boundary_first_call_captured(gpu_ctx):
-    """The scratch of the pixel term belongs to the call: a scene's first such
+    """The scratch of a small pixel term is its stream's: a scene's first such
     call may be a captured one."""
     import torch
     W, H, spp = 72, 40, 4
@@ -84,6 +84,53 @@ def test_pixel_boundary_first_call_captured(gpu_ctx):
         g.replay()
         torch.cuda.synchronize()
         _close(dpos.cpu().numpy().astype(np.float64), eager.cpu().numpy().astype(np.float64))
+        ds.render_fwd(cam, opt, film.data_ptr())
+        torch.cuda.synchronize()
+    del g
+    ds.close()
+
+
+# paths in one window of the stream's scratch; samples and paths in several (of
+# 2^18 samples, 2^19 paths; the last one is ragged)
+@pytest.mark.parametrize("kind,W,H,spp", [("pixel", 301, 220, 16), ("interior", 71, 40, 4), ("interior", 401, 300, 9)])
+def test_captured_windows(gpu_ctx, kind, W, H, spp):
+    """The windows of the pixel term and of the interior derivative image lie
+    in their stream's memory: a scene's first such call may be a captured one,
+    of any size, and its graph has no allocation node."""
+    import torch
+    spec = scenes.box_scene(subdiv=2)
+    ds = _capi.DeviceScene(gpu_ctx, spec)
+    cam = _capi.make_camera(W, H, **scenes.BOX_CAMERA)
+    opt = _capi.make_options(seed=31, max_bounces=2, spp=spp, sppe0=spp)
+    dl = torch.from_numpy(np.random.default_rng(2).uniform(0.2, 1.0, (3, W * H)).astype(np.float32)).cuda()
+    nv = ds.info().num_vertices
+    if kind == "pixel":
+        out, eager = torch.zeros(nv, 3, device="cuda"), torch.zeros(nv, 3, device="cuda")
+
+        def call(buf, stream=None):
+            ds.render_boundary(cam, opt, "pixel", dl.data_ptr(), buf.data_ptr(), stream=stream)
+    else:
+        out, eager = torch.zeros(3, W * H, device="cuda"), torch.zeros(3, W * H, device="cuda")
+        tpos = torch.zeros(nv, 3, device="cuda")
+        tpos[:len(spec.meshes[0].pos)] = torch.tensor([0.3, 0.8, -0.5], device="cuda")
+
+        def call(buf, stream=None):
+            ds.render_deriv(cam, opt, "interior", tpos.data_ptr(), None, buf.data_ptr(), stream=stream)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    film = torch.empty(3, W * H, device="cuda")
+    ds.render_fwd(cam, opt, film.data_ptr(), stream=st.cuda_stream)  # the stream's own buffers
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        call(out, st.cuda_stream)
+    call(eager)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _close(out.cpu().numpy().astype(np.float64), eager.cpu().numpy().astype(np.float64))
         ds.render_fwd(cam, opt, film.data_ptr())
         torch.cuda.synchronize()
     del g
