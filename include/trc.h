@@ -12,6 +12,16 @@
  * owned by the library and stay resident in HBM until trc_scene_destroy.
  * Films, adjoint images and gradient buffers are caller-owned device memory.
  *
+ * Working memory: the context keeps about 116 MB per stream that renders (a
+ * traversal stack spill, and 32 MB of scratch where they are to be had), until
+ * it is destroyed.  Requests of more than some 300,000 paths or samples take
+ * more on the stream for the time of the call: trc_render_fwd 12 bytes a path;
+ * trc_render_adj and the interior term of trc_render_deriv up to 248 MB, the
+ * pixel term of trc_render_boundary up to 377 MB, less where that is not to be
+ * had (the work is then done in more, smaller windows).  Small meshes' gradient
+ * copies take up to 16 MB.  A scene keeps up to 336 MB for its other boundary
+ * terms.
+ *
  * Streams: the kernels of a call hand results over in memory that the context
  * keeps per stream.  Threads may share a stream.  A call that is captured into
  * a HIP graph uses that memory of the captured stream at every replay: a

@@ -92,9 +92,22 @@ def build_pymodule():
     return out
 
 
+def build_tests():
+    """tests/_build/libtrc_unit.so: what the tests call below the C ABI."""
+    src = os.path.join(ROOT, "tests", "native", "unit.hip")
+    if not os.path.exists(src):
+        return None
+    out = os.path.join(ROOT, "tests", "_build", "libtrc_unit.so")
+    os.makedirs(os.path.dirname(out), exist_ok=True)
+    _run([HIPCC] + HIP_FLAGS + ["-shared", src, "-o", out + ".tmp"])
+    os.replace(out + ".tmp", out)
+    return out
+
+
 def build():
     build_lib()
     build_pymodule()
+    build_tests()
 
 
 if __name__ == "__main__":

@@ -12,6 +12,7 @@
 
 #include "trc_internal.h"
 #include "common/tr_bsdf.h"
+#include "host/window.h"
 
 using namespace trc;
 
@@ -103,33 +104,25 @@ bool is_capturing(hipStream_t st) {
   return false;
 }
 
-// Scratch of a pass that runs in windows of paths or samples: bytes(window),
-// the stream's own where that is enough for the first window, else allocated on
-// the stream, for the largest window (halved down to 32k) that can be; null
-// when none can.  A captured call runs in the largest window that the stream's
-// own holds: a graph then has no allocation node.
-struct WindowScratch {
-  void* ptr = nullptr;
-  bool kept = false;
-  uint64_t window = 0;
+// Memory of a pass that runs in windows of paths or samples (bytes(window) for
+// the largest, first_window): the stream's scratch for small requests, else
+// allocated on the stream; where that much is not to be had smaller windows,
+// down to what the scratch holds or kMinWindow.  A captured call takes the
+// largest window that the scratch holds: its graph then has no allocation node.
+struct WindowScratch : Window {
   hipStream_t st;
   template <class Bytes>
-  WindowScratch(const LaunchCfg& L, uint64_t first_window, hipStream_t stream, Bytes&& bytes)
-      : window(first_window), st(stream) {
-    auto halve = [&] { window = (window / 2 + 63) / 64 * 64; };
-    if (L.scratch && is_capturing(st))
-      while (bytes(window) > kStreamScratch && window > (32u << 10)) halve();
-    kept = L.scratch && bytes(window) <= kStreamScratch;
-    if (kept) {
-      ptr = L.scratch;
-      return;
-    }
-    while (hipMallocAsync(&ptr, (size_t)bytes(window), st) != hipSuccess) {
+  WindowScratch(const LaunchCfg& L, uint64_t first_window, hipStream_t stream, Bytes&& bytes) : st(stream) {
+    auto alloc = [&](uint64_t n) -> void* {
+      void* p = nullptr;
+      if (hipMallocAsync(&p, (size_t)n, st) == hipSuccess) return p;
       (void)hipGetLastError();
-      ptr = nullptr;
-      if (window <= (32u << 10)) return;
-      halve();
-    }
+      return nullptr;
+    };
+    auto fit = [&](bool may_alloc) { return fit_window(first_window, bytes, L.scratch, kStreamScratch, may_alloc, alloc); };
+    Window& w = *this;
+    if (is_capturing(st)) w = fit(false);
+    if (!ptr) w = fit(true);
   }
   ~WindowScratch() {
     if (ptr && !kept) hipFreeAsync(ptr, st);
@@ -181,11 +174,19 @@ struct StreamCfg : LaunchCfg {
       m = &ctx->streams[st];
     }
     own = std::unique_lock<std::mutex>(m->queueing);
-    if (!m->spill)
-      hip_check(hipMalloc((void**)&m->spill, (words + kTileCtrWords) * 4 + kStreamScratch), "hipMalloc(spill)");
+    if (!m->spill) {
+      // without the scratch where memory is short
+      const size_t need = (words + kTileCtrWords) * 4;
+      m->has_scratch = hipMalloc((void**)&m->spill, need + kStreamScratch) == hipSuccess;
+      if (!m->has_scratch) {
+        (void)hipGetLastError();
+        m->spill = nullptr;
+        hip_check(hipMalloc((void**)&m->spill, need), "hipMalloc(spill)");
+      }
+    }
     spill = m->spill;
     tiles = m->spill + words;
-    scratch = tiles + kTileCtrWords;
+    if (m->has_scratch) scratch = tiles + kTileCtrWords;
   }
 };
 
@@ -1447,7 +1448,7 @@ static void boundary_call(trc_scene* s, const trc_camera* cam, const trc_options
     WindowScratch q(L, kBndChunk, st, [=](uint64_t chunk) { return boundary_queue_bytes(kind, (uint64_t)N, chunk) + 4; });
     hip_check(!q.ptr ? hipErrorOutOfMemory
                      : launch_boundary(kind, s->dev, C, opt->seed, opt->max_bounces, spp, L, prim, guide, dLdI, dpos,
-                                       tpos, dimg, q.ptr, q.window, st),
+                                       tpos, dimg, q.ptr, q.size, st),
               "k_boundary");
     return;
   }
@@ -1495,7 +1496,7 @@ trc_status trc_render_deriv(trc_scene* s, const trc_camera* cam, const trc_optio
       hip_check(hipMallocAsync((void**)&tvn, 3 * (size_t)s->dev.n_verts * sizeof(float), st), "hipMallocAsync(tvn)");
     ReplayScratch rs(L, (uint64_t)np, opt->max_bounces, st);
     const hipError_t e = !rs.ptr ? hipErrorOutOfMemory : launch_render_deriv(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, tpos, tmat, tvn,
-                                             dimg, rs.ptr, rs.window, st);
+                                             dimg, rs.ptr, rs.size, st);
     if (tvn) hipFreeAsync(tvn, st);
     hip_check(e, "k_render_deriv");
   });
@@ -1515,7 +1516,7 @@ trc_status trc_render_adj(trc_scene* s, const trc_camera* cam, const trc_options
     ReplayScratch rs(L, (uint64_t)np, opt->max_bounces, (hipStream_t)stream);
     if (rs.ptr)
       e = launch_render_adj(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, dLdI, dpos, dmat, dtex, s->vn_adj, gc,
-                            rs.ptr, rs.window, (hipStream_t)stream);
+                            rs.ptr, rs.size, (hipStream_t)stream);
     if (gc.base) hipFreeAsync(gc.base, (hipStream_t)stream);
     hip_check(e, "k_render_adj");
   });

@@ -22,6 +22,7 @@ struct trc_ctx {
   // them: calls of several threads on one stream follow each other whole.
   struct StreamMem {
     uint32_t* spill = nullptr;
+    bool has_scratch = false;
     std::mutex queueing;
   };
   std::map<hipStream_t, StreamMem> streams;  // guarded by mu
