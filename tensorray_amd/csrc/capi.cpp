@@ -264,22 +264,19 @@ void upload_scene(trc_scene* s, hipStream_t st) {
   }
   d.verts = upload(s, verts, st);
   d.nodes = upload(s, h.nodes, st);
-  float ext = 0.0f;
   {
     const Bvh4Node& root = h.nodes[0];
-    const float* lo[3] = {root.lox, root.loy, root.loz};
-    const float* hi[3] = {root.hix, root.hiy, root.hiz};
-    for (int k = 0; k < 3; ++k) {
-      float a = lo[k][0], b = hi[k][0];
-      for (int i = 1; i < 4; ++i)
-        if (root.child[i] != kEmpty) {
-          a = std::min(a, lo[k][i]);
-          b = std::max(b, hi[k][i]);
-        }
-      ext = std::max(ext, b - a);
+    float lo[3] = {root.lox[0], root.loy[0], root.loz[0]}, hi[3] = {root.hix[0], root.hiy[0], root.hiz[0]};
+    for (int i = 1; i < 4; ++i) {
+      if (root.child[i] == kEmpty) continue;
+      const float l[3] = {root.lox[i], root.loy[i], root.loz[i]}, u[3] = {root.hix[i], root.hiy[i], root.hiz[i]};
+      for (int k = 0; k < 3; ++k) {
+        lo[k] = std::min(lo[k], l[k]);
+        hi[k] = std::max(hi[k], u[k]);
+      }
     }
+    d.qinv_scale = 1.0f / quant_scale(lo, hi);
   }
-  d.qinv_scale = 1.0f / quant_scale(ext);
   std::vector<QNode> qnodes(h.nodes.size());
   for (size_t i = 0; i < qnodes.size(); ++i) qnodes[i] = quantize_node(h.nodes[i], d.qinv_scale);
   d.qnodes = upload(s, qnodes, st);

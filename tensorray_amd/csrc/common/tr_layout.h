@@ -102,12 +102,21 @@ TR_HD uint32_t half_bits(float xf, bool up) {
 }
 #endif
 
-// The scale of a tree of extent `ext`: offsets up to 2^14 steps, which leaves
-// room for a refit to grow the boxes fourfold (beyond that the upper planes
-// become infinite: the boxes only stop culling).
-TR_HD float quant_scale(float ext) {
+// The scale of a tree with bounds lo .. hi: plane offsets up to 2^14 steps,
+// which leaves room for a refit to grow the boxes fourfold (beyond that the
+// upper planes become infinite: the boxes only stop culling).  A plane's offset
+// is at most the tree's extent and the rounding of its node's origin (2^-12 of
+// the coordinate), which is the larger part beyond 4,096 extents from zero.
+TR_HD float quant_scale(const float lo[3], const float hi[3]) {
+  float off = 0.0f;
+  for (int k = 0; k < 3; ++k) {
+    const float a = lo[k] < 0.0f ? -lo[k] : lo[k], b = hi[k] < 0.0f ? -hi[k] : hi[k];
+    const float mag = (a > b ? a : b) * (1.0f / 4096.0f), ext = hi[k] - lo[k];
+    off = ext > off ? ext : off;
+    off = mag > off ? mag : off;
+  }
   int e = 0;
-  if (ext > 0.0f && ext < 1e30f) frexp((double)ext, &e);
+  if (off > 0.0f && off < 1e30f) frexp((double)off, &e);
   e = e < -80 ? -80 : e;
   return (float)ldexp(1.0, e - 14);
 }

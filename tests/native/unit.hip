@@ -2,6 +2,7 @@
 // Built into tests/_build/libtrc_unit.so; loaded with ctypes.
 #include <hip/hip_runtime.h>
 
+#include "../../tensorray_amd/csrc/common/tr_layout.h"
 #include "../../tensorray_amd/csrc/host/window.h"
 
 using namespace trc;
@@ -23,4 +24,12 @@ extern "C" void unit_fit_window(uint64_t first, uint64_t total, uint64_t per_ite
   out[0] = w.size;
   out[1] = !w.ptr ? 0u : w.kept ? 1u : 2u;
   out[2] = asked;
+}
+
+// Reciprocal of the scale of a tree with bounds box[0 .. 3) .. box[3 .. 6).
+extern "C" float unit_quant_inv_scale(const float box[6]) { return 1.0f / quant_scale(box, box + 3); }
+
+// n nodes quantized on the host.
+extern "C" void unit_quantize(const Bvh4Node* nodes, int n, float inv_scale, QNode* out) {
+  for (int i = 0; i < n; ++i) out[i] = quantize_node(nodes[i], inv_scale);
 }

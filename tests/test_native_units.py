@@ -3,6 +3,7 @@ through tests/native (built with the library)."""
 import ctypes
 import os
 
+import numpy as np
 import pytest
 
 MB = 1 << 20
@@ -10,6 +11,7 @@ MB = 1 << 20
 
 @pytest.fixture(scope="module")
 def unit():
+    import torch  # noqa: F401  (its HIP runtime, before the library asks for one)
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_build", "libtrc_unit.so")
     if not os.path.exists(path):
         from tensorray_amd import build
@@ -52,3 +54,76 @@ def test_window_choice_ends_when_counters_outgrow_it(unit):
     no chunk fits the stream's memory, and the search ends."""
     w, how, _ = _fit(unit, 1 << 22, 1 << 33, 90, 1024, 32 * MB, 0, 1 << 40)
     assert how == 0 and w == 4096
+
+
+# ---------------------------------------------------------------------------
+# Quantized nodes
+# ---------------------------------------------------------------------------
+def _aligned(shape, dtype):
+    buf = np.zeros(int(np.prod(shape)) * np.dtype(dtype).itemsize + 128, np.uint8)
+    off = -buf.ctypes.data % 128
+    return buf[off:off + int(np.prod(shape)) * np.dtype(dtype).itemsize].view(dtype).reshape(shape)
+
+
+def _nodes(boxes):
+    """[N][4][2][3] boxes as Bvh4Node words [N][32]: all slots inner children."""
+    n = len(boxes)
+    w = _aligned((n, 32), np.float32)
+    for k in range(3):
+        w[:, 4 * k:4 * k + 4] = boxes[:, :, 0, k]
+        w[:, 12 + 4 * k:16 + 4 * k] = boxes[:, :, 1, k]
+    w.view(np.uint32)[:, 24:28] = np.arange(4 * n, dtype=np.uint32).reshape(n, 4)
+    return w
+
+
+def _decode(q, inv_scale):
+    """Child planes [N][4][2][3] of QNode words in float64."""
+    org = np.stack([q[:, 0] & 0xFFFFF800, (q[:, 0] << 21 | q[:, 1] >> 11) & 0xFFFFF800, (q[:, 1] << 10) & 0xFFFFF800],
+                   1).astype(np.uint32).view(np.float32).astype(np.float64)
+    out = np.empty((len(q), 4, 2, 3))
+    for k in range(3):
+        h = np.ascontiguousarray(q[:, 4 + 4 * k:8 + 4 * k]).view(np.float16).astype(np.float64)  # lower 4, upper 4
+        out[:, :, 0, k] = (org[:, None, k] + h[:, :4]) / inv_scale
+        out[:, :, 1, k] = (org[:, None, k] + h[:, 4:]) / inv_scale
+    return out
+
+
+def _quantize(unit, boxes, inv_scale):
+    nodes, q = _nodes(boxes), _aligned((len(boxes), 16), np.uint32)
+    unit.unit_quantize(nodes.ctypes.data_as(ctypes.c_void_p), len(boxes), ctypes.c_float(inv_scale),
+                       q.ctypes.data_as(ctypes.c_void_p))
+    return q
+
+
+def _random_boxes(n, centre, extent, smallest, seed):
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(-0.5, 0.5, (n, 1, 1, 3)) * extent
+    size = extent * 10.0 ** rng.uniform(np.log10(smallest), 0, (n, 1, 1, 1))
+    a = centre + c + size * rng.uniform(-0.5, 0.5, (n, 4, 1, 3))
+    d = size * rng.uniform(0, 0.5, (n, 4, 1, 3))
+    return np.concatenate([a - d, a + d], 2).astype(np.float32)
+
+
+def _inv_scale(unit, boxes):
+    unit.unit_quant_inv_scale.restype = ctypes.c_float
+    b = np.concatenate([boxes[:, :, 0].min((0, 1)), boxes[:, :, 1].max((0, 1))]).astype(np.float32)
+    return float(unit.unit_quant_inv_scale(b.ctypes.data_as(ctypes.c_void_p)))
+
+
+@pytest.mark.parametrize("extent", [1e-6, 2.0, 3e5])
+@pytest.mark.parametrize("distance", [0.0, 3.0, 5e3, 2e4, 1e6])
+def test_quantized_planes(unit, extent, distance):
+    """Planes lie outside their boxes, by no more than the formats' roundings:
+    2^-11 of an offset from the node's origin (a half), the widening of 2^-20,
+    and as offsets reach the node's size plus the origin's rounding of 2^-12,
+    2^-10 of the node's size and 2^-22 of the coordinate in all."""
+    centre = np.array([1.0, -0.7, 0.3]) * distance * extent
+    boxes = _random_boxes(2000, centre, extent, 1e-4, 5)
+    inv = _inv_scale(unit, boxes)
+    planes = _decode(_quantize(unit, boxes, inv), inv)
+    b = boxes.astype(np.float64)
+    assert np.isfinite(planes).all()
+    assert (planes[:, :, 0] <= b[:, :, 0]).all() and (planes[:, :, 1] >= b[:, :, 1]).all()
+    size = (b[:, :, 1].max(1) - b[:, :, 0].min(1))[:, None, None]
+    slack = size * 2.0**-10 + np.abs(b).max((1, 2))[:, None, None] * 2.0**-22 + extent * 2.0**-37
+    assert (np.abs(planes - b) <= slack).all()
