@@ -632,6 +632,16 @@ trc_status trc_scene_set_vertices(trc_scene* s, const float* pos, int32_t nv, in
       s->host.build_bvh();
       upload_scene(s, st);
       ++s->rebuilds;
+      return;
+    }
+    // a tree that has grown, shrunk or moved far (by more than 2 in its scale:
+    // the offsets have room for 4) is quantized anew; its cost does not show
+    // that, being relative to the root's area
+    const float inv = 1.0f / quant_scale(s->upd_host->box, s->upd_host->box + 3);
+    if (inv < 0.5f * d.qinv_scale || inv > 2.0f * d.qinv_scale) {
+      d.qinv_scale = inv;
+      hip_check(launch_quantize(d, s->upd.n_nodes, st), "k_quantize");
+      hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
     }
   });
 }

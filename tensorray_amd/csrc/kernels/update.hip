@@ -426,8 +426,15 @@ __global__ void k_sah(const Bvh4Node* nodes, uint32_t N, const float* nbox, Upda
   if (threadIdx.x == 0) atomicAdd(&out->sah, part[0]);
 }
 
-__global__ void k_zero_sah(UpdateScalars* out) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) out->sah = 0.0;
+__global__ void k_zero_sah(const float* nbox, UpdateScalars* out) {
+  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+  out->sah = 0.0;
+  for (int k = 0; k < 6; ++k) out->box[k] = nbox[k];  // the root's
+}
+
+__global__ void k_quantize(const Bvh4Node* nodes, QNode* qnodes, float inv_scale, uint32_t n) {
+  const uint32_t i = blockIdx.x * kUpdBlock + threadIdx.x;
+  if (i < n) qnodes[i] = quantize_node(nodes[i], inv_scale);
 }
 
 inline unsigned blocks_for(uint64_t n) { return (unsigned)((n + kUpdBlock - 1) / kUpdBlock); }
@@ -490,9 +497,15 @@ hipError_t launch_scene_update(const SceneDev& S, const SceneUpdateDev& U, hipSt
                        const_cast<QNode*>(S.qnodes), S.qinv_scale, U.nbox, (const TriRecord*)tris, U.refit_nodes + a,
                        n);
   }
-  hipLaunchKernelGGL(k_zero_sah, dim3(1), dim3(1), 0, st, U.scal);
+  hipLaunchKernelGGL(k_zero_sah, dim3(1), dim3(1), 0, st, (const float*)U.nbox, U.scal);
   hipLaunchKernelGGL(k_sah, dim3(blocks_for(U.n_nodes)), dim3(kUpdBlock), 0, st, (const Bvh4Node*)nodes, U.n_nodes,
                      (const float*)U.nbox, U.scal);
+  return hipGetLastError();
+}
+
+hipError_t launch_quantize(const SceneDev& S, uint32_t n_nodes, hipStream_t st) {
+  hipLaunchKernelGGL(k_quantize, dim3(blocks_for(n_nodes)), dim3(kUpdBlock), 0, st, S.nodes,
+                     const_cast<QNode*>(S.qnodes), S.qinv_scale, n_nodes);
   return hipGetLastError();
 }
 

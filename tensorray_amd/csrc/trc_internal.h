@@ -59,6 +59,7 @@ struct UpdateScalars {
   float light_integral;   // Distribution1D integral of the emitter table
   float pad;
   double sah;             // SAH cost of the refit tree (rebuild decision)
+  float box[6];           // bounds of the refit tree (scale of the quantized nodes)
 };
 // Device arrays of the update, owned by the scene.
 struct SceneUpdateDev {
@@ -291,6 +292,8 @@ uint32_t edge_scan_words(uint32_t n_edges);
 // Recomputes face normals and areas, vertex normals, the emitter table, the
 // secondary-edge list, the triangle records and the BVH boxes from S.pos.
 hipError_t launch_scene_update(const SceneDev& S, const SceneUpdateDev& U, hipStream_t st);
+// Every node's quantized form with the scale in S.
+hipError_t launch_quantize(const SceneDev& S, uint32_t n_nodes, hipStream_t st);
 // Primary edges seen from `eye` (boundary or silhouette) into out_* (capacity
 // U.n_edges), their count and length integral into *count.
 hipError_t launch_prim_edges(const SceneDev& S, const SceneUpdateDev& U, const float eye[3], EdgeDev* out_e,

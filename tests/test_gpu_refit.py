@@ -112,3 +112,45 @@ def test_sah_growth_triggers_rebuild(gpu_ctx, oracle_mod):
     assert np.array_equal(ds.vertices(), pos)
     _check_forward(gpu_ctx, oracle_mod, ds, moved, 48, 40, 4, 2, 21)
     ds.close()
+
+
+@pytest.mark.parametrize("factor", [128.0, 3.0, 2.0**-10])
+def test_refit_to_another_size(gpu_ctx, oracle_mod, factor):
+    """A scene that a refit makes `factor` times as large: its cost relative to
+    the root's area does not change, so the tree stays, and its hits are the
+    oracle's.  Scaling by a power of two keeps the tree a fresh scene of that
+    size gets, and a render then visits as many nodes as there (1 %: the
+    scales of the two trees' quantized nodes may differ by two)."""
+    import torch
+    full = scenes.sphere_scene(subdiv=3, amplitude=0.05)
+    pos = _allpos(full)
+    small = scenes.sphere_scene(subdiv=3, amplitude=0.05)
+    for m in small.meshes:
+        m.pos = (np.asarray(m.pos, np.float32) / np.float32(factor)).astype(np.float32)
+    ds = _capi.DeviceScene(gpu_ctx, small)
+    ds.set_vertices(pos.ctypes.data, len(pos), True)
+    info = ds.info()
+    assert info.bvh_refits == 1 and info.bvh_rebuilds == 0
+    rng = np.random.default_rng(8)
+    n = 20000
+    o = rng.normal(size=(n, 3))
+    o = 3.0 * o / np.linalg.norm(o, axis=1, keepdims=True)
+    d = rng.uniform(-1, 1, (n, 3)) - o
+    rays = np.concatenate([o, np.full((n, 1), 1e-3), d, np.full((n, 1), 1e30)], 1).astype(np.float32)
+    rd = torch.from_numpy(rays).cuda()
+    tri, uvt = torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, 3, device="cuda")
+    ds.intersect(rd.data_ptr(), n, tri.data_ptr(), uvt.data_ptr())
+    torch.cuda.synchronize()
+    want_tri, want_uvt = oracle_mod.Scene(full).intersect(rays)
+    assert np.array_equal(tri.cpu().numpy(), want_tri)
+    assert np.array_equal(uvt.cpu().numpy().view(np.uint32), want_uvt.view(np.uint32))
+    _check_forward(gpu_ctx, oracle_mod, ds, full, 48, 40, 2, 2, 15)
+    fresh = _capi.DeviceScene(gpu_ctx, full)
+    cam = _capi.make_camera(64, 64, **scenes.CAMERA_DEFAULT)
+    opt = _capi.make_options(seed=3, max_bounces=2, spp=4)
+    visits, fresh_visits = ds.render_stats(cam, opt)[2], fresh.render_stats(cam, opt)[2]
+    print(f"factor {factor}: {visits} node visits, {fresh_visits} of a fresh scene")
+    if factor != 3.0:
+        assert abs(visits - fresh_visits) <= 0.01 * fresh_visits
+    ds.close()
+    fresh.close()
