@@ -454,10 +454,11 @@ struct PathGroup {
 
 // The primary pass over one group: camera rays of the box filter (the sample
 // stays inside its pixel) and first hits, from the group's 64 lanes at once.
-// `paths` points at the words of path `paths_first`.
+// `paths` points at the words of path `paths_first`.  mask: dL/dI or null; the
+// paths of pixels where it is zero are not traced and count as missed.
 template <bool kCkpt>
 __device__ inline void trace_primary(const SceneDev& S, const CameraDev& C, const PathParams& P, TraceCtx& tc, const PathGroup& g,
-                                     const CkptDev& ck, float* paths, uint64_t paths_first) {
+                                     const CkptDev& ck, float* paths, uint64_t paths_first, const float* mask = nullptr) {
   const uint32_t lane = threadIdx.x & 63u;
   const bool has = g.has(lane);
   const uint64_t path = has ? g.path(lane) : g.base;
@@ -466,8 +467,10 @@ __device__ inline void trace_primary(const SceneDev& S, const CameraDev& C, cons
   const Rnd4 rc = rng4(P.seed, kRngInterior, path, 0u);
   const F3 eye{C.eye[0], C.eye[1], C.eye[2]};
   const F3 d = camera_dir(C, (float)px + rc.a, (float)py + rc.b);
+  const uint32_t wh = (uint32_t)C.width * (uint32_t)C.height;
+  const bool traced = has && (!mask || mask[pix] != 0.0f || mask[wh + pix] != 0.0f || mask[2 * wh + pix] != 0.0f);
   TraceState ts;
-  if (has) trace_begin(ts, 1e32f);
+  if (traced) trace_begin(ts, 1e32f);
   else trace_none(ts);
   trace_run<true>(S, tc, eye, d, d, 1e32f, kShadowEpsilon, false, ts, 0);
   const Hit h = trace_hit(ts);

@@ -59,17 +59,18 @@ __global__ void __launch_bounds__(kBlock) k_intersect(SceneDev S, LaunchCfg L, c
 }
 
 // Camera rays: a wave takes 64 slots at a time from the launch's counter.
-template <bool kCkpt>
+// kMask: none of the pixels where mask (dL/dI) is zero.
+template <bool kCkpt, bool kMask>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kFwdWaves)))
 k_primary(SceneDev S, CameraDev C, PathParams P, LaunchCfg L, PathRange R, uint32_t tile, float* paths,
-          uint64_t paths_first, CkptDev ck) {
+          uint64_t paths_first, CkptDev ck, const float* mask) {
   __shared__ __align__(8) uint32_t lds_stack[(kTraceLdsWords + kTraceSlotWords) * kBlock];
   TraceCtx tc = make_trace_ctx_wave(lds_stack, L);
   const uint64_t nwaves = (uint64_t)L.grid * (kBlock / 64);
   const uint64_t wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
   TileSupply sup = TileSupply::make(wave, nwaves, 0, R.slots, tile, L.tiles);
   while (sup.next < sup.end) {
-    trace_primary<kCkpt>(S, C, P, tc, PathGroup::at(C, R, sup.next), ck, paths, paths_first);
+    trace_primary<kCkpt>(S, C, P, tc, PathGroup::at(C, R, sup.next), ck, paths, paths_first, kMask ? mask : nullptr);
     sup.next += 64u;
     if (sup.next >= sup.end) sup.more();
   }
@@ -568,18 +569,18 @@ static uint32_t forward_tile(uint64_t slots, int grid, bool dynamic) {
   return (uint32_t)(t < 64 ? 64 : (t > 4096 ? 4096 : t));
 }
 
-template <bool kCkpt>
+template <bool kCkpt, bool kMask = false>
 static hipError_t launch_paths(const SceneDev& S, const CameraDev& C, const PathParams& P, const LaunchCfg& L,
                                uint64_t first, uint64_t count, float* paths, uint64_t paths_first, const CkptDev& ck,
-                               hipStream_t st) {
-  const LaunchCfg Lp = fit_grid(k_primary<kCkpt>, L), Lb = fit_grid(k_bounces<kCkpt>, L);
+                               hipStream_t st, const float* mask = nullptr) {
+  const LaunchCfg Lp = fit_grid(k_primary<kCkpt, kMask>, L), Lb = fit_grid(k_bounces<kCkpt>, L);
   if (L.tiles) {
     const hipError_t e = launch_fill_zero(reinterpret_cast<float*>(L.tiles), 2 * kTileSet, st);
     if (e != hipSuccess) return e;
   }
   const PathRange R = path_range(C, first, count);
-  hipLaunchKernelGGL((k_primary<kCkpt>), dim3(Lp.grid), dim3(kBlock), 0, st, S, C, P, Lp, R,
-                     forward_tile(R.slots, Lp.grid, L.tiles != nullptr), paths, paths_first, ck);
+  hipLaunchKernelGGL((k_primary<kCkpt, kMask>), dim3(Lp.grid), dim3(kBlock), 0, st, S, C, P, Lp, R,
+                     forward_tile(R.slots, Lp.grid, L.tiles != nullptr), paths, paths_first, ck, mask);
   hipLaunchKernelGGL((k_bounces<kCkpt>), dim3(Lb.grid), dim3(kBlock), 0, st, S, C, P, Lb, R,
                      forward_tile(R.slots, Lb.grid, L.tiles != nullptr), paths, paths_first, ck);
   return hipGetLastError();
@@ -699,21 +700,25 @@ constexpr uint64_t kReplayWindow = 2u << 20;
 uint64_t replay_window(uint64_t npaths) { return npaths < kReplayWindow ? npaths : kReplayWindow; }
 uint64_t replay_bytes(uint64_t window, int max_bounces) { return 12ull * window + ckpt_bytes(window, max_bounces); }
 
-// Calls pass(first, count, checkpoint, chunk counter) for windows of the
-// request's paths, each traced into `scratch` (replay_bytes(window)) first.
+// Calls pass(first, count, checkpoint) for windows of the request's paths, each
+// traced into `scratch` (replay_bytes(window)) first; mask: dL/dI of a pass
+// that needs no paths of the pixels where it is zero, else null.
 // One launch that re-traced a path and swept it backwards on the same lane
 // carried the adjoint's registers through the traversal (301 x 211 x 16 smooth
 // scene: 1.74 ms against 0.45 for the forward and 0.26 for the sweep).
 template <class Pass>
 static hipError_t replay_windows(const SceneDev& S, const CameraDev& C, uint32_t seed, int max_bounces, int spp,
-                                 const LaunchCfg& L, void* scratch, uint64_t window, hipStream_t st, Pass&& pass) {
+                                 const LaunchCfg& L, void* scratch, uint64_t window, const float* mask, hipStream_t st,
+                                 Pass&& pass) {
   const uint64_t np = (uint64_t)spp * (uint64_t)C.width * (uint64_t)C.height;
   if (!L.spill) return hipErrorInvalidValue;
   for (uint64_t first = 0; first < np; first += window) {
     const uint64_t count = first + window < np ? window : np - first;
     float* paths = (float*)scratch;
     const CkptDev ck = ckpt_window(paths + 3 * window, first, count, max_bounces);
-    hipError_t e = launch_paths<true>(S, C, PathParams{seed, max_bounces, spp, 0u}, L, first, count, paths, first, ck, st);
+    const PathParams P{seed, max_bounces, spp, 0u};
+    hipError_t e = mask ? launch_paths<true, true>(S, C, P, L, first, count, paths, first, ck, st, mask)
+                        : launch_paths<true>(S, C, P, L, first, count, paths, first, ck, st);
     // the traversal is done with the stream's spill buffer: word 0 becomes the
     // chunk counter of the sweep
     if (e == hipSuccess) e = launch_fill_zero((float*)L.spill, 1, st);
@@ -728,7 +733,7 @@ hipError_t launch_render_adj(const SceneDev& S, const CameraDev& C, uint32_t see
                              float* vn_adj, const GradCopies& gc, void* scratch, uint64_t window, hipStream_t st) {
   const LaunchCfg Lk = fit_grid(k_render_adj_ckpt, L);
   hipError_t e = replay_windows(
-      S, C, seed, max_bounces, spp, L, scratch, window, st, [&](uint64_t first, uint64_t count, const CkptDev& ck) {
+      S, C, seed, max_bounces, spp, L, scratch, window, dLdI, st, [&](uint64_t first, uint64_t count, const CkptDev& ck) {
         hipLaunchKernelGGL(k_render_adj_ckpt, dim3(Lk.grid), dim3(kBlock), 0, st, S, C,
                            (PathParams{seed, max_bounces, spp, 0u}), Lk, first, count, ck, dLdI, dpos, dmat, vn_adj,
                            dtex, gc, L.spill);
@@ -750,7 +755,7 @@ hipError_t launch_render_deriv(const SceneDev& S, const CameraDev& C, uint32_t s
   }
   const LaunchCfg Lk = fit_grid(k_render_deriv, L);
   return replay_windows(
-      S, C, seed, max_bounces, spp, L, scratch, window, st, [&](uint64_t first, uint64_t count, const CkptDev& ck) {
+      S, C, seed, max_bounces, spp, L, scratch, window, nullptr, st, [&](uint64_t first, uint64_t count, const CkptDev& ck) {
         hipLaunchKernelGGL(k_render_deriv, dim3(Lk.grid), dim3(kBlock), 0, st, S, C,
                            (PathParams{seed, max_bounces, spp, 0u}), Lk, first, count, ck, tpos, tmat,
                            (const float*)tvn, dimg, L.spill);

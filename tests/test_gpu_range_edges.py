@@ -159,6 +159,34 @@ def test_replay_windows(gpu_ctx, W, H, spp):
     ds.close()
 
 
+# dL/dI zero in all pixels but one, in whole blocks and halves of the image
+@pytest.mark.parametrize("keep", ["pixel", "block", "half", "none"])
+def test_replay_of_a_masked_image(gpu_ctx, oracle_mod, keep):
+    import torch
+    W, H, spp = 50, 37, 3
+    spec = scenes.sphere_scene(subdiv=2)
+    ds = _capi.DeviceScene(gpu_ctx, spec)
+    cam = _capi.make_camera(W, H, **scenes.CAMERA_DEFAULT)
+    opt = _capi.make_options(seed=5, max_bounces=2, spp=spp)
+    mask = np.zeros((H, W), np.float32)
+    y, x = {"pixel": (20, 25), "block": (slice(16, 24), slice(24, 32)), "half": (slice(None), slice(0, 25)),
+            "none": (slice(0), slice(0))}[keep]
+    mask[y, x] = 1.0
+    dl = (np.random.default_rng(3).uniform(0.2, 1.0, (3, W * H)) * mask.reshape(-1)).astype(np.float32)
+    dl[1:] *= 0.5 if keep != "pixel" else 0.0  # a pixel counts with any of its channels
+    dpos = torch.zeros(ds.info().num_vertices, 3, device="cuda")
+    ds.render_adj(cam, opt, torch.from_numpy(dl).cuda().data_ptr(), dpos.data_ptr())
+    torch.cuda.synchronize()
+    got = dpos.cpu().numpy().astype(np.float64)
+    if keep == "none":
+        assert not got.any()
+    else:
+        ref, _ = oracle_mod.Scene(spec).render_adj(scenes.CAMERA_DEFAULT, W, H, 5, 2, spp, dl)
+        m = spec.diff_vertex_mask()
+        _close(got[m], ref[m])
+    ds.close()
+
+
 # rows: less than a slice of 64, one over, several slices with a remainder
 @pytest.mark.parametrize("freq", [1, 2, 3, 8])
 def test_solver_slices(gpu_ctx, oracle_mod, freq):
