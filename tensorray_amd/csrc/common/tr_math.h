@@ -72,11 +72,18 @@ TR_HD float rcp_rn(float b) {
   const float y = __builtin_amdgcn_rcpf(b);
   return fmaf(fmaf(-b, y, 1.0f), y, y);
 }
-// a / b with y = RN(1 / b); the fixup handles zero, infinite and NaN operands.
+// a / b with y = RN(1 / b), for |a / b| < 2^127; the fixup handles zero,
+// infinite and NaN operands.
 TR_HD float div_by(float a, float b, float y) {
   float q = a * y;
   q = fmaf(fmaf(-b, q, a), y, q);
   return __builtin_amdgcn_div_fixupf(q, b, a);
+}
+// The same for all quotients: the residual of an overflowing one is not a
+// number, and it stays infinite.
+TR_HD float div_by_any(float a, float b, float y) {
+  const float q = a * y, r = fmaf(fmaf(-b, q, a), y, q);
+  return __builtin_amdgcn_div_fixupf(fabsf(q) < INFINITY ? r : q, b, a);
 }
 // RN(sqrt(x)) for x in [2^-96, 2^126).
 TR_HD float sqrt_plain(float x) {
@@ -96,9 +103,9 @@ TR_HD float rsqrt_rn(float x) { return rcp_rn(sqrt_plain(x)); }
 TR_HD F3 operator/(F3 a, float b) {
   if (TR_UNLIKELY(!plain_divisor(b))) return F3{a.x / b, a.y / b, a.z / b};
   const float y = rcp_rn(b);
-  return F3{div_by(a.x, b, y), div_by(a.y, b, y), div_by(a.z, b, y)};
+  return F3{div_by_any(a.x, b, y), div_by_any(a.y, b, y), div_by_any(a.z, b, y)};
 }
-// a / sqrt(l2), the root in *len.
+// a / sqrt(l2), the root in *len; l2 = len2(a), so that no quotient overflows.
 TR_HD F3 over_sqrt(F3 a, float l2, float* len) {
   if (TR_UNLIKELY(!plain_radicand(l2))) {
     const float l = sqrtf(l2);

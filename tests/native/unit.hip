@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../tensorray_amd/csrc/common/tr_layout.h"
+#include "../../tensorray_amd/csrc/common/tr_math.h"
 #include "../../tensorray_amd/csrc/host/window.h"
 
 using namespace trc;
@@ -32,4 +33,53 @@ extern "C" float unit_quant_inv_scale(const float box[6]) { return 1.0f / quant_
 // n nodes quantized on the host.
 extern "C" void unit_quantize(const Bvh4Node* nodes, int n, float inv_scale, QNode* out) {
   for (int i = 0; i < n; ++i) out[i] = quantize_node(nodes[i], inv_scale);
+}
+
+namespace {
+constexpr int kThreads = 256;
+
+// What a thread's arithmetic unit gives for x / b, 1 / sqrt and lengths (see below).
+__global__ void k_math(int what, const float* a, const float* b, float* out, uint32_t n) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= n) return;
+  if (what == 0) {
+    const F3 q = F3{a[i], -a[i], 0.5f * a[i]} / b[i];
+    out[3 * i] = q.x;
+    out[3 * i + 1] = q.y;
+    out[3 * i + 2] = q.z;
+  } else if (what == 1) {
+    out[i] = sqrt_rn(a[i]);
+  } else if (what == 2) {
+    out[i] = rsqrt_rn(a[i]);
+  } else if (what == 3) {
+    const F3 v{a[3 * i], a[3 * i + 1], a[3 * i + 2]};
+    float l;
+    const F3 d = over_sqrt(v, len2(v), &l);
+    out[4 * i] = d.x;
+    out[4 * i + 1] = d.y;
+    out[4 * i + 2] = d.z;
+    out[4 * i + 3] = l;
+  } else {
+    out[i] = ratio_self(a[i]);
+  }
+}
+
+__global__ void k_quantize_nodes(const Bvh4Node* nodes, uint32_t n, float inv_scale, QNode* out) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i < n) out[i] = quantize_node(nodes[i], inv_scale);
+}
+}  // namespace
+
+// Device arithmetic on device arrays of n items; what: 0 (a, -a, a / 2) / b to
+// out [n][3], 1 sqrt_rn(a), 2 rsqrt_rn(a), 3 a [n][3] normalized, and its
+// length, to out [n][4], 4 ratio_self(a).
+extern "C" int unit_math(int what, const float* a, const float* b, float* out, uint32_t n) {
+  k_math<<<(n + kThreads - 1) / kThreads, kThreads>>>(what, a, b, out, n);
+  return (int)hipGetLastError();
+}
+
+// n nodes quantized on the device (device arrays).
+extern "C" int unit_quantize_device(const Bvh4Node* nodes, uint32_t n, float inv_scale, QNode* out) {
+  k_quantize_nodes<<<(n + kThreads - 1) / kThreads, kThreads>>>(nodes, n, inv_scale, out);
+  return (int)hipGetLastError();
 }

@@ -127,3 +127,114 @@ def test_quantized_planes(unit, extent, distance):
     size = (b[:, :, 1].max(1) - b[:, :, 0].min(1))[:, None, None]
     slack = size * 2.0**-10 + np.abs(b).max((1, 2))[:, None, None] * 2.0**-22 + extent * 2.0**-37
     assert (np.abs(planes - b) <= slack).all()
+
+
+@pytest.mark.gpu
+def test_device_quantizes_as_the_host(unit):
+    """Half-precision subnormals, zero, the largest and infinite planes too:
+    the scales run from one at which all offsets underflow to one at which
+    they overflow."""
+    import torch
+    for distance in (0.0, 3.0, 3e4):
+        boxes = _random_boxes(3001, np.array([1.0, -0.7, 0.3]) * distance, 1.0, 1e-6, 6)
+        boxes[::7, 1] = boxes[::7, 0]  # flat nodes: offsets of zero
+        nodes = _nodes(boxes)
+        for e in (-40, -24, -20, 0, 11, 14, 16, 17, 20):
+            want = _quantize(unit, boxes, 2.0**e)
+            dn = torch.from_numpy(nodes.copy()).cuda()
+            out = torch.zeros(len(boxes), 16, dtype=torch.int32, device="cuda")
+            p = ctypes.c_void_p
+            assert unit.unit_quantize_device(p(dn.data_ptr()), len(boxes), ctypes.c_float(2.0**e), p(out.data_ptr())) == 0
+            torch.cuda.synchronize()
+            got = out.cpu().numpy().view(np.uint32)
+            # the words behind the planes of a node are not set by either
+            assert np.array_equal(got, want), (distance, e)
+
+
+# ---------------------------------------------------------------------------
+# Correctly rounded arithmetic of the device
+# ---------------------------------------------------------------------------
+def _math(unit, what, a, b=None, width=1):
+    import torch
+    n = len(a)
+    da = torch.from_numpy(np.ascontiguousarray(a, np.float32)).cuda()
+    db = torch.from_numpy(np.ascontiguousarray(b if b is not None else a, np.float32)).cuda()
+    out = torch.zeros(n, width, device="cuda")
+    p = ctypes.c_void_p
+    assert unit.unit_math(what, p(da.data_ptr()), p(db.data_ptr()), p(out.data_ptr()), n) == 0
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _same(got, want):
+    """The same bits; any NaN for a NaN."""
+    nan = np.isnan(want)
+    return np.array_equal(np.isnan(got), nan) and np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
+def _floats(rng, n, lo, hi):
+    """Random signs and mantissas (some of them all ones or zeros), exponents in [lo, hi]."""
+    m = rng.integers(0, 1 << 23, n, dtype=np.uint32)
+    m[::17] = (1 << 23) - 1
+    m[1::17] = 0
+    e = rng.integers(lo + 127, hi + 128, n, dtype=np.uint32)
+    return (rng.integers(0, 2, n, dtype=np.uint32) << 31 | e << 23 | m).view(np.float32)
+
+
+SPECIAL = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-45, -1e-45, 1.1754944e-38, 3.4028235e38, -3.4028235e38, 1.0,
+                    2.0**-96, 2.0**-97, 2.0**126, 2.0**127], np.float32)
+
+
+@pytest.mark.gpu
+def test_device_divisions(unit):
+    """Quotients by a shared reciprocal are those of IEEE division (float32
+    division of numpy), overflowing ones and special operands included.
+    Excepted are last bits of quotients of numerators below 2^-100 and of
+    subnormal quotients."""
+    rng = np.random.default_rng(1)
+    n = 4_000_000
+    a, b = _floats(rng, n, -98, 126), _floats(rng, n, -126, 125)
+    sa, sb = (x.reshape(-1) for x in np.meshgrid(SPECIAL, np.concatenate([SPECIAL, _floats(rng, 50, -126, 126)])))
+    for a, b in ((a, b), (sa, sb)):
+        got = _math(unit, 0, a, b, 3)
+        with np.errstate(all="ignore"):
+            want = np.stack([a / b, -a / b, (np.float32(0.5) * a) / b], 1)
+        tiny = (np.abs(want) < 2.0**-125) | (np.abs(np.stack([a, a, 0.5 * a], 1)) < 2.0**-100)
+        ulp = np.float32(2.0**-23) * np.abs(want) + np.float32(1e-45)
+        with np.errstate(all="ignore"):
+            near = ~tiny | ~np.isfinite(want) | (np.abs(got - want) <= ulp)
+        assert near.all()
+        assert _same(got[~tiny], want[~tiny])
+        assert np.isinf(want).any()
+
+
+@pytest.mark.gpu
+def test_device_roots(unit):
+    rng = np.random.default_rng(2)
+    # every mantissa over two exponents, then random positive floats and special ones
+    every = np.arange(0x3F800000, 0x40800000, dtype=np.uint32).view(np.float32)
+    x = np.concatenate([every, np.abs(_floats(rng, 1_000_000, -126, 127)), SPECIAL])
+    with np.errstate(all="ignore"):
+        assert _same(_math(unit, 1, x)[:, 0], np.sqrt(x))
+        inside = x[(x >= 2.0**-96) & (x < 2.0**126)]
+        assert _same(_math(unit, 2, inside)[:, 0], np.float32(1.0) / np.sqrt(inside))
+        want = x / x
+    assert _same(_math(unit, 4, x)[:, 0], want)
+
+
+@pytest.mark.gpu
+def test_device_normalize(unit):
+    rng = np.random.default_rng(3)
+    n = 1_000_000
+    v = rng.normal(size=(n, 3)).astype(np.float32) * (2.0 ** rng.integers(-45, 60, (n, 1))).astype(np.float32)
+    v[: n // 2] /= np.sqrt((v[: n // 2] ** 2).sum(1, dtype=np.float32))[:, None]  # nearly normalized
+    v[::1001] = 0.0
+    v[1::1001, 0] = np.inf
+    v[2::1001] = 1e-30
+    got = _math(unit, 3, v, width=4)
+    with np.errstate(all="ignore"):
+        l = np.sqrt(v[:, 0] * v[:, 0] + v[:, 1] * v[:, 1] + v[:, 2] * v[:, 2])
+        want = np.concatenate([v / l[:, None], l[:, None]], 1)
+    tiny = (np.abs(v) < 2.0**-100) & (v != 0)
+    ok = ~np.concatenate([tiny, np.zeros((n, 1), bool)], 1)
+    assert _same(got[ok], want[ok])
