@@ -281,8 +281,9 @@ struct Collapser {
     }
     out[out_index] = node;
     out.resize(out.size() + (size_t)ni);
-    // at most nk-1 siblings are pending on the stack while a child is visited
-    for (int s = 0; s < ni; ++s) need = std::max(need, (nk - 1) + collapse(kids[s], first_child + (uint32_t)s, depth + 1));
+    // only inner children are pushed (leaves go to the lane's queue): at most
+    // ni - 1 are pending on the stack while one of them is visited
+    for (int s = 0; s < ni; ++s) need = std::max(need, (ni - 1) + collapse(kids[s], first_child + (uint32_t)s, depth + 1));
     return need;
   }
 };

@@ -16,7 +16,8 @@ namespace trc {
 // the direction, kx / ky the two after it, S the shear constants.  The paper
 // swaps kx and ky when d[kz] < 0 to keep the winding; that only flips the
 // signs of U, V, W, of det and of T, so (t, u, v) are the same bits without
-// it, and the test below accepts either winding.
+// it (but for the sign of a zero u or v, where the ray meets an edge), and the
+// test below accepts either winding.
 struct RayPre {
   F3 o;
   int kz;

@@ -322,6 +322,20 @@ def perlin_texture(w, h, seed, octaves=4, base=8.0):
 CAMERA_DEFAULT = dict(pos=(0.0, 1.0, 3.0), target=(0.0, 0.0, 0.0), up=(0.0, 1.0, 0.0), fov=45.0)
 
 
+def chain_scene(levels, per, ratio, seed=0):
+    """sphere_scene with clusters of `per` triangles, each cluster `ratio`
+    times as large and as far from the origin as the one before, in place of
+    its sphere: the shape with the deepest trees."""
+    rng = np.random.default_rng(seed)
+    c = np.stack([np.ones((levels, per)), *(0.2 * rng.uniform(-1, 1, (2, levels, per)))], -1)
+    tri = c[:, :, None] + rng.uniform(-0.05, 0.05, (levels, per, 3, 3))
+    pos = (tri * (float(ratio) ** np.arange(levels))[:, None, None, None]).reshape(-1, 3)
+    spec = sphere_scene(subdiv=0)
+    spec.meshes[0].pos = pos.astype(np.float32)
+    spec.meshes[0].idx = np.arange(len(pos), dtype=np.uint32).reshape(-1, 3)
+    return spec
+
+
 def sphere_scene(subdiv=2, amplitude=0.0, noise_seed=1, material=None, diff=True, smooth=False,
                  ground_albedo=(0.5, 0.5, 0.5), light_radiance=(10.0, 10.0, 10.0), texture_res=0,
                  texture_seed=7, freq=0):

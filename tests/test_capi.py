@@ -121,6 +121,24 @@ def test_bvh_invariants(host_ctx, subdiv, amp):
     ds.close()
 
 
+@pytest.mark.parametrize("per,levels,ratio", [(2, 74, 0.5), (3, 56, 0.4), (4, 66, 0.5), (5, 64, 0.5), (4, 60, 0.25)])
+def test_stack_need_of_deep_trees(host_ctx, per, levels, ratio):
+    """Clusters of triangles on a geometric progression make the deepest
+    trees.  The stack holds inner siblings only (leaves are queued), and these
+    fit its 80 entries."""
+    ds = _capi.DeviceScene(host_ctx, scenes.chain_scene(levels, per, ratio))
+    info = ds.info()
+    child = ds.bvh()[0][:, 24:28]
+    inner = (child & 0x80000000) == 0  # empty slots have the bit too
+    need = np.zeros(len(child), np.int64)
+    for n in range(len(child) - 1, -1, -1):  # children come after their parents
+        kids = child[n][inner[n]]
+        need[n] = max([0] + [len(kids) - 1 + need[k] for k in kids])
+    assert info.bvh_stack_need == need[0] + 1 <= 80
+    assert info.bvh_max_depth > 20
+    ds.close()
+
+
 def test_invalid_scene_is_rejected(host_ctx):
     spec = scenes.config1_scene()
     spec.meshes[0].idx = spec.meshes[0].idx.copy()

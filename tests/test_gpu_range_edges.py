@@ -39,6 +39,39 @@ def test_path_order(gpu_ctx, oracle_mod, W, H, spp, B):
     ds.close()
 
 
+# trees whose stack spills out of LDS, and one that needs all of its 80 entries
+@pytest.mark.parametrize("levels,per,ratio", [(40, 4, 0.5), (60, 4, 0.25)])
+def test_deep_tree(gpu_ctx, oracle_mod, levels, per, ratio):
+    import torch
+    spec = scenes.chain_scene(levels, per, ratio)
+    ds = _capi.DeviceScene(gpu_ctx, spec)
+    assert 40 <= ds.info().bvh_stack_need <= 80
+    rng = np.random.default_rng(9)
+    n = 20000
+    # along the chain, from its far end and from its tip, and across it
+    pos = spec.meshes[0].pos
+    to = pos[rng.integers(0, len(pos), n)].astype(np.float64)
+    o = np.where(rng.random((n, 1)) < 0.5, rng.normal(size=(n, 3)) * 1e-3, np.array([1.5, 0.0, 0.0]) * rng.uniform(0.7, 1, (n, 1)))
+    o[::5] = rng.normal(size=(len(o[::5]), 3))
+    rays = np.concatenate([o, np.full((n, 1), 1e-9), to - o, np.full((n, 1), 1e30)], 1).astype(np.float32)
+    rd = torch.from_numpy(rays).cuda()
+    tri, uvt = torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, 3, device="cuda")
+    ds.intersect(rd.data_ptr(), n, tri.data_ptr(), uvt.data_ptr())
+    torch.cuda.synchronize()
+    want_tri, want_uvt = oracle_mod.Scene(spec).intersect(rays, brute=True)
+    assert np.array_equal(tri.cpu().numpy(), want_tri)
+    assert np.array_equal(uvt.cpu().numpy(), want_uvt)  # rays through vertices: zeros of either sign
+    cam = _capi.make_camera(24, 20, pos=(1.3, 0.05, 0.0), target=(0.0, 0.0, 0.0))
+    opt = _capi.make_options(seed=2, max_bounces=2, spp=2)
+    paths = torch.zeros(960, 3, device="cuda")
+    ds.render_paths(cam, opt, paths.data_ptr())
+    torch.cuda.synchronize()
+    ref = oracle_mod.Scene(spec).render_paths(dict(scenes.CAMERA_DEFAULT, pos=(1.3, 0.05, 0.0), target=(0.0, 0.0, 0.0)),
+                                              24, 20, 2, 2, 0, 960)
+    assert np.array_equal(paths.cpu().numpy(), ref)
+    ds.close()
+
+
 # one sample group; ragged and whole blocks; more samples than a chunk of 2^22
 @pytest.mark.parametrize("W,H,spp", [(5, 4, 4), (64, 64, 4), (70, 50, 8), (256, 256, 68)])
 def test_pixel_boundary(gpu_ctx, oracle_mod, W, H, spp):
