@@ -27,11 +27,11 @@ namespace trc {
 constexpr int kMaxBounces = 8;
 
 // 4-wide BVH node.  Child boxes are stored SoA; `child` encodes inner nodes
-// (index), leaves (kLeafBit | (count-1) << 27 | first) and empty slots
-// (kEmpty).  The builder fills the slots with the inner children first, then
-// the leaves, numbers the inner children of a node consecutively, and puts
-// one triangle into each leaf, consecutive ones into the leaves of a node:
-// QNode names all children by two base indices.
+// (index), leaves (kLeafBit | triangle record) and empty slots (kEmpty).  The
+// builder fills the slots with the inner children first, then the leaves,
+// numbers the inner children of a node consecutively, and puts one triangle
+// into each leaf, consecutive ones into the leaves of a node: QNode names all
+// children by two base indices.
 struct alignas(128) Bvh4Node {
   float lox[4], loy[4], loz[4];
   float hix[4], hiy[4], hiz[4];
@@ -42,15 +42,11 @@ static_assert(sizeof(Bvh4Node) == 128, "node must be one 128-byte line");
 
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 constexpr uint32_t kLeafBit = 0x80000000u;
-constexpr uint32_t kLeafFirstMask = (1u << 27) - 1u;
-constexpr int kMaxLeafTris = 8;
+constexpr uint32_t kLeafTriMask = (1u << 27) - 1u;
 
 TR_HD bool child_is_leaf(uint32_t c) { return (c & kLeafBit) != 0u && c != kEmpty; }
-TR_HD uint32_t leaf_first(uint32_t c) { return c & kLeafFirstMask; }
-TR_HD uint32_t leaf_count(uint32_t c) { return ((c >> 27) & 0xFu) + 1u; }
-TR_HD uint32_t make_leaf(uint32_t first, uint32_t count) {
-  return kLeafBit | ((count - 1u) << 27) | first;
-}
+TR_HD uint32_t leaf_tri(uint32_t c) { return c & kLeafTriMask; }
+TR_HD uint32_t make_leaf(uint32_t tri) { return kLeafBit | tri; }
 
 // A 4-wide node as the traversal reads it: 64 bytes, four 16-byte loads.
 // Child box planes are half-precision offsets from the node's origin in units
@@ -132,7 +128,7 @@ TR_HD QNode quantize_node(const Bvh4Node& n, float inv_scale) {
   for (int s = 0; s < 4; ++s) {
     if (n.child[s] == kEmpty) continue;
     if (n.child[s] & kLeafBit) {
-      if (nl == 0u) leaf = leaf_first(n.child[s]);
+      if (nl == 0u) leaf = leaf_tri(n.child[s]);
       ++nl;
     } else {
       ++ni;
@@ -170,12 +166,11 @@ TR_HD QNode quantize_node(const Bvh4Node& n, float inv_scale) {
   return q;
 }
 
-// SAH costs of a 4-wide node visit and of a triangle test, used by the
-// builder and by the cost that decides when a refit tree is rebuilt.
-// Forward time on the 20k-triangle metric scene against the traversal cost
-// (leaves of at most 4 triangles): 0.25-0.35 fastest (every leaf then holds
-// one triangle); 0.1 and 0.5 +0.5-1 %; 1 +4 %; 1.5 +6 %; 2 +11 % (also
-// with leaves of up to 8); 3 with leaves of up to 8 +23 %.
+// SAH costs of a 4-wide node visit and of a triangle test in the cost that
+// decides when a refit tree is rebuilt.  The builder has no use for them: at a
+// visit cost of 0.25 to 0.35, which rendered the 20k-triangle metric scene
+// fastest when it built leaves of up to 4 triangles, every leaf held one (0.1
+// and 0.5 +0.5-1 %; 1 +4 %; 1.5 +6 %; 2 +11 %).
 constexpr double kSahTraverse = 0.25;
 constexpr double kSahIntersect = 1.0;
 

@@ -37,17 +37,11 @@ struct Box {
 struct BinNode {
   Box box;
   int32_t left = -1, right = -1;  // children (inner) or -1
-  uint32_t first = 0, count = 0;  // leaf range in the order array
+  uint32_t first = 0;             // a leaf's place in the order array
   bool leaf() const { return left < 0; }
 };
 
 constexpr int kBins = 32;
-constexpr double kCostTraverse = kSahTraverse;
-constexpr double kCostIntersect = kSahIntersect;
-// One triangle per leaf: the quantized node names its leaves' triangles by
-// one base index.  (At a node visit costing kSahTraverse triangle tests,
-// almost no larger leaf was ever chosen.)
-constexpr int kMaxLeaf = 1;
 
 struct Builder {
   const std::vector<float>& pos;
@@ -84,27 +78,25 @@ struct Builder {
     for (auto& x : th) x.join();
   }
 
-  static int32_t make_leaf(std::vector<BinNode>& out, uint32_t first, uint32_t count, const Box& box) {
-    BinNode n;
-    n.box = box;
-    n.first = first;
-    n.count = count;
-    out.push_back(n);
-    return (int32_t)out.size() - 1;
-  }
-
   // The subtree over order[first, first + count) appended to `out` in
   // preorder (node, left subtree, right subtree); its root is the first node
   // appended.  With par_depth > 0 the two subtrees of a large node are built
   // on two threads into their own arrays and appended left then right, which
-  // gives the same array as the sequential build.
+  // gives the same array as the sequential build.  One triangle per leaf: the
+  // quantized node names its leaves' triangles by one base index.
   int32_t build_into(std::vector<BinNode>& out, uint32_t first, uint32_t count, int par_depth) {
     Box box, cbox;
     for (uint32_t i = first; i < first + count; ++i) {
       box.grow(tbox[order[i]]);
       cbox.grow(&cent[3 * (size_t)order[i]]);
     }
-    if (count <= 1) return make_leaf(out, first, count, box);
+    if (count <= 1) {
+      BinNode n;
+      n.box = box;
+      n.first = first;
+      out.push_back(n);
+      return (int32_t)out.size() - 1;
+    }
     double best_cost = DBL_MAX;
     int best_axis = -1, best_split = -1;
     for (int axis = 0; axis < 3; ++axis) {
@@ -140,10 +132,6 @@ struct Builder {
         if (cost < best_cost) { best_cost = cost; best_axis = axis; best_split = b; }
       }
     }
-    double parent_area = std::max(box.area(), 1e-30);
-    double leaf_cost = kCostIntersect * count;
-    double split_cost = best_axis >= 0 ? kCostTraverse + kCostIntersect * best_cost / parent_area : DBL_MAX;
-    if (count <= (uint32_t)kMaxLeaf && leaf_cost <= split_cost) return make_leaf(out, first, count, box);
     uint32_t mid;
     if (best_axis < 0) {
       // all centroids coincide: split the range in half
@@ -219,24 +207,21 @@ struct Collapser {
   BvhBuildStats& st;
   std::vector<int> depth_of;  // depth of every 4-wide node (root 1)
 
-  // Emits one leaf's triangles.
+  // Emits a leaf's triangle.
   uint32_t emit_leaf(const BinNode& n) {
-    uint32_t first = (uint32_t)tris.size();
-    for (uint32_t i = n.first; i < n.first + n.count; ++i) {
-      uint32_t t = order[i];
-      TriRecord r;
-      for (int k = 0; k < 3; ++k) {
-        r.v0[k] = pos[3 * (size_t)idx[3 * t] + k];
-        r.v1[k] = pos[3 * (size_t)idx[3 * t + 1] + k];
-        r.v2[k] = pos[3 * (size_t)idx[3 * t + 2] + k];
-      }
-      std::memcpy(&r.v0[3], &t, 4);
-      r.v1[3] = 0.0f;
-      r.v2[3] = 0.0f;
-      tris.push_back(r);
+    const uint32_t t = order[n.first];
+    TriRecord r;
+    for (int k = 0; k < 3; ++k) {
+      r.v0[k] = pos[3 * (size_t)idx[3 * t] + k];
+      r.v1[k] = pos[3 * (size_t)idx[3 * t + 1] + k];
+      r.v2[k] = pos[3 * (size_t)idx[3 * t + 2] + k];
     }
+    std::memcpy(&r.v0[3], &t, 4);
+    r.v1[3] = 0.0f;
+    r.v2[3] = 0.0f;
+    tris.push_back(r);
     st.leaves++;
-    return make_leaf(first, n.count);
+    return make_leaf((uint32_t)tris.size() - 1u);
   }
 
   // Converts binary node `b` (an inner node) into a 4-wide node at index
@@ -295,7 +280,7 @@ void bvh_build(const std::vector<float>& pos, const std::vector<uint32_t>& idx,
                std::vector<uint32_t>& order, BvhBuildStats& stats, BvhRefitPlan* plan) {
   const size_t T = idx.size() / 3;
   if (T == 0) throw std::runtime_error("bvh_build: no triangles");
-  if (T >= (size_t)kLeafFirstMask) throw std::runtime_error("bvh_build: too many triangles");
+  if (T >= (size_t)kLeafTriMask) throw std::runtime_error("bvh_build: too many triangles");
   Builder b(pos, idx);
   // threads: up to 16, as 2^par_depth subtree builders
   const unsigned hc = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
@@ -347,7 +332,7 @@ void bvh_build(const std::vector<float>& pos, const std::vector<uint32_t>& idx,
       if (n.child[s] == kEmpty) continue;
       double dx = (double)n.hix[s] - n.lox[s], dy = (double)n.hiy[s] - n.loy[s], dz = (double)n.hiz[s] - n.loz[s];
       double a = 2.0 * (dx * dy + dy * dz + dz * dx) / std::max(root_area, 1e-30);
-      cost += a * (child_is_leaf(n.child[s]) ? leaf_count(n.child[s]) * kCostIntersect : kCostTraverse);
+      cost += a * (child_is_leaf(n.child[s]) ? kSahIntersect : kSahTraverse);
     }
   stats.sah_cost = cost;
 }
@@ -374,9 +359,8 @@ void bvh_refit(const std::vector<float>& pos, const std::vector<uint32_t>& idx,
       if (c == kEmpty) continue;
       Box cb;
       if (child_is_leaf(c)) {
-        for (uint32_t i = leaf_first(c); i < leaf_first(c) + leaf_count(c); ++i) {
-          cb.grow(tris[i].v0); cb.grow(tris[i].v1); cb.grow(tris[i].v2);
-        }
+        const TriRecord& r = tris[leaf_tri(c)];
+        cb.grow(r.v0); cb.grow(r.v1); cb.grow(r.v2);
       } else {
         cb = nb[c];
       }

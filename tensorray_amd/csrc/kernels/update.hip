@@ -364,11 +364,10 @@ __global__ void k_refit_level(Bvh4Node* nodes, QNode* qnodes, float inv_scale, f
     DBox cb;
     cb.clear();
     if (child_is_leaf(c)) {
-      for (uint32_t i = leaf_first(c); i < leaf_first(c) + leaf_count(c); ++i) {
-        cb.grow(tris[i].v0);
-        cb.grow(tris[i].v1);
-        cb.grow(tris[i].v2);
-      }
+      const TriRecord& r = tris[leaf_tri(c)];
+      cb.grow(r.v0);
+      cb.grow(r.v1);
+      cb.grow(r.v2);
     } else {
       const float* b = nbox + 6 * (size_t)c;
       for (int k = 0; k < 3; ++k) {
@@ -395,7 +394,7 @@ __global__ void k_refit_level(Bvh4Node* nodes, QNode* qnodes, float inv_scale, f
 
 // SAH cost of the 4-wide tree relative to the root box (the build's
 // diagnostic): sum over child slots of area(child) / area(root) times the
-// slot's triangle count x kSahIntersect (leaves) or kSahTraverse (inner
+// slot's kSahIntersect (leaves, of one triangle) or kSahTraverse (inner
 // nodes).  Order of the double
 // additions is not fixed; the value only drives the rebuild decision.
 __global__ void k_sah(const Bvh4Node* nodes, uint32_t N, const float* nbox, UpdateScalars* out) {
@@ -414,7 +413,7 @@ __global__ void k_sah(const Bvh4Node* nodes, uint32_t N, const float* nbox, Upda
       const double dx = (double)n.hix[s] - n.lox[s], dy = (double)n.hiy[s] - n.loy[s],
                    dz = (double)n.hiz[s] - n.loz[s];
       const double a = 2.0 * (dx * dy + dy * dz + dz * dx) / ra;
-      cost += a * (child_is_leaf(c) ? (double)leaf_count(c) * kSahIntersect : kSahTraverse);
+      cost += a * (child_is_leaf(c) ? kSahIntersect : kSahTraverse);
     }
   }
   part[threadIdx.x] = cost;
