@@ -746,7 +746,7 @@ trc_status trc_render_paths(trc_scene* s, const trc_camera* cam, const trc_optio
     const StreamCfg L(s->ctx, s, (hipStream_t)stream, np);
     hip_check(launch_render_paths(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, paths, nullptr,
                                   (hipStream_t)stream),
-              "k_render_paths");
+              "k_primary/k_bounces");
   });
 }
 
@@ -765,7 +765,7 @@ static void render_fwd_impl(trc_scene* s, const trc_camera* cam, const trc_optio
   hipError_t e = launch_render_paths(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, paths, ckpt, st);
   if (e == hipSuccess) e = launch_film_reduce(paths, opt->spp, C.width * C.height, film, st);
   hipFreeAsync(paths, st);
-  hip_check(e, "k_render_paths/k_film_reduce");
+  hip_check(e, "k_primary/k_bounces/k_film_reduce");
 }
 
 trc_status trc_render_fwd(trc_scene* s, const trc_camera* cam, const trc_options* opt, float* film,
@@ -813,7 +813,7 @@ trc_status trc_render_fwd_noalloc(trc_scene* s, const trc_camera* cam, const trc
       if (e == hipSuccess)
         e = launch_film_accum(chunk, ns, (int)wh, film, s0 == 0, s0 + ns == opt->spp, opt->spp, st);
     }
-    hip_check(e, "k_render_paths/k_film_accum");
+    hip_check(e, "k_primary/k_bounces/k_film_accum");
   });
 }
 
@@ -1502,8 +1502,10 @@ trc_status trc_render_deriv(trc_scene* s, const trc_camera* cam, const trc_optio
     if (s->vn_adj)
       hip_check(hipMallocAsync((void**)&tvn, 3 * (size_t)s->dev.n_verts * sizeof(float), st), "hipMallocAsync(tvn)");
     ReplayScratch rs(L, (uint64_t)np, opt->max_bounces, st);
-    const hipError_t e = !rs.ptr ? hipErrorOutOfMemory : launch_render_deriv(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, tpos, tmat, tvn,
-                                             dimg, rs.ptr, rs.size, st);
+    hipError_t e = hipErrorOutOfMemory;
+    if (rs.ptr)
+      e = launch_render_deriv(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, tpos, tmat, tvn, dimg, rs.ptr,
+                              rs.size, st);
     if (tvn) hipFreeAsync(tvn, st);
     hip_check(e, "k_render_deriv");
   });
@@ -1525,7 +1527,7 @@ trc_status trc_render_adj(trc_scene* s, const trc_camera* cam, const trc_options
       e = launch_render_adj(s->dev, C, opt->seed, opt->max_bounces, opt->spp, L, dLdI, dpos, dmat, dtex, s->vn_adj, gc,
                             rs.ptr, rs.size, (hipStream_t)stream);
     if (gc.base) hipFreeAsync(gc.base, (hipStream_t)stream);
-    hip_check(e, "k_render_adj");
+    hip_check(e, "k_primary/k_bounces/k_render_adj_ckpt");
   });
 }
 

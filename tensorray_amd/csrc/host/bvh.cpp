@@ -1,5 +1,6 @@
-// Binned-SAH BVH build, collapsed to a 4-wide BVH laid out for the GPU
-// traversal kernel (128-byte nodes, triangles reordered into leaf order).
+// Binned-SAH BVH build, collapsed to a 4-wide BVH: nodes with exact boxes
+// (Bvh4Node), which the refits update and the traversal's quantized nodes are
+// made from, and triangles reordered into leaf order.
 //
 // Replaces the OptiX GAS build/compaction/update of the reference
 // (LibTensorRay/Renderer/Scene.cpp:171-366, 368-469).

@@ -305,12 +305,12 @@ struct BoundaryParams {
 };
 
 // ---------------------------------------------------------------------------
-// Survivor queues.  The primary, direct and indirect terms run in two
-// kernels per chunk of samples: a select kernel draws the samples, traces
-// their first rays and keeps the few that can contribute; an eval kernel
-// traces the long radiance / importance paths of those only, so its waves
-// start full instead of carrying the lanes whose samples died at the first
-// test.  The queue is structure-of-arrays (word k of slot s at
+// Survivor queues.  All terms start, per chunk of samples, with a select kernel
+// that draws the samples, traces their first rays and keeps the few that can
+// contribute.  Of those only, an eval kernel (direct, indirect) or a bounce and
+// a scatter kernel (primary, pixel) trace the long radiance / importance paths,
+// so their waves start full instead of carrying the lanes whose samples died at
+// the first test.  The queue is structure-of-arrays (word k of slot s at
 // w[k * cap + s]) and filled by wave-level ballot compaction: one atomic
 // per wave and consecutive slots for the surviving lanes.  Chunks are large
 // (4M samples, one chunk for a 512^2 x 16 request): every chunk ends in two

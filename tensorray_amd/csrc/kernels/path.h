@@ -1,8 +1,12 @@
-// One camera path of the interior integrator with next-event estimation and
-// MIS, evaluated per thread.  The same routine drives the forward kernel
-// (kRecord = false) and the first sweep of the adjoint kernel (kRecord =
-// true), which stores the discrete decisions and throughputs of the path in
-// a small per-thread record instead of an expression tape.
+// Paths of the interior integrator with next-event estimation and MIS.
+//
+// path_forward evaluates one camera path per thread: the adjoint kernels
+// re-evaluate a path from its checkpoint with it (kRecord = true, which stores
+// the discrete decisions and throughputs of the path in a small per-thread
+// record instead of an expression tape), and k_render_stats counts the work of
+// the paths it traces (kRecord = false).  path_bounces is its bounce loop, and
+// the indirect boundary term's.  The forward itself runs in two passes over
+// waves, trace_primary and render_bounces below.
 //
 // Reference: PathTracer::Radiance (LibTensorRay/Renderer/PathTracer.cpp:37-76),
 // EvalRadianceEmitted (Integrator.cpp:55-73), EvalRadianceDirect

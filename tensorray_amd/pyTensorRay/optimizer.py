@@ -4,8 +4,8 @@ on the device.
 The reference builds M = I + lmbda L (largesteps' compute_matrix, uniform
 Laplacian), optimizes u = M x with largesteps' AdamUniform and maps back
 with a Cholesky solve (cholespy).  Here M lives in the native library
-(trc_lsolver: CSR matrix, conjugate-gradient solves on the three coordinate
-columns at once) and the uniform Adam step is trc_adam_uniform_step; the
+(trc_lsolver: matrix in sliced rows, conjugate-gradient solves on the three
+coordinate columns at once) and the uniform Adam step is trc_adam_uniform_step; the
 parameter keeps the reference's layout, a flat [3 * n] tensor of x-plane,
 y-plane, z-plane (optimizer.py:170-172).
 """
